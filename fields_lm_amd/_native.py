@@ -55,6 +55,9 @@ SIGNATURES = {
     "fl_scan_backward_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "fl_gate_residual_norm": (_int, [_vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp, ctypes.c_float,
                                      _vp, _vp, _vp]),
+    "fl_gate_residual_norm_w": (_int, [_vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp, _int,
+                                       ctypes.c_float, _vp, _vp, _vp]),
+    "fl_field_params": (_int, [_vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp]),
     "fl_swiglu": (_int, [_vp, _int, _i64, _i64, _vp, _vp]),
     "fl_boundary_scan": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
     "fl_version": (ctypes.c_char_p, []),

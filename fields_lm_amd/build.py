@@ -13,11 +13,13 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
-SOURCES = [PKG_DIR / "csrc" / "field_scan.hip"]
+SOURCES = [PKG_DIR / "csrc" / name for name in ("field_scan.hip", "block_tail.hip")]
 INCLUDE_DIR = REPO_DIR / "include"
 LIB_PATH = PKG_DIR / "libfields_amd.so"
 # measurement kernels for bench.py (the scan's access pattern without its arithmetic), kept out of
@@ -53,16 +55,25 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None, out: Path
     """Compile the HIP sources into ``libfields_amd.so`` (always recompiles)."""
     target = Path(out) if out is not None else LIB_PATH
     tmp = target.with_suffix(".so.tmp")
-    cmd = [hipcc(), *HIP_FLAGS, *(extra_flags or []), f"-I{INCLUDE_DIR}",
-           *[str(s) for s in (sources or SOURCES)], "-o", str(tmp)]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    env = dict(os.environ)
-    proc = subprocess.run(cmd, capture_output=True, text=True, env=env)
-    if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{proc.stdout}\n{proc.stderr}")
-    if verbose and proc.stderr.strip():
-        print(proc.stderr, file=sys.stderr)
+    flags = [*HIP_FLAGS, *(extra_flags or []), f"-I{INCLUDE_DIR}"]
+
+    def run(cmd: list[str]) -> None:
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{proc.stdout}\n{proc.stderr}")
+        if verbose and proc.stderr.strip():
+            print(proc.stderr, file=sys.stderr)
+
+    # one object per source, compiled side by side, then one link
+    with tempfile.TemporaryDirectory() as work:
+        objects = [str(Path(work) / f"{i}_{s.stem}.o") for i, s in enumerate(sources or SOURCES)]
+        compile_flags = [f for f in flags if f != "-shared"]
+        with ThreadPoolExecutor(max_workers=4) as pool:
+            list(pool.map(run, [[hipcc(), *compile_flags, "-c", str(s), "-o", o]
+                                for s, o in zip(sources or SOURCES, objects)]))
+        run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", str(tmp)])
     missing = unresolved_kernel_stubs(tmp)
     if missing:
         tmp.unlink()

@@ -1,0 +1,287 @@
+// block_tail.hip — the Field block's elementwise work around its GEMMs and its scan
+// (reference: src/fields_official/reference/field_only_v4_chunked_triton_wiki100.py, "canon"):
+//   fl_field_params         canon:1169-1173   transition parameters, and norm weights as fp32
+//   fl_gate_residual_norm   canon:1193-1195 and 1219-1221, RMSNorm 300-309
+//   fl_swiglu               canon:312-325
+// Each value is rounded exactly where the stock ops round it: an op on bf16 tensors computes in
+// fp32 and rounds its result to bf16.
+#include "fl_common.h"
+
+namespace {
+
+using namespace fl;
+
+// Sigmoid of a value that is then rounded to T. For bf16 one v_exp_f32 and one v_rcp_f32: their
+// relative error (below 2e-6 over the range where the result is a normal number) is far below the
+// 2^-9 of the rounding that follows. For fp32 the library exponential and a true division.
+template <typename T>
+__device__ __forceinline__ float sigmoid_for(float x);
+template <>
+__device__ __forceinline__ float sigmoid_for<float>(float x) { return 1.0f / (1.0f + expf(-x)); }
+template <>
+__device__ __forceinline__ float sigmoid_for<bf16_bits>(float x) {
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -kLog2e));
+}
+template <typename T>
+__device__ __forceinline__ float silu_for(float x);
+template <>
+__device__ __forceinline__ float silu_for<float>(float x) { return x / (1.0f + expf(-x)); }
+template <>
+__device__ __forceinline__ float silu_for<bf16_bits>(float x) { return x * sigmoid_for<bf16_bits>(x); }
+
+// N norm weights of either type as fp32
+template <int N>
+__device__ __forceinline__ void load_weight(const void* w, int w16, int c, float* o) {
+  if (w16) {
+    Vec<bf16_bits, N>::load(static_cast<const bf16_bits*>(w) + c, o);
+  } else {
+    Vec<float, N>::load(static_cast<const float*>(w) + c, o);
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// gate = sigmoid(g), prod = out * gate (in the GEMM output type G), x1 = x + prod (in the
+// residual type X), h = RMSNorm(x1) * w (fp32 math, rounded to X).
+// Bound by memory at prefill sizes (five [rows, dim] streams) and by the launch at decode sizes.
+// One wave per row: the row's sum needs shuffles only, no barrier, and with N = 8 every access is
+// 16 bytes per lane (bf16). NV > 0: the row's values stay in registers (dim <= 64 * N * NV);
+// NV = 0 forms them twice. Rows 8,192 x dim 1,024, bf16 (84 MB): 14.0 us, 6.0 TB/s; one 256-thread
+// block per row with 2-byte accesses took 19.2 us.
+// ------------------------------------------------------------------------------------------
+template <typename XT, typename GT, int N, int NV>
+__global__ __launch_bounds__(256) void fl_gate_residual_norm_kernel(
+    const XT* __restrict__ x, const GT* __restrict__ out, const GT* __restrict__ gpre,
+    int64_t gstride, int64_t rows, int dim, const void* __restrict__ w, int w16, float eps,
+    float inv_dim, XT* __restrict__ x_new, XT* __restrict__ normed) {
+  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t base = row * dim;
+  const GT* grow = gpre + row * gstride;
+  auto residual = [&](int c, float* v) {
+    float g[N], o[N], xx[N];
+    Vec<GT, N>::load(grow + c, g);
+    Vec<GT, N>::load(out + base + c, o);
+    Vec<XT, N>::load(x + base + c, xx);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      v[j] = round_as<XT>(xx[j] + round_as<GT>(o[j] * round_as<GT>(sigmoid_for<GT>(g[j]))));
+  };
+  auto finish = [&](int c, const float* v, float scale) {
+    float ww[N], h[N];
+    load_weight<N>(w, w16, c, ww);
+#pragma unroll
+    for (int j = 0; j < N; ++j) h[j] = (v[j] * scale) * ww[j];
+    Vec<XT, N>::store(x_new + base + c, v);
+    Vec<XT, N>::store(normed + base + c, h);
+  };
+  float acc = 0.f;
+  if constexpr (NV > 0) {
+    float v[NV][N];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * 64 + lane) * N;
+      if (c < dim) {
+        residual(c, v[i]);
+#pragma unroll
+        for (int j = 0; j < N; ++j) acc = fmaf(v[i][j], v[i][j], acc);
+      }
+    }
+    const float scale = rsqrtf(fmaf(wave_sum(acc), inv_dim, eps));
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * 64 + lane) * N;
+      if (c < dim) finish(c, v[i], scale);
+    }
+  } else {
+    for (int c = lane * N; c < dim; c += 64 * N) {
+      float v[N];
+      residual(c, v);
+#pragma unroll
+      for (int j = 0; j < N; ++j) acc = fmaf(v[j], v[j], acc);
+    }
+    const float scale = rsqrtf(fmaf(wave_sum(acc), inv_dim, eps));
+    for (int c = lane * N; c < dim; c += 64 * N) {
+      float v[N];
+      residual(c, v);
+      finish(c, v, scale);
+    }
+  }
+}
+
+template <typename XT, typename GT>
+int launch_gate_residual_norm(const void* x, const void* out, const void* gate_pre, int64_t rows,
+                              int64_t dim, int64_t gate_stride, const void* w, int w16, float eps,
+                              void* x_new, void* normed, hipStream_t s) {
+  const float inv = (float)(1.0 / (double)dim);
+  // four rows per block once that still gives every CU several blocks; below, one row per block,
+  // so that the rows of a decode batch spread over as many CUs as there are rows
+  const unsigned waves = rows >= 4096 ? 4 : 1;
+  const unsigned blocks = (unsigned)cdiv(rows, waves);
+#define FL_GRN1(N, NV)                                                                          \
+  {                                                                                             \
+    fl_gate_residual_norm_kernel<XT, GT, N, NV><<<blocks, waves * 64, 0, s>>>(                  \
+        static_cast<const XT*>(x), static_cast<const GT*>(out), static_cast<const GT*>(gate_pre), \
+        gate_stride, rows, (int)dim, w, w16, eps, inv, static_cast<XT*>(x_new),                 \
+        static_cast<XT*>(normed));                                                              \
+    return hip_status(hipGetLastError());                                                       \
+  }
+  // 16-byte accesses: whole vectors per row and every row start aligned
+  const bool vec = dim % 8 == 0 && gate_stride % 8 == 0 && aligned(x, 16) && aligned(out, 16) &&
+                   aligned(gate_pre, 16) && aligned(w, 16) && aligned(x_new, 16) && aligned(normed, 16);
+  if (vec) {
+    if (dim <= 512) FL_GRN1(8, 1)
+    if (dim <= 1024) FL_GRN1(8, 2)
+    if (dim <= 2048) FL_GRN1(8, 4)
+    FL_GRN1(8, 0)
+  }
+  if (dim <= 512) FL_GRN1(1, 8)
+  FL_GRN1(1, 0)
+#undef FL_GRN1
+}
+
+// ------------------------------------------------------------------------------------------
+// out = silu(gate) * up with [gate | up] = the packed GEMM output, 3 * rows * hidden elements
+// moved: bound by memory. 8 elements (16 bytes of bf16) per thread and access.
+// Rows 8,192 x hidden 2,528, bf16 (124 MB): 21.2 us, 5.9 TB/s with part of it in the Infinity Cache;
+// one element per thread with a 64-bit division for its row took 43.0 us.
+// ------------------------------------------------------------------------------------------
+template <typename T>
+__global__ __launch_bounds__(256) void fl_swiglu_vec_kernel(const T* __restrict__ gu, uint32_t n_vec,
+                                                            uint32_t row_vecs, int hidden,
+                                                            T* __restrict__ out) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n_vec) return;
+  const uint32_t r = i / row_vecs;
+  const T* p = gu + (int64_t)r * hidden + (int64_t)i * 8;  // row r of 2 * hidden, column 8 * (i % row_vecs)
+  float g[8], u[8], o[8];
+  Vec<T, 8>::load(p, g);
+  Vec<T, 8>::load(p + hidden, u);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = round_as<T>(silu_for<T>(g[j])) * u[j];
+  Vec<T, 8>::store(out + (int64_t)i * 8, o);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void fl_swiglu_kernel(const T* __restrict__ gu, int64_t rows,
+                                                        int hidden, T* __restrict__ out) {
+  const int64_t n = rows * hidden;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = i / hidden;
+    const int j = (int)(i - r * hidden);
+    const float g = load_as<T>(gu + r * 2 * hidden + j);
+    const float u = load_as<T>(gu + r * 2 * hidden + hidden + j);
+    store_as(out + i, round_as<T>(silu_for<T>(g)) * u);
+  }
+}
+
+template <typename T>
+int launch_swiglu(const void* gate_up, int64_t rows, int64_t hidden, void* out, hipStream_t s) {
+  const T* gu = static_cast<const T*>(gate_up);
+  T* o = static_cast<T*>(out);
+  const int64_t n = rows * hidden;
+  if (hidden % 8 == 0 && aligned(gate_up, 16) && aligned(out, 16) && n / 8 < ((int64_t)1 << 31)) {
+    fl_swiglu_vec_kernel<T><<<(unsigned)cdiv(n / 8, 256), 256, 0, s>>>(gu, (uint32_t)(n / 8),
+                                                                       (uint32_t)(hidden / 8), (int)hidden, o);
+  } else {
+    const unsigned blocks = (unsigned)(cdiv(n, 256) < 4096 ? cdiv(n, 256) : 4096);
+    fl_swiglu_kernel<T><<<blocks, 256, 0, s>>>(gu, rows, (int)hidden, o);
+  }
+  return hip_status(hipGetLastError());
+}
+
+// ------------------------------------------------------------------------------------------
+// Transition parameters (canon:1169-1173): radius = clamp(sigmoid(radius_logit), 0.5, 0.99995),
+// tr = radius cos(theta), ti = radius sin(theta), gamma = sqrt(max(1 - radius^2, 1e-4)); and a
+// bf16 norm weight widened to fp32. A few KB, bound by the launch: one launch where the stock ops
+// take twelve of 3.5-4.3 us each (C = 512: 4.2 us against 45 us).
+// ------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void fl_field_params_kernel(
+    const float* __restrict__ radius_logit, const float* __restrict__ theta, int C,
+    const bf16_bits* __restrict__ w16, int n_w, float* __restrict__ tr, float* __restrict__ ti,
+    float* __restrict__ gamma, float* __restrict__ w32) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < C) {
+    // no contraction: products and sums round separately, as the stock ops do
+#pragma clang fp contract(off)
+    const float sg = 1.0f / (1.0f + expf(-radius_logit[i]));
+    // a NaN logit stays NaN, as through the stock clamp
+    const float r = sg != sg ? sg : fminf(fmaxf(sg, 0.50f), 0.99995f);
+    const float th = theta[i];
+    tr[i] = r * cosf(th);
+    ti[i] = r * sinf(th);
+    const float sq = r * r;
+    const float d = 1.0f - sq;
+    gamma[i] = d != d ? d : sqrtf(fmaxf(d, 1e-4f));
+  }
+  if (i < n_w) w32[i] = __uint_as_float((uint32_t)w16[i] << 16);
+}
+
+}  // namespace
+
+extern "C" {
+
+int fl_gate_residual_norm_w(const void* x, int x_dtype, const void* out, const void* gate_pre,
+                            int g_dtype, int64_t rows, int64_t dim, int64_t gate_stride,
+                            const void* norm_weight, int w_dtype, float eps, void* x_new,
+                            void* normed, void* stream) {
+  if (!dtype_ok(x_dtype) || !dtype_ok(g_dtype) || !dtype_ok(w_dtype)) return FL_ERR_DTYPE;
+  if (rows <= 0 || dim <= 0 || rows > ((int64_t)1 << 31) - 1 || dim > ((int64_t)1 << 24))
+    return FL_ERR_INVALID_ARGUMENT;
+  if (gate_stride < dim || gate_stride > ((int64_t)1 << 31)) return FL_ERR_INVALID_ARGUMENT;
+  if (!x || !out || !gate_pre || !norm_weight || !x_new || !normed || !(eps >= 0.f))
+    return FL_ERR_INVALID_ARGUMENT;
+  const size_t xs = esize(x_dtype), gs = esize(g_dtype);
+  if (!aligned(x, xs) || !aligned(x_new, xs) || !aligned(normed, xs) || !aligned(out, gs) ||
+      !aligned(gate_pre, gs) || !aligned(norm_weight, esize(w_dtype)))
+    return FL_ERR_INVALID_ARGUMENT;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool x16 = x_dtype == FL_DTYPE_BF16, g16 = g_dtype == FL_DTYPE_BF16;
+  const int w16 = w_dtype == FL_DTYPE_BF16;
+#define FL_GRN(X, G) \
+  return launch_gate_residual_norm<X, G>(x, out, gate_pre, rows, dim, gate_stride, norm_weight, w16, eps, x_new, normed, s);
+  if (x16 && g16) { FL_GRN(bf16_bits, bf16_bits) }
+  if (x16) { FL_GRN(bf16_bits, float) }
+  if (g16) { FL_GRN(float, bf16_bits) }
+  FL_GRN(float, float)
+#undef FL_GRN
+}
+
+int fl_gate_residual_norm(const void* x, int x_dtype, const void* out, const void* gate_pre,
+                          int g_dtype, int64_t rows, int64_t dim, int64_t gate_stride,
+                          const float* norm_weight, float eps, void* x_new, void* normed,
+                          void* stream) {
+  return fl_gate_residual_norm_w(x, x_dtype, out, gate_pre, g_dtype, rows, dim, gate_stride,
+                                 norm_weight, FL_DTYPE_F32, eps, x_new, normed, stream);
+}
+
+int fl_swiglu(const void* gate_up, int dtype, int64_t rows, int64_t hidden, void* out,
+              void* stream) {
+  if (!dtype_ok(dtype)) return FL_ERR_DTYPE;
+  if (rows <= 0 || hidden <= 0 || hidden > ((int64_t)1 << 30)) return FL_ERR_INVALID_ARGUMENT;
+  if (!gate_up || !out) return FL_ERR_INVALID_ARGUMENT;
+  if (!aligned(gate_up, esize(dtype)) || !aligned(out, esize(dtype))) return FL_ERR_INVALID_ARGUMENT;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == FL_DTYPE_BF16 ? launch_swiglu<bf16_bits>(gate_up, rows, hidden, out, s)
+                                : launch_swiglu<float>(gate_up, rows, hidden, out, s);
+}
+
+int fl_field_params(const float* radius_logit, const float* theta, int64_t C, const void* weight16,
+                    int64_t n_weight, float* tr, float* ti, float* gamma, float* weight32,
+                    void* stream) {
+  if (C <= 0 || C > ((int64_t)1 << 24) || n_weight < 0 || n_weight > ((int64_t)1 << 26))
+    return FL_ERR_INVALID_ARGUMENT;
+  if (!radius_logit || !theta || !tr || !ti || !gamma) return FL_ERR_INVALID_ARGUMENT;
+  if (n_weight > 0 && (!weight16 || !weight32)) return FL_ERR_INVALID_ARGUMENT;
+  if (!aligned(radius_logit, 4) || !aligned(theta, 4) || !aligned(tr, 4) || !aligned(ti, 4) ||
+      !aligned(gamma, 4) || !aligned(weight32, 4) || !aligned(weight16, 2))
+    return FL_ERR_INVALID_ARGUMENT;
+  const int64_t n = C > n_weight ? C : n_weight;
+  fl_field_params_kernel<<<(unsigned)cdiv(n, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+      radius_logit, theta, (int)C, static_cast<const bf16_bits*>(weight16), (int)n_weight, tr, ti,
+      gamma, weight32);
+  return hip_status(hipGetLastError());
+}
+
+}  // extern "C"

@@ -136,9 +136,12 @@ def field_scan_norm(raw: torch.Tensor, transition_r: torch.Tensor, transition_i:
     weight: [4C] (the mixer's ``read_norm.weight``). out_dtype fp32, or bf16 (the fp32 value
     rounded to nearest even, as bf16 autocast hands it to out_proj). C <= 4096.
     """
+    if raw.is_cuda:
+        weight = _norm_weight(weight, raw.shape[-1] // 3, raw.device)  # shape check before any launch
+
     def launch(lib, a):
         raw_, batch, length, channels, tr, ti, gm, sin, sout, out, ws = a
-        w = _norm_weight(weight, channels, raw_.device)
+        w = weight
         code = lib.fl_scan_norm_forward(
             nat.ptr(raw_), nat.dtype_code(raw_.dtype), batch, length, channels,
             raw_.stride(0), raw_.stride(1), nat.ptr(tr), nat.ptr(ti), nat.ptr(gm), nat.ptr(sin),
@@ -147,8 +150,6 @@ def field_scan_norm(raw: torch.Tensor, transition_r: torch.Tensor, transition_i:
         nat.check(code, "fl_scan_norm_forward")
         nat.check_waits(ws, "fl_scan_norm_forward")
 
-    if raw.is_cuda:
-        _norm_weight(weight, raw.shape[-1] // 3, raw.device)  # shape check before any launch
     return _scan_call(raw, transition_r, transition_i, gamma, state_in, return_state, out_dtype,
                       launch)
 
@@ -401,15 +402,18 @@ def gate_residual_norm(x: torch.Tensor, out: torch.Tensor, gate_pre: torch.Tenso
     if gate_stride is None:
         gate_pre = gate_pre.contiguous()
         gate_stride = dim
-    w = weight.detach().to(device=x.device, dtype=torch.float32).contiguous()
+    w = weight.detach()
+    if w.dtype != torch.bfloat16 or w.device != x.device:  # a bf16 weight is widened in the kernel
+        w = w.to(device=x.device, dtype=torch.float32)
+    w = w.contiguous()
     x_new, normed = torch.empty_like(x), torch.empty_like(x)
     rows = x.numel() // dim if dim else 0
     if rows == 0:
         return x_new, normed
-    code = lib.fl_gate_residual_norm(nat.ptr(x), nat.dtype_code(x.dtype), nat.ptr(out), nat.ptr(gate_pre),
-                                     nat.dtype_code(out.dtype), rows, dim, gate_stride, nat.ptr(w),
-                                     ctypes.c_float(float(eps)), nat.ptr(x_new), nat.ptr(normed),
-                                     nat.stream_handle(x.device))
+    code = lib.fl_gate_residual_norm_w(nat.ptr(x), nat.dtype_code(x.dtype), nat.ptr(out), nat.ptr(gate_pre),
+                                       nat.dtype_code(out.dtype), rows, dim, gate_stride, nat.ptr(w),
+                                       nat.dtype_code(w.dtype), ctypes.c_float(float(eps)), nat.ptr(x_new),
+                                       nat.ptr(normed), nat.stream_handle(x.device))
     nat.check(code, "fl_gate_residual_norm")
     return x_new, normed
 
@@ -516,12 +520,39 @@ class IndependentVacancyField(nn.Module):
 
     def transition(self) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
         """(tr, ti, gamma) fp32 [C] (canon:1169-1173), computed in the parameters' dtype."""
+        if self._native_params():
+            return self._scan_params()[:3]
         radius = torch.sigmoid(self.radius_logit).clamp(0.50, 0.99995).float()
         theta = self.theta.float()
         tr = radius * torch.cos(theta)
         ti = radius * torch.sin(theta)
         gamma = torch.sqrt((1.0 - radius.square()).clamp_min(1e-4))
         return tr.contiguous(), ti.contiguous(), gamma.contiguous()
+
+    def _native_params(self) -> bool:
+        """The transition parameters from one launch (fl_field_params): fp32 parameters on the
+        device that no gradient flows to."""
+        p, q = self.radius_logit, self.theta
+        return (p.is_cuda and q.device == p.device and p.dtype == torch.float32 and q.dtype == torch.float32
+                and p.shape == q.shape and p.ndim == 1 and p.numel() > 0 and p.is_contiguous() and q.is_contiguous()
+                and not (torch.is_grad_enabled() and (p.requires_grad or q.requires_grad)))
+
+    def _scan_params(self) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+        """(tr, ti, gamma, read_norm weight), all fp32: what the fused scan and step read. One
+        launch where :meth:`_native_params` holds, a bf16 norm weight widened in the same one."""
+        w = self.read_norm.weight.detach()
+        if not self._native_params():
+            return (*self.transition(), w.float().contiguous())
+        lib, c, p = nat.load(), self.radius_logit.numel(), self.radius_logit
+        widen = w.dtype == torch.bfloat16 and w.device == p.device and w.is_contiguous()
+        n_w = w.numel() if widen else 0
+        buf = torch.empty(3 * c + n_w, device=p.device, dtype=torch.float32)
+        tr, ti, gamma, w32 = buf.split((c, c, c, n_w))
+        code = lib.fl_field_params(nat.ptr(p), nat.ptr(self.theta), c, nat.ptr(w) if widen else None, n_w,
+                                   nat.ptr(tr), nat.ptr(ti), nat.ptr(gamma), nat.ptr(w32) if widen else None,
+                                   nat.stream_handle(p.device))
+        nat.check(code, "fl_field_params")
+        return tr, ti, gamma, w32 if widen else w.float().contiguous()
 
     def _raw(self, x: torch.Tensor, raw: Optional[torch.Tensor] = None) -> torch.Tensor:
         # bf16 (autocast) and fp32 raw go to the kernel as they are; the kernel's upcast of
@@ -588,11 +619,12 @@ class IndependentVacancyField(nn.Module):
     def normed_read(self, x: torch.Tensor, raw: Optional[torch.Tensor] = None) -> torch.Tensor:
         """read_norm(read) of the scan of x: what out_proj consumes (``raw`` = write_proj(x) when
         already computed)."""
-        tr, ti, gamma = self.transition()
         raw = self._raw(x, raw)
         if self._fused(x):
-            return _FieldNormReadFunction.apply(raw, tr, ti, gamma, self.read_norm.weight,
-                                                self.read_norm.eps, self._read_dtype(raw))
+            tr, ti, gamma, weight = self._scan_params()
+            return _FieldNormReadFunction.apply(raw, tr, ti, gamma, weight, self.read_norm.eps,
+                                                self._read_dtype(raw))
+        tr, ti, gamma = self.transition()
         read = fused_field_read(raw, tr, ti, gamma, self.triton_block_c, self.triton_chunk_t,
                                 read_dtype=self._unfused_read_dtype())
         return self.read_norm(read)
@@ -603,11 +635,12 @@ class IndependentVacancyField(nn.Module):
     def normed_prefill(self, x: torch.Tensor, state: Optional[torch.Tensor] = None,
                        raw: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
         """read_norm(read) over [B,T,dim] and the recurrent state s[T-1] (fp32 [B,2C])."""
-        tr, ti, gamma = self.transition()
         raw = self._raw(x, raw)
         if self._fused(x):
-            return field_scan_norm(raw, tr, ti, gamma, self.read_norm.weight, self.read_norm.eps,
+            tr, ti, gamma, weight = self._scan_params()
+            return field_scan_norm(raw, tr, ti, gamma, weight, self.read_norm.eps,
                                    state_in=state, return_state=True, out_dtype=self._read_dtype(raw))
+        tr, ti, gamma = self.transition()
         read, new_state = field_scan(raw, tr, ti, gamma, state_in=state, return_state=True,
                                      read_dtype=self._unfused_read_dtype())
         return self.read_norm(read), new_state
@@ -624,7 +657,7 @@ class IndependentVacancyField(nn.Module):
     def decode_params(self) -> Tuple[torch.Tensor, ...]:
         """(tr, ti, gamma, read_norm weight in fp32): what :meth:`step` reads, cached once per
         decode loop."""
-        return (*self.transition(), self.read_norm.weight.detach().float().contiguous())
+        return self._scan_params()
 
     def step(self, x_t: torch.Tensor, state: torch.Tensor,
              params: Optional[Tuple[torch.Tensor, ...]] = None) -> torch.Tensor:
@@ -650,6 +683,34 @@ class IndependentVacancyField(nn.Module):
 
     def new_state(self, batch: int, device=None) -> torch.Tensor:
         return torch.zeros((batch, 2 * self.channels), device=device, dtype=torch.float32)
+
+
+def _plain_linear(layer: nn.Module) -> bool:
+    """An nn.Linear whose call is nothing but its GEMM: no subclass or parametrisation, no hook, no
+    replaced forward, an ordinary weight. Only such a layer's GEMM may be run other than by
+    calling it."""
+    m = nn.modules.module
+    return (type(layer) is nn.Linear and "forward" not in layer.__dict__
+            and type(layer.weight) in (nn.Parameter, torch.Tensor)
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
+                     or layer._backward_pre_hooks or m._global_forward_hooks or m._global_forward_pre_hooks))
+
+
+def _autocast_keeps(dtype: torch.dtype) -> bool:
+    """Whether a linear layer on ``dtype`` operands runs in ``dtype`` (autocast off, or to it)."""
+    return not torch.is_autocast_enabled() or torch.get_autocast_dtype("cuda") == dtype
+
+
+def _linear_residual(x: torch.Tensor, layer: nn.Module, h: torch.Tensor) -> torch.Tensor:
+    """``x + layer(h)`` for a contiguous ``x`` that the caller owns. A plain bias-free layer of x's
+    dtype accumulates onto x inside its GEMM (one rounding instead of two, and no add launch); any
+    other layer is called as it is."""
+    if _plain_linear(layer) and layer.bias is None and not torch.is_grad_enabled() \
+            and x.dtype == h.dtype == layer.weight.dtype and _autocast_keeps(x.dtype) \
+            and layer.weight.shape == (x.shape[-1], h.shape[-1]):
+        x.view(-1, x.shape[-1]).addmm_(h.view(-1, h.shape[-1]), layer.weight.t())
+        return x
+    return x + layer(h)
 
 
 class FieldBlock(nn.Module):
@@ -678,7 +739,7 @@ class FieldBlock(nn.Module):
         m = self.mixer
         x1, h = gate_residual_norm(x, m.out_proj(normed), gate_pre, self.ff_norm.weight, self.ff_norm.eps)
         first, second = (self.ff.w12, self.ff.w3) if hasattr(self.ff, "w12") else (self.ff.gate_up, self.ff.down)
-        return x1 + second(swiglu(first(h)))
+        return _linear_residual(x1, second, swiglu(first(h)))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._fused_tail(x):

@@ -246,6 +246,24 @@ int fl_gate_residual_norm(const void* x, int x_dtype, const void* out, const voi
                           const float* norm_weight, float eps, void* x_new, void* normed,
                           void* stream);
 
+/* fl_gate_residual_norm with norm_weight of either element type (w_dtype): the bf16 values are
+ * widened exactly, as the stock RMSNorm's weight.float() does. */
+int fl_gate_residual_norm_w(const void* x, int x_dtype, const void* out, const void* gate_pre,
+                            int g_dtype, int64_t rows, int64_t dim, int64_t gate_stride,
+                            const void* norm_weight, int w_dtype, float eps, void* x_new,
+                            void* normed, void* stream);
+
+/*
+ * Transition parameters of the Field mixer (field_only_v4_chunked_triton_wiki100.py:1169-1173),
+ * fp32 [C] each: radius = clamp(sigmoid(radius_logit), 0.5, 0.99995), tr = radius cos(theta),
+ * ti = radius sin(theta), gamma = sqrt(max(1 - radius^2, 1e-4)). With n_weight > 0, weight32
+ * [n_weight] also receives the bf16 vector weight16 as fp32 (the read_norm weight, which the scan
+ * takes in fp32); weight16 / weight32 may be NULL when n_weight is 0.
+ */
+int fl_field_params(const float* radius_logit, const float* theta, int64_t C, const void* weight16,
+                    int64_t n_weight, float* tr, float* ti, float* gamma, float* weight32,
+                    void* stream);
+
 /*
  * SwiGLU activation of the Field block FFN (PackedSwiGLU.forward, same file 312-325):
  * out[r, j] = silu(gate_up[r, j]) * gate_up[r, hidden + j], [rows, 2*hidden] -> [rows, hidden].
