@@ -19,7 +19,9 @@ from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
-SOURCES = [PKG_DIR / "csrc" / name for name in ("field_scan.hip", "block_tail.hip")]
+SOURCES = [PKG_DIR / "csrc" / name for name in ("field_scan.hip", "block_tail.hip", "field_params.hip")]
+# what a source needs beside HIP_FLAGS (a later flag of a kind replaces an earlier one)
+SOURCE_FLAGS = {"field_params.hip": ["-ffp-contract=on"]}
 INCLUDE_DIR = REPO_DIR / "include"
 LIB_PATH = PKG_DIR / "libfields_amd.so"
 # measurement kernels for bench.py (the scan's access pattern without its arithmetic), kept out of
@@ -71,7 +73,7 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None, out: Path
         objects = [str(Path(work) / f"{i}_{s.stem}.o") for i, s in enumerate(sources or SOURCES)]
         compile_flags = [f for f in flags if f != "-shared"]
         with ThreadPoolExecutor(max_workers=4) as pool:
-            list(pool.map(run, [[hipcc(), *compile_flags, "-c", str(s), "-o", o]
+            list(pool.map(run, [[hipcc(), *compile_flags, *SOURCE_FLAGS.get(Path(s).name, []), "-c", str(s), "-o", o]
                                 for s, o in zip(sources or SOURCES, objects)]))
         run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", str(tmp)])
     missing = unresolved_kernel_stubs(tmp)

@@ -1,6 +1,5 @@
 // block_tail.hip — the Field block's elementwise work around its GEMMs and its scan
 // (reference: src/fields_official/reference/field_only_v4_chunked_triton_wiki100.py, "canon"):
-//   fl_field_params         canon:1169-1173   transition parameters, and norm weights as fp32
 //   fl_gate_residual_norm   canon:1193-1195 and 1219-1221, RMSNorm 300-309
 //   fl_swiglu               canon:312-325
 // Each value is rounded exactly where the stock ops round it: an op on bf16 tensors computes in
@@ -11,23 +10,24 @@ namespace {
 
 using namespace fl;
 
-// Sigmoid of a value that is then rounded to T. For bf16 one v_exp_f32 and one v_rcp_f32: their
-// relative error (below 2e-6 over the range where the result is a normal number) is far below the
-// 2^-9 of the rounding that follows. For fp32 the library exponential and a true division.
+// sigmoid and silu of a loaded T. Of a bf16 value the sigmoid is one v_exp_f32 and one v_rcp_f32:
+// compared over all 65,536 inputs, its bf16 rounding is the library form's except at -87.5, -88 and
+// -88.5, where that is a denormal (below 1.1e-38) and this is 0. The plain form of silu would miss one
+// more (5.9375), so it takes the residual step. fp32 keeps the library exponential and division.
 template <typename T>
-__device__ __forceinline__ float sigmoid_for(float x);
+__device__ __forceinline__ float sigmoid(float x);
 template <>
-__device__ __forceinline__ float sigmoid_for<float>(float x) { return 1.0f / (1.0f + expf(-x)); }
+__device__ __forceinline__ float sigmoid<float>(float x) { return 1.0f / (1.0f + expf(-x)); }
 template <>
-__device__ __forceinline__ float sigmoid_for<bf16_bits>(float x) {
+__device__ __forceinline__ float sigmoid<bf16_bits>(float x) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -kLog2e));
 }
 template <typename T>
-__device__ __forceinline__ float silu_for(float x);
+__device__ __forceinline__ float silu(float x);
 template <>
-__device__ __forceinline__ float silu_for<float>(float x) { return x / (1.0f + expf(-x)); }
+__device__ __forceinline__ float silu<float>(float x) { return x / (1.0f + expf(-x)); }
 template <>
-__device__ __forceinline__ float silu_for<bf16_bits>(float x) { return x * sigmoid_for<bf16_bits>(x); }
+__device__ __forceinline__ float silu<bf16_bits>(float x) { return silu_precise(x); }
 
 // N norm weights of either type as fp32
 template <int N>
@@ -43,68 +43,77 @@ __device__ __forceinline__ void load_weight(const void* w, int w16, int c, float
 // gate = sigmoid(g), prod = out * gate (in the GEMM output type G), x1 = x + prod (in the
 // residual type X), h = RMSNorm(x1) * w (fp32 math, rounded to X).
 // Bound by memory at prefill sizes (five [rows, dim] streams) and by the launch at decode sizes.
-// One wave per row: the row's sum needs shuffles only, no barrier, and with N = 8 every access is
-// 16 bytes per lane (bf16). NV > 0: the row's values stay in registers (dim <= 64 * N * NV);
-// NV = 0 forms them twice. Rows 8,192 x dim 1,024, bf16 (84 MB): 14.0 us, 6.0 TB/s; one 256-thread
-// block per row with 2-byte accesses took 19.2 us.
+// One wave per row, 16 bytes per lane and access with N = 8 (bf16). The sum of squares keeps one
+// order for every N and launch shape: 256 strided chains over the row (c = i, i + 256, ...), each
+// 64 of them added by a butterfly, the four sums in sequence; the row's values reach their chains
+// through LDS (RES floats per wave; longer rows in pieces). So a row's result does not depend on
+// its alignment or on the size of the batch. Rows 8,192 x dim 1,024, bf16 (84 MB): 14.2 us,
+// 5.9 TB/s; one 256-thread block per row with 2-byte accesses and a library sigmoid took 19.2 us.
 // ------------------------------------------------------------------------------------------
-template <typename XT, typename GT, int N, int NV>
+template <typename XT, typename GT, int N, int RES>
 __global__ __launch_bounds__(256) void fl_gate_residual_norm_kernel(
     const XT* __restrict__ x, const GT* __restrict__ out, const GT* __restrict__ gpre,
     int64_t gstride, int64_t rows, int dim, const void* __restrict__ w, int w16, float eps,
     float inv_dim, XT* __restrict__ x_new, XT* __restrict__ normed) {
+  constexpr int NV = RES / (64 * N);  // accesses per piece and lane
+  extern __shared__ float s_rows[];
   const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  if (row >= rows) return;  // whole waves; no barrier follows
   const int lane = threadIdx.x & 63;
+  float* s_row = s_rows + (threadIdx.x >> 6) * RES;
   const int64_t base = row * dim;
   const GT* grow = gpre + row * gstride;
-  auto residual = [&](int c, float* v) {
-    float g[N], o[N], xx[N];
+  float v[NV][N];
+  auto residual = [&](int c, float* o) {
+    float g[N], y[N], xx[N];
     Vec<GT, N>::load(grow + c, g);
-    Vec<GT, N>::load(out + base + c, o);
+    Vec<GT, N>::load(out + base + c, y);
     Vec<XT, N>::load(x + base + c, xx);
 #pragma unroll
     for (int j = 0; j < N; ++j)
-      v[j] = round_as<XT>(xx[j] + round_as<GT>(o[j] * round_as<GT>(sigmoid_for<GT>(g[j]))));
+      o[j] = round_as<XT>(xx[j] + round_as<GT>(y[j] * round_as<GT>(sigmoid<GT>(g[j]))));
   };
-  auto finish = [&](int c, const float* v, float scale) {
-    float ww[N], h[N];
-    load_weight<N>(w, w16, c, ww);
-#pragma unroll
-    for (int j = 0; j < N; ++j) h[j] = (v[j] * scale) * ww[j];
-    Vec<XT, N>::store(x_new + base + c, v);
-    Vec<XT, N>::store(normed + base + c, h);
-  };
-  float acc = 0.f;
-  if constexpr (NV > 0) {
-    float v[NV][N];
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int c0 = 0; c0 < dim; c0 += RES) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = (i * 64 + lane) * N;
-      if (c < dim) {
-        residual(c, v[i]);
+      const int o = (i * 64 + lane) * N, c = c0 + o;
 #pragma unroll
-        for (int j = 0; j < N; ++j) acc = fmaf(v[i][j], v[i][j], acc);
+      for (int j = 0; j < N; ++j) v[i][j] = 0.f;
+      if (c < dim) residual(c, v[i]);
+#pragma unroll
+      for (int j = 0; j < N; ++j) s_row[o + j] = v[i][j];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // one wave's LDS operations complete in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int i = 0; i < RES / 256; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float q = s_row[256 * i + 64 * k + lane];
+        acc[k] = fmaf(q, q, acc[k]);
       }
-    }
-    const float scale = rsqrtf(fmaf(wave_sum(acc), inv_dim, eps));
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  float tot = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) tot += wave_sum(acc[k]);
+  const float scale = rsqrtf(fmaf(tot, inv_dim, eps));
+  for (int c0 = 0; c0 < dim; c0 += RES) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = (i * 64 + lane) * N;
-      if (c < dim) finish(c, v[i], scale);
-    }
-  } else {
-    for (int c = lane * N; c < dim; c += 64 * N) {
-      float v[N];
-      residual(c, v);
+      const int c = c0 + (i * 64 + lane) * N;
+      if (c >= dim) continue;
+      if (dim > RES) residual(c, v[i]);  // only the last piece is still held
+      float ww[N], h[N];
+      load_weight<N>(w, w16, c, ww);
 #pragma unroll
-      for (int j = 0; j < N; ++j) acc = fmaf(v[j], v[j], acc);
-    }
-    const float scale = rsqrtf(fmaf(wave_sum(acc), inv_dim, eps));
-    for (int c = lane * N; c < dim; c += 64 * N) {
-      float v[N];
-      residual(c, v);
-      finish(c, v, scale);
+      for (int j = 0; j < N; ++j) h[j] = (v[i][j] * scale) * ww[j];
+      Vec<XT, N>::store(x_new + base + c, v[i]);
+      Vec<XT, N>::store(normed + base + c, h);
     }
   }
 }
@@ -118,9 +127,9 @@ int launch_gate_residual_norm(const void* x, const void* out, const void* gate_p
   // so that the rows of a decode batch spread over as many CUs as there are rows
   const unsigned waves = rows >= 4096 ? 4 : 1;
   const unsigned blocks = (unsigned)cdiv(rows, waves);
-#define FL_GRN1(N, NV)                                                                          \
+#define FL_GRN1(N, RES)                                                                         \
   {                                                                                             \
-    fl_gate_residual_norm_kernel<XT, GT, N, NV><<<blocks, waves * 64, 0, s>>>(                  \
+    fl_gate_residual_norm_kernel<XT, GT, N, RES><<<blocks, waves * 64, waves * RES * 4, s>>>(                 \
         static_cast<const XT*>(x), static_cast<const GT*>(out), static_cast<const GT*>(gate_pre), \
         gate_stride, rows, (int)dim, w, w16, eps, inv, static_cast<XT*>(x_new),                 \
         static_cast<XT*>(normed));                                                              \
@@ -130,20 +139,18 @@ int launch_gate_residual_norm(const void* x, const void* out, const void* gate_p
   const bool vec = dim % 8 == 0 && gate_stride % 8 == 0 && aligned(x, 16) && aligned(out, 16) &&
                    aligned(gate_pre, 16) && aligned(w, 16) && aligned(x_new, 16) && aligned(normed, 16);
   if (vec) {
-    if (dim <= 512) FL_GRN1(8, 1)
-    if (dim <= 1024) FL_GRN1(8, 2)
-    if (dim <= 2048) FL_GRN1(8, 4)
-    FL_GRN1(8, 0)
+    if (dim <= 512) FL_GRN1(8, 512)
+    if (dim <= 1024) FL_GRN1(8, 1024)
+    FL_GRN1(8, 2048)
   }
-  if (dim <= 512) FL_GRN1(1, 8)
-  FL_GRN1(1, 0)
+  FL_GRN1(1, 256)
 #undef FL_GRN1
 }
 
 // ------------------------------------------------------------------------------------------
 // out = silu(gate) * up with [gate | up] = the packed GEMM output, 3 * rows * hidden elements
 // moved: bound by memory. 8 elements (16 bytes of bf16) per thread and access.
-// Rows 8,192 x hidden 2,528, bf16 (124 MB): 21.2 us, 5.9 TB/s with part of it in the Infinity Cache;
+// Rows 8,192 x hidden 2,528, bf16 (124 MB): 22.9 us, 5.4 TB/s with part of it in the Infinity Cache;
 // one element per thread with a 64-bit division for its row took 43.0 us.
 // ------------------------------------------------------------------------------------------
 template <typename T>
@@ -158,7 +165,7 @@ __global__ __launch_bounds__(256) void fl_swiglu_vec_kernel(const T* __restrict_
   Vec<T, 8>::load(p, g);
   Vec<T, 8>::load(p + hidden, u);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) o[j] = round_as<T>(silu_for<T>(g[j])) * u[j];
+  for (int j = 0; j < 8; ++j) o[j] = round_as<T>(silu<T>(g[j])) * u[j];
   Vec<T, 8>::store(out + (int64_t)i * 8, o);
 }
 
@@ -172,7 +179,7 @@ __global__ __launch_bounds__(256) void fl_swiglu_kernel(const T* __restrict__ gu
     const int j = (int)(i - r * hidden);
     const float g = load_as<T>(gu + r * 2 * hidden + j);
     const float u = load_as<T>(gu + r * 2 * hidden + hidden + j);
-    store_as(out + i, round_as<T>(silu_for<T>(g)) * u);
+    store_as(out + i, round_as<T>(silu<T>(g)) * u);
   }
 }
 
@@ -189,33 +196,6 @@ int launch_swiglu(const void* gate_up, int64_t rows, int64_t hidden, void* out, 
     fl_swiglu_kernel<T><<<blocks, 256, 0, s>>>(gu, rows, (int)hidden, o);
   }
   return hip_status(hipGetLastError());
-}
-
-// ------------------------------------------------------------------------------------------
-// Transition parameters (canon:1169-1173): radius = clamp(sigmoid(radius_logit), 0.5, 0.99995),
-// tr = radius cos(theta), ti = radius sin(theta), gamma = sqrt(max(1 - radius^2, 1e-4)); and a
-// bf16 norm weight widened to fp32. A few KB, bound by the launch: one launch where the stock ops
-// take twelve of 3.5-4.3 us each (C = 512: 4.2 us against 45 us).
-// ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void fl_field_params_kernel(
-    const float* __restrict__ radius_logit, const float* __restrict__ theta, int C,
-    const bf16_bits* __restrict__ w16, int n_w, float* __restrict__ tr, float* __restrict__ ti,
-    float* __restrict__ gamma, float* __restrict__ w32) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < C) {
-    // no contraction: products and sums round separately, as the stock ops do
-#pragma clang fp contract(off)
-    const float sg = 1.0f / (1.0f + expf(-radius_logit[i]));
-    // a NaN logit stays NaN, as through the stock clamp
-    const float r = sg != sg ? sg : fminf(fmaxf(sg, 0.50f), 0.99995f);
-    const float th = theta[i];
-    tr[i] = r * cosf(th);
-    ti[i] = r * sinf(th);
-    const float sq = r * r;
-    const float d = 1.0f - sq;
-    gamma[i] = d != d ? d : sqrtf(fmaxf(d, 1e-4f));
-  }
-  if (i < n_w) w32[i] = __uint_as_float((uint32_t)w16[i] << 16);
 }
 
 }  // namespace
@@ -265,23 +245,6 @@ int fl_swiglu(const void* gate_up, int dtype, int64_t rows, int64_t hidden, void
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == FL_DTYPE_BF16 ? launch_swiglu<bf16_bits>(gate_up, rows, hidden, out, s)
                                 : launch_swiglu<float>(gate_up, rows, hidden, out, s);
-}
-
-int fl_field_params(const float* radius_logit, const float* theta, int64_t C, const void* weight16,
-                    int64_t n_weight, float* tr, float* ti, float* gamma, float* weight32,
-                    void* stream) {
-  if (C <= 0 || C > ((int64_t)1 << 24) || n_weight < 0 || n_weight > ((int64_t)1 << 26))
-    return FL_ERR_INVALID_ARGUMENT;
-  if (!radius_logit || !theta || !tr || !ti || !gamma) return FL_ERR_INVALID_ARGUMENT;
-  if (n_weight > 0 && (!weight16 || !weight32)) return FL_ERR_INVALID_ARGUMENT;
-  if (!aligned(radius_logit, 4) || !aligned(theta, 4) || !aligned(tr, 4) || !aligned(ti, 4) ||
-      !aligned(gamma, 4) || !aligned(weight32, 4) || !aligned(weight16, 2))
-    return FL_ERR_INVALID_ARGUMENT;
-  const int64_t n = C > n_weight ? C : n_weight;
-  fl_field_params_kernel<<<(unsigned)cdiv(n, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
-      radius_logit, theta, (int)C, static_cast<const bf16_bits*>(weight16), (int)n_weight, tr, ti,
-      gamma, weight32);
-  return hip_status(hipGetLastError());
 }
 
 }  // extern "C"

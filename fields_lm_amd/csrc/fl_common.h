@@ -18,7 +18,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+// raw buffer over `bytes` from base: loads past it give 0, stores past it are dropped
+__device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
+}
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
@@ -93,10 +100,40 @@ struct Vec<bf16_bits, 8> {
   }
 };
 
+// Sum over the wave's 64 lanes, the same bits in every lane, as the butterfly of lane distances 1, 2,
+// 4, 8, 16, 32 gives them (mirrors stand for distances 4 and 8: by then their lanes hold equal
+// sums). All in vector registers: six LDS round trips of a shuffle butterfly are a serial chain.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m);
-  return v;
+  v = dpp_add<0xb1>(v);   // quad_perm [1, 0, 3, 2]
+  v = dpp_add<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+  v = dpp_add<0x141>(v);  // row_half_mirror
+  v = dpp_add<0x140>(v);  // row_mirror
+  const u32x2 a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a.x) + __uint_as_float(a.y);
+  const u32x2 b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b.x) + __uint_as_float(b.y);
+}
+
+// x / (1 + e^-x) to about an ulp: v_exp_f32 of the rounded product x log2(e) with the product's
+// rounding error put back (first order), and one residual step on v_rcp_f32's quotient. The
+// exponent is held within +-88, where e^-x is finite (its reciprocal is 0 there). Where the residual
+// is NaN (an infinite x) the plain quotient stands: inf, and NaN for -inf, as in the stock op. For
+// every bf16 x the result rounds to the stock op's bf16 value, but for 0 below -87.4, where that is
+// under 1e-36.
+__device__ __forceinline__ float silu_precise(float x) {
+  constexpr float kL = -kLog2e, kLlo = -1.9259629911266175e-8f;  // -log2(e) = kL + kLlo
+  const float xc = __builtin_amdgcn_fmed3f(x, -88.0f, 88.0f);
+  const float hi = xc * kL;
+  const float lo = fmaf(xc, kLlo, fmaf(xc, kL, -hi));
+  const float e0 = __builtin_amdgcn_exp2f(hi);
+  const float corr = fmaf(e0, lo * 0.6931471805599453f, e0);
+  const float d = 1.0f + corr, r = __builtin_amdgcn_rcpf(d), q = x * r;
+  const float res = fmaf(-q, d, x);
+  return res == res ? fmaf(res, r, q) : q;
 }
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -27,6 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _native as nat
+from ._dispatch import eager, free_rounding, no_grad_needed, plain_linear
 
 VAC_MAX = 0.90  # canon:68
 BACKENDS = ("reference", "triton", "hip")
@@ -533,9 +534,9 @@ class IndependentVacancyField(nn.Module):
         """The transition parameters from one launch (fl_field_params): fp32 parameters on the
         device that no gradient flows to."""
         p, q = self.radius_logit, self.theta
-        return (p.is_cuda and q.device == p.device and p.dtype == torch.float32 and q.dtype == torch.float32
+        return (p.dtype == torch.float32 and q.dtype == torch.float32 and no_grad_needed(p, q)
                 and p.shape == q.shape and p.ndim == 1 and p.numel() > 0 and p.is_contiguous() and q.is_contiguous()
-                and not (torch.is_grad_enabled() and (p.requires_grad or q.requires_grad)))
+                and eager(p, q))
 
     def _scan_params(self) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         """(tr, ti, gamma, read_norm weight), all fp32: what the fused scan and step read. One
@@ -685,28 +686,12 @@ class IndependentVacancyField(nn.Module):
         return torch.zeros((batch, 2 * self.channels), device=device, dtype=torch.float32)
 
 
-def _plain_linear(layer: nn.Module) -> bool:
-    """An nn.Linear whose call is nothing but its GEMM: no subclass or parametrisation, no hook, no
-    replaced forward, an ordinary weight. Only such a layer's GEMM may be run other than by
-    calling it."""
-    m = nn.modules.module
-    return (type(layer) is nn.Linear and "forward" not in layer.__dict__
-            and type(layer.weight) in (nn.Parameter, torch.Tensor)
-            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
-                     or layer._backward_pre_hooks or m._global_forward_hooks or m._global_forward_pre_hooks))
-
-
-def _autocast_keeps(dtype: torch.dtype) -> bool:
-    """Whether a linear layer on ``dtype`` operands runs in ``dtype`` (autocast off, or to it)."""
-    return not torch.is_autocast_enabled() or torch.get_autocast_dtype("cuda") == dtype
-
-
 def _linear_residual(x: torch.Tensor, layer: nn.Module, h: torch.Tensor) -> torch.Tensor:
     """``x + layer(h)`` for a contiguous ``x`` that the caller owns. A plain bias-free layer of x's
     dtype accumulates onto x inside its GEMM (one rounding instead of two, and no add launch); any
     other layer is called as it is."""
-    if _plain_linear(layer) and layer.bias is None and not torch.is_grad_enabled() \
-            and x.dtype == h.dtype == layer.weight.dtype and _autocast_keeps(x.dtype) \
+    if plain_linear(layer) and layer.bias is None and not torch.is_grad_enabled() \
+            and x.dtype == h.dtype == layer.weight.dtype and free_rounding() \
             and layer.weight.shape == (x.shape[-1], h.shape[-1]):
         x.view(-1, x.shape[-1]).addmm_(h.view(-1, h.shape[-1]), layer.weight.t())
         return x
