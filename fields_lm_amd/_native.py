@@ -59,6 +59,11 @@ SIGNATURES = {
                                        ctypes.c_float, _vp, _vp, _vp]),
     "fl_field_params": (_int, [_vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp]),
     "fl_swiglu": (_int, [_vp, _int, _i64, _i64, _vp, _vp]),
+    "fl_mamba_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "fl_mamba_prefill": (_int, [_vp, _int] + [_i64] * 5 + [_vp, _vp, _int] + [_vp] * 4 +
+                         [_int, ctypes.c_float, _vp, _int, _vp, _vp, _sz, _vp]),
+    "fl_mamba_step": (_int, [_vp, _int] + [_i64] * 3 + [_vp, _vp, _int] + [_vp] * 4 +
+                      [_int, ctypes.c_float, _vp, _vp, _vp, _int, _vp, _sz, _vp]),
     "fl_boundary_scan": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
     "fl_version": (ctypes.c_char_p, []),
 }

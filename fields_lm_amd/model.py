@@ -37,6 +37,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _native as nat
+from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_call
 from .field import FieldBlock, RMSNorm, boundary_scan
 
 # api:72-91
@@ -479,9 +481,52 @@ class Mamba2Mixer(nn.Module):
         dt = F.softplus(dt.float() + self.dt_bias.float())
         return x, bm, cm, dt
 
+    def _native(self, zxbcdt: torch.Tensor) -> bool:
+        """The kernels of ``fl_mamba_prefill`` / ``fl_mamba_step`` take this call: the promoted
+        geometry, no gradient, every tensor where and what they read."""
+        params = (self.conv1d.weight, self.conv1d.bias, self.A_log, self.dt_bias, self.D, self.norm.weight)
+        return (free_rounding() and type(self) is Mamba2Mixer and plain_call(self.norm, GatedRMSNorm)
+                and (self.headdim, self.d_state, self.d_conv) == (64, 128, 4) and self.nheads <= 1024
+                and no_grad_needed(zxbcdt, *params) and eager(zxbcdt, *params)
+                and zxbcdt.dtype in KERNEL_DTYPES and zxbcdt.is_contiguous() and zxbcdt.numel() > 0
+                and zxbcdt.shape[-1] % 2 == 0 and zxbcdt.data_ptr() % 8 == 0
+                and self.conv1d.weight.dtype == self.conv1d.bias.dtype and self.conv1d.weight.is_contiguous()
+                and self.conv1d.bias.is_contiguous() and self.norm.weight.is_contiguous()
+                and self.conv1d.weight.dtype in KERNEL_DTYPES and self.norm.weight.dtype in KERNEL_DTYPES
+                and zxbcdt.shape[0] <= 65535 and zxbcdt.shape[0] * self.nheads <= 1 << 20
+                and zxbcdt.shape[-2] <= 1 << 26)
+
+    def _native_call(self, name: str, zxbcdt: torch.Tensor, length: int, shape, strides, out_dtype, *state):
+        """Runs ``name`` (its arguments past the strides are alike); returns what out_proj reads."""
+        lib = nat.load()
+        b = zxbcdt.shape[0]
+        out = torch.empty((*zxbcdt.shape[:-1], self.d_inner), device=zxbcdt.device, dtype=out_dtype)
+        ws = torch.empty(int(lib.fl_mamba_workspace_bytes(b, length, self.nheads)), device=zxbcdt.device,
+                         dtype=torch.uint8)
+        conv = self.conv1d
+        fp32 = [t.detach().float().contiguous() for t in (self.A_log, self.dt_bias, self.D)]
+        before, after = ([], [nat.ptr(t) for t in state]) if name == "fl_mamba_prefill" \
+            else ([nat.ptr(t) for t in state], [])
+        code = getattr(lib, name)(
+            nat.ptr(zxbcdt), nat.dtype_code(zxbcdt.dtype), *shape, *strides, nat.ptr(conv.weight),
+            nat.ptr(conv.bias), nat.dtype_code(conv.weight.dtype), *[nat.ptr(t) for t in fp32],
+            nat.ptr(self.norm.weight), nat.dtype_code(self.norm.weight.dtype), self.norm.eps, *before,
+            nat.ptr(out), nat.dtype_code(out_dtype), *after, nat.ptr(ws), ws.numel(),
+            nat.stream_handle(zxbcdt.device))
+        nat.check(code, name)
+        return out
+
     def forward(self, u: torch.Tensor, return_state: bool = False):
         b, l, _ = u.shape
-        z, xbc_raw, dt = self._split(self.in_proj(u))
+        zxbcdt = self.in_proj(u)
+        z, xbc_raw, dt = self._split(zxbcdt)
+        if u.dtype in KERNEL_DTYPES and self._native(zxbcdt):
+            state = torch.empty((b, self.nheads, self.headdim, self.d_state), device=u.device,
+                                dtype=torch.float32) if return_state else None
+            out = self.out_proj(self._native_call(
+                "fl_mamba_prefill", zxbcdt, l, (b, l, self.nheads), (zxbcdt.stride(0), zxbcdt.stride(1)), u.dtype,
+                state))
+            return (out, self._new_state(xbc_raw, state)) if return_state else out
         # causal depthwise convolution as d_conv shifted multiply-adds in the channel-last
         # layout: out[t] = bias + sum_k w[k] * in[t - (d_conv-1) + k]
         w = self.conv1d.weight.float()[:, 0]                                           # [C, K]
@@ -495,12 +540,14 @@ class Mamba2Mixer(nn.Module):
         y, state = ssd_chunked(xh, dt, A, bm, cm, self.chunk_size)
         y = y + self.D.float()[:, None] * xh
         out = self.out_proj(self.norm(y.reshape(b, l, self.d_inner), z).to(u.dtype))
-        if not return_state:
-            return out
+        return (out, self._new_state(xbc_raw, state)) if return_state else out
+
+    def _new_state(self, xbc_raw: torch.Tensor, ssm: torch.Tensor) -> Dict[str, torch.Tensor]:
+        """Decode state after a sequence: the last d_conv convolution inputs and the SSM state."""
         conv = xbc_raw.transpose(1, 2)[..., -self.d_conv:].float()
         if conv.shape[-1] < self.d_conv:
             conv = F.pad(conv, (self.d_conv - conv.shape[-1], 0))
-        return out, {"conv": conv.contiguous(), "ssm": state.contiguous()}
+        return {"conv": conv.contiguous(), "ssm": ssm.contiguous()}
 
     def new_state(self, batch: int, device) -> Dict[str, torch.Tensor]:
         return {"conv": torch.zeros(batch, self.conv_dim, self.d_conv, device=device),
@@ -509,8 +556,17 @@ class Mamba2Mixer(nn.Module):
     def step(self, u_t: torch.Tensor, st: Dict[str, torch.Tensor]) -> torch.Tensor:
         """One token: u_t [B, d_model] -> [B, d_model]; conv and SSM state advance in place."""
         b = u_t.shape[0]
-        z, xbc_raw, dt = self._split(self.in_proj(u_t))
-        conv = st["conv"]
+        zxbcdt = self.in_proj(u_t)
+        conv, ssm = st["conv"], st["ssm"]
+        if (u_t.dtype in KERNEL_DTYPES and u_t.ndim == 2 and self._native(zxbcdt) and eager(conv, ssm)
+                and conv.dtype == ssm.dtype == torch.float32 and conv.is_contiguous() and ssm.is_contiguous()
+                and conv.device == ssm.device == zxbcdt.device
+                and conv.shape == (b, self.conv_dim, self.d_conv)
+                and ssm.shape == (b, self.nheads, self.headdim, self.d_state)
+                and conv.data_ptr() % 16 == 0 and ssm.data_ptr() % 16 == 0):
+            return self.out_proj(self._native_call("fl_mamba_step", zxbcdt, 1, (b, self.nheads),
+                                                   (zxbcdt.stride(0),), u_t.dtype, conv, ssm))
+        z, xbc_raw, dt = self._split(zxbcdt)
         conv.copy_(torch.roll(conv, shifts=-1, dims=-1))
         conv[..., -1] = xbc_raw.float()
         xbc = (conv * self.conv1d.weight.float()[:, 0]).sum(-1) + self.conv1d.bias.float()
@@ -518,7 +574,6 @@ class Mamba2Mixer(nn.Module):
         A = -torch.exp(self.A_log.float())
         xh = x.view(b, self.nheads, self.headdim)
         decay = torch.exp(dt * A)                                                       # [B,H]
-        ssm = st["ssm"]
         ssm.mul_(decay[:, :, None, None]).add_((xh * dt[..., None])[..., None] * bm[:, None, None, :])
         y = torch.matmul(ssm, cm[:, None, :, None]).squeeze(-1) + self.D.float()[:, None] * xh
         return self.out_proj(self.norm(y.reshape(b, self.d_inner), z).to(u_t.dtype))

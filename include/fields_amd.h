@@ -271,6 +271,35 @@ int fl_field_params(const float* radius_logit, const float* theta, int64_t C, co
 int fl_swiglu(const void* gate_up, int dtype, int64_t rows, int64_t hidden, void* out,
               void* stream);
 
+/*
+ * The Mamba-2 mixer between its projections (no gradients), geometry headdim 64, d_state 128,
+ * d_conv 4, one group (src/fields_official/reference/official_source/
+ * field_fusion_wiki100_mamba2_v25.py:73-91, 455-468): with inner = 64 heads and a row of the input
+ * projection zxbcdt = [z inner | x inner | B 128 | C 128 | dt heads],
+ *   [x | B | C] = silu(causal depthwise conv),  dt = softplus(dt + dt_bias),  A = -exp(A_log),
+ *   h_t = exp(dt_t A) h_{t-1} + dt_t x_t B_t^T,  y_t = h_t C_t + D x_t                 (per head)
+ *   out = RMSNorm(y silu(z)) norm_w       over the inner width, fp32 maths, written as out_dtype.
+ * zxbcdt [B, L, *] of dtype, rows stride_t and sequences stride_b elements apart (both even),
+ * conv_w [inner + 256, 4] and conv_b of conv_dtype, A_log / dt_bias / D [heads] fp32, norm_w [inner]
+ * of norm_dtype, out [B, L, inner] contiguous; ssm_out [B, heads, 64, 128] fp32 receives h_{L-1}
+ * (NULL: not wanted). workspace: fl_mamba_workspace_bytes(B, L, heads) bytes, 16-byte aligned, no
+ * initial contents needed.
+ *
+ * fl_mamba_step advances one token: zxbcdt [B, *], conv_state [B, inner + 256, 4] (the last four
+ * inputs, newest last) and ssm updated in place; workspace as for L = 1.
+ */
+size_t fl_mamba_workspace_bytes(int64_t B, int64_t L, int64_t heads);
+int fl_mamba_prefill(const void* zxbcdt, int dtype, int64_t B, int64_t L, int64_t heads, int64_t stride_b,
+                     int64_t stride_t, const void* conv_w, const void* conv_b, int conv_dtype,
+                     const float* A_log, const float* dt_bias, const float* D, const void* norm_w,
+                     int norm_dtype, float eps, void* out, int out_dtype, float* ssm_out,
+                     void* workspace, size_t workspace_bytes, void* stream);
+int fl_mamba_step(const void* zxbcdt, int dtype, int64_t B, int64_t heads, int64_t stride_b,
+                  const void* conv_w, const void* conv_b, int conv_dtype, const float* A_log,
+                  const float* dt_bias, const float* D, const void* norm_w, int norm_dtype, float eps,
+                  float* conv_state, float* ssm, void* out, int out_dtype, void* workspace,
+                  size_t workspace_bytes, void* stream);
+
 /* Library version string (host function). No counterpart in the reference. */
 const char* fl_version(void);
 
