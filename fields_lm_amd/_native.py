@@ -64,6 +64,12 @@ SIGNATURES = {
                          [_int, ctypes.c_float, _vp, _int, _vp, _vp, _sz, _vp]),
     "fl_mamba_step": (_int, [_vp, _int] + [_i64] * 3 + [_vp, _vp, _int] + [_vp] * 4 +
                       [_int, ctypes.c_float, _vp, _vp, _vp, _int, _vp, _sz, _vp]),
+    "fl_refresh_workspace_bytes": (_sz, [_i64] * 4),
+    "fl_refresh_attention": (_int, [_vp, _i64, _i64, _vp, _vp] + [_i64] * 7 + [_vp, _vp, _vp, _int, _vp, _vp, _sz,
+                                                                             _vp]),
+    "fl_refresh_state": (_int, [_vp] * 3 + [_i64] * 6 + [_vp] * 5),
+    "fl_latent_mean": (_int, [_vp] + [_i64] * 6 + [_vp, _vp, _vp]),
+    "fl_rms_norm": (_int, [_vp, _i64, _i64, _vp, _int, ctypes.c_float, _vp, _vp]),
     "fl_boundary_scan": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
     "fl_version": (ctypes.c_char_p, []),
 }

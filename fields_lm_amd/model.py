@@ -39,7 +39,7 @@ import torch.nn.functional as F
 
 from . import _native as nat
 from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_call
-from .field import FieldBlock, RMSNorm, boundary_scan
+from .field import FieldBlock, RMSNorm, _linear_residual, boundary_scan, gate_residual_norm, swiglu
 
 # api:72-91
 OFFICIAL_ARCHITECTURE: Mapping[str, Any] = {
@@ -70,6 +70,19 @@ LATE_FF_DELTA = 256
 # shared pieces (v20:94-163)
 # ======================================================================================
 
+def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """``fl_rms_norm``: bf16 rows of at most 4,096 (a multiple of 8), fp32 maths."""
+    x = x.contiguous()
+    if x.data_ptr() % 16:
+        x = x.clone()
+    out = torch.empty_like(x)
+    dim = x.shape[-1]
+    code = nat.load().fl_rms_norm(nat.ptr(x), x.numel() // dim, dim, nat.ptr(weight), nat.dtype_code(weight.dtype),
+                                  eps, nat.ptr(out), nat.stream_handle(x.device))
+    nat.check(code, "fl_rms_norm")
+    return out
+
+
 class NativeRMSNorm(nn.Module):
     """v20:94-104: F.rms_norm with the weight cast to the input dtype (eps 1e-6)."""
 
@@ -80,6 +93,12 @@ class NativeRMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        w = self.weight
+        if (x.dtype == torch.bfloat16 and w.dtype in KERNEL_DTYPES and free_rounding() and no_grad_needed(x, w)
+                and x.ndim > 1 and x.shape[-1] == self.dim == w.numel() and self.dim % 8 == 0 and self.dim <= 4096
+                and 0 < x.numel() < self.dim << 31 and eager(x, w) and w.is_contiguous()
+                and w.data_ptr() % 16 == 0):
+            return rms_norm(x, w, self.eps)
         return F.rms_norm(x, (self.dim,), self.weight.to(dtype=x.dtype), self.eps)
 
 
@@ -221,9 +240,57 @@ class LandmarkAttention(nn.Module):
                              torch.arange(full, device=q.device)[None, :] < chunk_of[:, None]), 1)
         return gqa_attention(q, lk, lv, allowed, False)
 
+    def _native(self, qlat: torch.Tensor) -> bool:
+        """The kernels of ``fl_refresh_attention`` take this projection [B, T, q | latent]."""
+        params = (*self.kv_up.parameters(), self.global_mix_logit)
+        rep = self.q_heads // self.kv_heads
+        return (free_rounding() and type(self) is LandmarkAttention and qlat.dtype == torch.bfloat16
+                and self.head_dim == 64 and rep in (1, 2, 4, 8) and self.kv_heads <= 4096
+                and self.local_window % 64 == 0 and self.local_window <= 1 << 20
+                and self.landmark_chunk % 32 == 0 and self.latent_dim % 8 == 0
+                and self.latent_dim <= 1 << 16 and self.global_mix_logit.dtype in KERNEL_DTYPES
+                and no_grad_needed(qlat, *params) and eager(qlat, *params) and qlat.is_contiguous()
+                and qlat.data_ptr() % 16 == 0 and qlat.numel() > 0 and qlat.shape[0] <= 65535
+                and qlat.shape[1] <= 1 << 26)
+
+    def _native_attend(self, qlat: torch.Tensor, cos, sin, max_len: Optional[int] = None):
+        """What out_proj reads, [B, T, dim], and with ``max_len`` the decode state."""
+        lib = nat.load()
+        b, length, _ = qlat.shape
+        hk, c, dev, dt = self.kv_heads, self.landmark_chunk, qlat.device, qlat.dtype
+        stream = nat.stream_handle(dev)
+        latent = qlat[..., self.q_width:]
+        full = length // c
+        mean = torch.empty((b, full, self.latent_dim), device=dev, dtype=dt)
+        tail = torch.empty((b, self.latent_dim), device=dev, dtype=torch.float32)
+        nat.check(lib.fl_latent_mean(nat.ptr(latent), qlat.stride(0), qlat.stride(1), b, length, c, self.latent_dim,
+                                     nat.ptr(mean), nat.ptr(tail), stream), "fl_latent_mean")
+        kv = self.kv_up(latent).contiguous()
+        land = self.kv_up(mean).contiguous() if full else None
+        ws = torch.empty(int(lib.fl_refresh_workspace_bytes(b, length, hk, full)), device=dev, dtype=torch.uint8)
+        y = torch.empty((b, length, self.dim), device=dev, dtype=dt)
+        nat.check(lib.fl_refresh_attention(
+            nat.ptr(qlat), qlat.stride(0), qlat.stride(1), nat.ptr(kv), nat.ptr(land), b, length, self.q_heads, hk,
+            self.local_window, full, c, nat.ptr(cos), nat.ptr(sin), nat.ptr(self.global_mix_logit),
+            nat.dtype_code(self.global_mix_logit.dtype), nat.ptr(y), nat.ptr(ws), ws.numel(), stream),
+            "fl_refresh_attention")
+        if max_len is None:
+            return y, None
+        self._rope_len = int(max_len)
+        st = {name: torch.empty(shape, device=dev, dtype=dt) for name, shape in self._state_shapes(b, max_len).items()}
+        nat.check(lib.fl_refresh_state(nat.ptr(ws), nat.ptr(kv), nat.ptr(land), b, length, hk, self.local_window, full,
+                                       st["lv"].shape[2], nat.ptr(st["kt"]), nat.ptr(st["v"]), nat.ptr(st["lkt"]),
+                                       nat.ptr(st["lv"]), stream), "fl_refresh_state")
+        st["lat_sum"] = tail
+        return y, st
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         b, length, _ = x.shape
-        qraw, latent = self.q_latent_proj(x).split((self.q_width, self.latent_dim), dim=-1)
+        qlat = self.q_latent_proj(x)
+        if self._native(qlat):
+            cos, sin = rope_cos_sin(x.device, qlat.dtype, length, self.head_dim)
+            return self.out_proj(self._native_attend(qlat, cos, sin)[0])
+        qraw, latent = qlat.split((self.q_width, self.latent_dim), dim=-1)
         kraw, vraw = self.kv_up(latent).split(self.kv_heads * self.head_dim, dim=-1)
         q, k, v = self._heads(qraw, self.q_heads), self._heads(kraw, self.kv_heads), self._heads(vraw, self.kv_heads)
         cos, sin = rope_cos_sin(x.device, x.dtype, length, self.head_dim)
@@ -235,29 +302,34 @@ class LandmarkAttention(nn.Module):
     # ---------------------------------------------------------------- incremental decode
     def new_state(self, batch: int, max_len: int, device, dtype) -> Dict[str, torch.Tensor]:
         self._rope_len = int(max_len)
+        st = {name: torch.zeros(shape, device=device, dtype=dtype)
+              for name, shape in self._state_shapes(batch, max_len).items()}
+        st["lat_sum"] = torch.zeros(batch, self.latent_dim, device=device, dtype=torch.float32)
+        return st
+
+    def _state_shapes(self, batch: int, max_len: int) -> Dict[str, Tuple[int, ...]]:
         hd, h, w = self.head_dim, self.kv_heads, self.local_window
         # landmark slots: 0 is the null slot, slot k + 1 holds chunk k's landmark. The step at
         # position p writes its own chunk's running landmark to slot p // c + 1, so positions
         # below max_len use slots up to (max_len - 1) // c + 1 (with fewer, the last chunk's
         # running landmark would land on the one before it, which later tokens read)
         n_land = (max_len - 1) // self.landmark_chunk + 1
-        return {
-            "kt": torch.zeros(batch, h, hd, w, device=device, dtype=dtype),   # keys, transposed
-            "v": torch.zeros(batch, h, w, hd, device=device, dtype=dtype),
-            "lkt": torch.zeros(batch, h, hd, 1 + n_land, device=device, dtype=dtype),
-            "lv": torch.zeros(batch, h, 1 + n_land, hd, device=device, dtype=dtype),
-            "lat_sum": torch.zeros(batch, self.latent_dim, device=device, dtype=torch.float32),
-        }
+        return {"kt": (batch, h, hd, w), "v": (batch, h, w, hd),  # keys transposed
+                "lkt": (batch, h, hd, 1 + n_land), "lv": (batch, h, 1 + n_land, hd)}
 
     def prefill(self, x: torch.Tensor, max_len: int) -> Tuple[torch.Tensor, Dict[str, torch.Tensor]]:
         """forward(x) plus the decode state after position T-1."""
         b, length, _ = x.shape
         if length + 1 > max_len:
             raise ValueError("max_len must exceed the prompt length")
-        qraw, latent = self.q_latent_proj(x).split((self.q_width, self.latent_dim), dim=-1)
+        qlat = self.q_latent_proj(x)
+        cos, sin = rope_cos_sin(x.device, x.dtype, max_len, self.head_dim)
+        if x.dtype == qlat.dtype and b * self.kv_heads <= 65535 and max_len < 1 << 24 and self._native(qlat):
+            y, st = self._native_attend(qlat, cos, sin, max_len)
+            return self.out_proj(y), st
+        qraw, latent = qlat.split((self.q_width, self.latent_dim), dim=-1)
         kraw, vraw = self.kv_up(latent).split(self.kv_heads * self.head_dim, dim=-1)
         q, k, v = self._heads(qraw, self.q_heads), self._heads(kraw, self.kv_heads), self._heads(vraw, self.kv_heads)
-        cos, sin = rope_cos_sin(x.device, x.dtype, max_len, self.head_dim)
         cl, sl = cos[:, :, :length], sin[:, :, :length]
         q, k = apply_rope(q, cl, sl), apply_rope(k, cl, sl)
         y = self._local(q, k, v)
@@ -357,16 +429,27 @@ class RefreshBlock(nn.Module):
             return torch.sigmoid(self.residual_gate_logit).to(z.dtype)
         return torch.sigmoid(self.residual_gate(z))
 
+    def _tail(self, x: torch.Tensor, z: torch.Tensor, a: torch.Tensor) -> torch.Tensor:
+        """x + gate * a, then its feed-forward. Without gradients the elementwise work runs in the
+        Field block's two kernels (gated residual with the next norm, SwiGLU activation), rounded where
+        the stock ops round, and the last product accumulates onto the residual."""
+        n2, ff = self.norm2, self.ff
+        if (x.dtype == a.dtype == torch.bfloat16 and free_rounding() and type(self) is RefreshBlock
+                and not self.light_gate and plain_call(n2, NativeRMSNorm) and plain_call(ff, GateUpSwiGLU)
+                and not torch.is_grad_enabled() and eager(x, a, n2.weight) and x.numel() > 0):
+            x, h = gate_residual_norm(x, a, self.residual_gate(z), n2.weight, n2.eps)
+            return _linear_residual(x, ff.down, swiglu(ff.gate_up(h)))
+        x = x + self._gate(z) * a
+        return x + ff(n2(x))
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         z = self.norm1(x)
-        x = x + self._gate(z) * self.attn(z)
-        return x + self.ff(self.norm2(x))
+        return self._tail(x, z, self.attn(z))
 
     def prefill(self, x: torch.Tensor, max_len: int):
         z = self.norm1(x)
         a, st = self.attn.prefill(z, max_len)
-        x = x + self._gate(z) * a
-        return x + self.ff(self.norm2(x)), st
+        return self._tail(x, z, a), st
 
     def step(self, x_t: torch.Tensor, pos: torch.Tensor, st) -> torch.Tensor:
         z = self.norm1(x_t)

@@ -300,6 +300,45 @@ int fl_mamba_step(const void* zxbcdt, int dtype, int64_t B, int64_t heads, int64
                   float* conv_state, float* ssm, void* out, int out_dtype, void* workspace,
                   size_t workspace_bytes, void* stream);
 
+/*
+ * Attention of the refresh blocks over a whole sequence (no gradients), bf16, head dimension 64
+ * (src/fields_official/reference/official_source/field_fusion_system_smoke_v21.py:131-253):
+ *   out[b,t,h,:] = local + sigmoid(mix_logit) * global,
+ * local: RoPE'd causal attention inside t's window of `window` tokens; global: attention to a null
+ * slot (score 0, value 0) and the landmarks of the chunks completed before t's.
+ * q [B, T, q_heads * 64] with row / sequence strides (multiples of 8), not yet rotated; kv
+ * [B, T, 2 * kv_heads * 64] contiguous, keys then values; landmark_kv [B, n_landmarks, 2 * kv_heads * 64]
+ * likewise (row j's key sits at position (j + 1) * landmark_chunk - 1); cos / sin [>= T, 32] bf16;
+ * q_heads / kv_heads in {1, 2, 4, 8}; window a multiple of 64, landmark_chunk of 32; mix_logit one
+ * value of mix_dtype; out [B, T, q_heads * 64]. The workspace
+ * (fl_refresh_workspace_bytes, 16-byte aligned) then holds the rotated keys, for fl_refresh_state.
+ *
+ * fl_refresh_state: from that workspace and the same kv / landmark_kv, the decode state after the
+ * sequence, zeros included: kt [B, kv_heads, 64, window] and v [B, kv_heads, window, 64] (the rows after
+ * the last whole window in slots 0 ..), lkt [B, kv_heads, 64, slots] and lv [B, kv_heads, slots, 64]
+ * (landmark j in slot j + 1; slots > n_landmarks), bf16.
+ *
+ * fl_latent_mean: mean over every completed chunk of rows, [B, T / chunk, width] bf16 (fp32 sums), and
+ * the fp32 sum of the rows after the last one, tail [B, width] (zeros if none). latent [B, T, width]
+ * bf16 with strides (multiples of 8), width a multiple of 8.
+ *
+ * fl_rms_norm: out = x rsqrt(mean x^2 + eps) weight over rows of dim (a multiple of 8, at most 4,096),
+ * bf16 with fp32 maths (field_fusion_300m_screen_v20.py:94-104).
+ */
+size_t fl_refresh_workspace_bytes(int64_t B, int64_t T, int64_t kv_heads, int64_t n_landmarks);
+int fl_refresh_attention(const void* q, int64_t q_stride_b, int64_t q_stride_t, const void* kv,
+                         const void* landmark_kv, int64_t B, int64_t T, int64_t q_heads, int64_t kv_heads,
+                         int64_t window, int64_t n_landmarks, int64_t landmark_chunk, const void* cos,
+                         const void* sin, const void* mix_logit, int mix_dtype, void* out, void* workspace,
+                         size_t workspace_bytes, void* stream);
+int fl_refresh_state(const void* workspace, const void* kv, const void* landmark_kv, int64_t B, int64_t T,
+                     int64_t kv_heads, int64_t window, int64_t n_landmarks, int64_t slots, void* kt, void* v,
+                     void* lkt, void* lv, void* stream);
+int fl_latent_mean(const void* latent, int64_t stride_b, int64_t stride_t, int64_t B, int64_t T, int64_t chunk,
+                   int64_t width, void* mean, float* tail, void* stream);
+int fl_rms_norm(const void* x, int64_t rows, int64_t dim, const void* weight, int w_dtype, float eps, void* out,
+                void* stream);
+
 /* Library version string (host function). No counterpart in the reference. */
 const char* fl_version(void);
 

@@ -1,0 +1,102 @@
+"""GPU: the refresh block's attention kernels at the edges of their query tiles, key steps, windows and
+landmark chunks, against the stock ops in fp32 on the same bf16 weights.
+
+Tolerances: no more than the stock bf16 ops are off (they round their scores too), and 2e-2 norm-wise:
+the weights are scaled so that scores reach 5 to 6, q and k carry 2^-9 each into them, so the
+probabilities move by up to 6 * 2^-8. States 1e-2.
+"""
+from __future__ import annotations
+
+import copy
+
+import pytest
+import torch
+
+from fields_lm_amd import model as M
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    return torch.device("cuda:0")
+
+
+def _norm(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30))
+
+
+def _block(dev, heads, kv, window, chunk, latent=64, seed=0):
+    torch.manual_seed(seed)
+    blk = M.RefreshBlock(64 * heads, heads, kv, latent, window, chunk, 96).to(dev)
+    with torch.no_grad():
+        blk.residual_gate.weight.normal_(0, 0.05)
+        blk.attn.global_mix_logit.fill_(0.7)
+        blk.attn.q_latent_proj.weight.mul_(3.0)  # scores that spread the softmax
+        blk.attn.kv_up.weight.mul_(3.0)
+        blk.norm2.weight.add_(0.1 * torch.randn_like(blk.norm2.weight))
+    return M.cast_for_inference(blk).eval()
+
+
+CASES = [(16, 4, 256, 256, 1, 1), (16, 4, 256, 256, 2, 31), (8, 2, 64, 32, 1, 33), (8, 2, 64, 32, 2, 64), (8, 2, 64, 32, 3, 321),
+         (4, 4, 128, 64, 2, 200), (4, 2, 192, 96, 1, 400), (8, 1, 64, 64, 1, 150), (16, 4, 512, 256, 1, 1300),
+         (12, 3, 256, 32, 1, 2100), (16, 4, 1024, 256, 1, 1025)]
+
+
+@pytest.mark.parametrize("heads,kv,window,chunk,B,T", CASES)
+def test_attention_against_fp32(dev, heads, kv, window, chunk, B, T):
+    print(f"[case] refresh attention heads={heads}/{kv} window={window} chunk={chunk} B={B} T={T}", flush=True)
+    att = _block(dev, heads, kv, window, chunk, seed=T).attn
+    ref = copy.deepcopy(att).float()
+    x = torch.randn(B, T, 64 * heads, device=dev, generator=torch.Generator(device=dev).manual_seed(T)).to(torch.bfloat16)
+    stock = att(x).detach()  # gradients enabled: the stock ops
+    with torch.no_grad():
+        y = att(x)
+        exp, st_exp = ref.prefill(x.float(), T + 70)
+        yp, st = att.prefill(x, T + 70)
+    assert torch.equal(y, yp)
+    e, e_stock = _norm(y, exp), _norm(stock, exp)
+    print(f"[case] native {e:.2e} stock {e_stock:.2e}", flush=True)
+    assert e <= 2e-2 and e <= e_stock + 1e-4
+    assert set(st) == set(st_exp)
+    for name in st:
+        assert st[name].shape == st_exp[name].shape and st[name].dtype == (torch.float32 if name == "lat_sum" else x.dtype)
+        assert torch.equal(st[name] == 0, st_exp[name] == 0) or _norm(st[name], st_exp[name]) <= 1e-2, name
+        assert _norm(st[name], st_exp[name]) <= 1e-2, name
+
+
+@pytest.mark.parametrize("T", [40, 63, 130])
+def test_block_forward_prefill_and_steps_agree(dev, T):
+    print(f"[case] refresh block T={T}", flush=True)
+    blk = _block(dev, 8, 2, 64, 32, seed=T)
+    ref = copy.deepcopy(blk).float()
+    x = torch.randn(2, T + 40, 512, device=dev, generator=torch.Generator(device=dev).manual_seed(T)).to(torch.bfloat16)
+    keep = x.clone()
+    with torch.no_grad():
+        full = blk(x)
+        y, st = blk.prefill(x[:, :T], T + 41)
+        steps = torch.stack([blk.step(x[:, T + i], torch.tensor(T + i, device=dev), st) for i in range(40)], 1)
+        exp = ref(x.float())
+    assert torch.equal(x, keep)  # the residual product accumulates onto its own buffer
+    assert _norm(full, exp) <= 2e-2
+    assert _norm(y, exp[:, :T]) <= 2e-2
+    assert _norm(steps, exp[:, T:]) <= 2e-2
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 8), (5, 1024), (4097, 520), (3, 2056), (2, 4096)])
+@pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float32], ids=["w16", "w32"])
+def test_rms_norm_edges(dev, rows, dim, wdtype):
+    print(f"[case] rms_norm {rows}x{dim} {wdtype}", flush=True)
+    n = M.NativeRMSNorm(dim).to(dev)
+    g = torch.Generator(device=dev).manual_seed(dim)
+    n.weight.data = (1 + 0.2 * torch.randn(dim, device=dev, generator=g)).to(wdtype)
+    x = (3 * torch.randn(rows, dim, device=dev, generator=g)).to(torch.bfloat16)
+    with torch.no_grad():
+        y = n(x)
+        shifted = n(torch.cat((x.new_zeros(1), x.view(-1)))[1:].view(rows, dim))  # not 16-byte aligned
+    xf = x.double()
+    exp = xf * torch.rsqrt(xf.square().mean(-1, keepdim=True) + n.eps) * n.weight.double()
+    assert torch.equal(y, shifted)
+    assert bool(((y.double() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-6).all())  # one rounding: half a step
