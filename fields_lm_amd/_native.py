@@ -70,6 +70,9 @@ SIGNATURES = {
     "fl_refresh_state": (_int, [_vp] * 3 + [_i64] * 6 + [_vp] * 5),
     "fl_latent_mean": (_int, [_vp] + [_i64] * 6 + [_vp, _vp, _vp]),
     "fl_rms_norm": (_int, [_vp, _i64, _i64, _vp, _int, ctypes.c_float, _vp, _vp]),
+    "fl_softpatch_norm": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float] + [_vp] * 5),
+    "fl_softpatch_workspace_bytes": (_sz, [_i64] * 3),
+    "fl_softpatch_scan": (_int, [_vp] * 3 + [_i64] * 3 + [_vp, _vp, _vp, _sz, _vp]),
     "fl_boundary_scan": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
     "fl_version": (ctypes.c_char_p, []),
 }

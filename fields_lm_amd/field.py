@@ -27,7 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _native as nat
-from ._dispatch import eager, free_rounding, no_grad_needed, plain_linear
+from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_linear
 
 VAC_MAX = 0.90  # canon:68
 BACKENDS = ("reference", "triton", "hip")
@@ -438,6 +438,30 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """x * rsqrt(mean x^2 + eps) * weight over the last dimension (``fl_rms_norm``), for what
+    :func:`rms_norm_takes` accepts."""
+    x = x.contiguous()
+    if x.data_ptr() % 16:
+        x = x.clone()
+    out = torch.empty_like(x)
+    dim = x.shape[-1]
+    code = nat.load().fl_rms_norm(nat.ptr(x), x.numel() // dim, dim, nat.ptr(weight), nat.dtype_code(weight.dtype),
+                                  eps, nat.ptr(out), nat.stream_handle(x.device))
+    nat.check(code, "fl_rms_norm")
+    return out
+
+
+def rms_norm_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether a norm over ``x``'s last dimension may run in ``fl_rms_norm``: bf16, no gradient, no
+    autocast, rows of at most 4,096 (a multiple of 8)."""
+    dim = weight.numel()
+    return (x.dtype == torch.bfloat16 and weight.dtype in KERNEL_DTYPES and free_rounding()
+            and no_grad_needed(x, weight) and x.ndim > 1 and x.shape[-1] == dim and dim % 8 == 0 and dim <= 4096
+            and 0 < x.numel() < dim << 31 and eager(x, weight) and weight.is_contiguous()
+            and weight.data_ptr() % 16 == 0)
+
+
 def state_to_complex(state: torch.Tensor) -> torch.Tensor:
     """Planar [B,2C] fp32 state -> complex64 [B,C]."""
     c = state.shape[-1] // 2
@@ -457,6 +481,8 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if rms_norm_takes(x, self.weight):
+            return rms_norm(x, self.weight, self.eps)
         xf = x.float()
         y = xf * torch.rsqrt(xf.square().mean(dim=-1, keepdim=True) + self.eps)
         return (y * self.weight.float()).to(x.dtype)

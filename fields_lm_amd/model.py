@@ -38,8 +38,9 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _native as nat
-from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_call
-from .field import FieldBlock, RMSNorm, _linear_residual, boundary_scan, gate_residual_norm, swiglu
+from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_call, plain_linear
+from .field import (FieldBlock, RMSNorm, _linear_residual, boundary_scan, gate_residual_norm, rms_norm,
+                    rms_norm_takes, swiglu)
 
 # api:72-91
 OFFICIAL_ARCHITECTURE: Mapping[str, Any] = {
@@ -70,19 +71,6 @@ LATE_FF_DELTA = 256
 # shared pieces (v20:94-163)
 # ======================================================================================
 
-def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
-    """``fl_rms_norm``: bf16 rows of at most 4,096 (a multiple of 8), fp32 maths."""
-    x = x.contiguous()
-    if x.data_ptr() % 16:
-        x = x.clone()
-    out = torch.empty_like(x)
-    dim = x.shape[-1]
-    code = nat.load().fl_rms_norm(nat.ptr(x), x.numel() // dim, dim, nat.ptr(weight), nat.dtype_code(weight.dtype),
-                                  eps, nat.ptr(out), nat.stream_handle(x.device))
-    nat.check(code, "fl_rms_norm")
-    return out
-
-
 class NativeRMSNorm(nn.Module):
     """v20:94-104: F.rms_norm with the weight cast to the input dtype (eps 1e-6)."""
 
@@ -93,12 +81,8 @@ class NativeRMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        w = self.weight
-        if (x.dtype == torch.bfloat16 and w.dtype in KERNEL_DTYPES and free_rounding() and no_grad_needed(x, w)
-                and x.ndim > 1 and x.shape[-1] == self.dim == w.numel() and self.dim % 8 == 0 and self.dim <= 4096
-                and 0 < x.numel() < self.dim << 31 and eager(x, w) and w.is_contiguous()
-                and w.data_ptr() % 16 == 0):
-            return rms_norm(x, w, self.eps)
+        if rms_norm_takes(x, self.weight):
+            return rms_norm(x, self.weight, self.eps)
         return F.rms_norm(x, (self.dim,), self.weight.to(dtype=x.dtype), self.eps)
 
 
@@ -719,7 +703,41 @@ class BoundaryStateMixer(nn.Module):
             raise NotImplementedError("only the learned boundary scorer of the promoted model")
         return torch.sigmoid(self.score(h).float().squeeze(-1) + 1.5 * prior).clamp(0.01, 0.99)
 
+    def _native(self, x: torch.Tensor, tokens: torch.Tensor) -> bool:
+        """The kernels of ``fl_softpatch_norm`` / ``fl_softpatch_scan`` take this call."""
+        score, norm, lut = self.score, self.norm, self._boundary_lut
+        return (free_rounding() and type(self) is BoundaryStateMixer and self.learned and x.ndim == 3
+                and plain_call(norm, RMSNorm) and plain_linear(score) and score.bias is not None
+                and plain_linear(self.up) and self.up.bias is None and x.is_contiguous()
+                and rms_norm_takes(x, norm.weight) and x.data_ptr() % 16 == 0
+                and no_grad_needed(*self.parameters()) and eager(x, tokens, lut, *self.parameters())
+                and lut.dtype == torch.float32 and tokens.shape == x.shape[:2]
+                and all(t.dtype == x.dtype and t.is_contiguous()
+                        for t in (norm.weight, score.weight, score.bias, self.up.weight))
+                and score.weight.data_ptr() % 16 == 0 and x.shape[0] <= 65535 and x.shape[1] <= 1 << 26)
+
+    def _native_forward(self, x: torch.Tensor, tokens: torch.Tensor):
+        lib, stream = nat.load(), nat.stream_handle(x.device)
+        b, t, dim = x.shape
+        h = torch.empty_like(x)
+        score = torch.empty((b, t), device=x.device, dtype=x.dtype)
+        nat.check(lib.fl_softpatch_norm(nat.ptr(x), b * t, dim, nat.ptr(self.norm.weight), self.norm.eps,
+                                        nat.ptr(self.score.weight), nat.ptr(self.score.bias), nat.ptr(h),
+                                        nat.ptr(score), stream), "fl_softpatch_norm")
+        z = self.down(h).contiguous()
+        prior = self._boundary_lut[tokens]
+        r = z.shape[-1]
+        zs = torch.empty((b * t, 2 * r), device=x.device, dtype=x.dtype)
+        last = torch.empty((b, r), device=x.device, dtype=torch.float32)
+        ws = torch.empty(int(lib.fl_softpatch_workspace_bytes(b, t, r)), device=x.device, dtype=torch.uint8)
+        nat.check(lib.fl_softpatch_scan(nat.ptr(z), nat.ptr(score), nat.ptr(prior), b, t, r, nat.ptr(last),
+                                        nat.ptr(zs), nat.ptr(ws), ws.numel(), stream), "fl_softpatch_scan")
+        return torch.addmm(x.view(-1, dim), zs, self.up.weight.t()).view_as(x), last
+
     def forward(self, x: torch.Tensor, tokens: torch.Tensor, return_state: bool = False):
+        if self._native(x, tokens):
+            out, last = self._native_forward(x, tokens)
+            return (out, last) if return_state else out
         h = self.norm(x)
         z = self.down(h).float()
         boundary = self._boundary(h, tokens)

@@ -231,6 +231,21 @@ int fl_boundary_scan(const float* a, const float* drive, int64_t B, int64_t T, i
                      const float* state_in, float* state_out, float* out, void* stream);
 
 /*
+ * The softpatch mixer around that scan (no gradients), bf16 in and out, fp32 maths:
+ * fl_softpatch_norm: h = RMSNorm(x) weight over rows of dim (a multiple of 8, at most 4,096) and
+ *   score[row] = h . w_score + bias[0];
+ * fl_softpatch_scan: with boundary = clamp(sigmoid(score + 1.5 prior), 0.01, 0.99) per token,
+ *   s_t = (1 - boundary_t) s_{t-1} + boundary_t z_t from s_{-1} = 0; out [B, T, 2R] = [z | s],
+ *   state_out [B, R] = s_{T-1} in fp32. z [B, T, R], score and (fp32) prior [B, T], contiguous;
+ *   workspace: fl_softpatch_workspace_bytes, no initial contents needed.
+ */
+int fl_softpatch_norm(const void* x, int64_t rows, int64_t dim, const void* weight, float eps, const void* w_score,
+                      const void* bias, void* h, void* score, void* stream);
+size_t fl_softpatch_workspace_bytes(int64_t B, int64_t T, int64_t R);
+int fl_softpatch_scan(const void* z, const void* score, const float* prior, int64_t B, int64_t T, int64_t R,
+                      float* state_out, void* out, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Field block elementwise tail for inference, one launch per row block:
  *   x_new  = x + out * sigmoid(gate_pre)            (IndependentVacancyField.forward return,
  *                                                    field_only_v4_chunked_triton_wiki100.py:1193-1195)

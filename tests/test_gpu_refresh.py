@@ -100,3 +100,33 @@ def test_rms_norm_edges(dev, rows, dim, wdtype):
     exp = xf * torch.rsqrt(xf.square().mean(-1, keepdim=True) + n.eps) * n.weight.double()
     assert torch.equal(y, shifted)
     assert bool(((y.double() - exp).abs() <= 2.0 ** -8 * exp.abs() + 1e-6).all())  # one rounding: half a step
+
+
+@pytest.mark.parametrize("dim,rank,B,T", [(64, 64, 1, 1), (128, 64, 2, 15), (512, 64, 3, 16), (128, 8, 2, 17), (1024, 64, 4, 1030),
+                                          (128, 100, 1, 300), (2056, 64, 2, 130), (512, 64, 1, 4099)])
+def test_softpatch_against_fp32(dev, dim, rank, B, T):
+    print(f"[case] softpatch dim={dim} rank={rank} B={B} T={T}", flush=True)
+    torch.manual_seed(T)
+    sp = M.BoundaryStateMixer(dim, rank, vocab=50).to(dev)
+    with torch.no_grad():
+        sp.up.weight.normal_(0, 0.1)
+        sp.score.weight.normal_(0, 0.2)
+        sp.norm.weight.add_(0.1 * torch.randn_like(sp.norm.weight))
+        sp._boundary_lut.copy_(torch.randn(50, device=dev))
+    M.cast_for_inference(sp)
+    ref = copy.deepcopy(sp).float()
+    g = torch.Generator(device=dev).manual_seed(T)
+    x = torch.randn(B, T, dim, device=dev, generator=g).to(torch.bfloat16)
+    tok = torch.randint(0, 50, (B, T), device=dev, generator=g)
+    keep = x.clone()
+    with torch.no_grad():
+        y, last = sp(x, tok, return_state=True)
+        assert torch.equal(sp(x, tok), y)
+        exp, last_exp = ref(x.float(), tok, return_state=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            stock = sp(x, tok)
+    assert torch.equal(x, keep) and last.dtype == torch.float32
+    e, e_stock = _norm(y, exp), _norm(stock, exp)
+    print(f"[case] softpatch native {e:.2e} stock {e_stock:.2e}", flush=True)
+    assert e <= 1.1 * e_stock + 1e-4 and e <= 1e-2
+    assert _norm(last, last_exp) <= 2e-2  # z rounded to bf16, boundaries from a bf16 score
