@@ -59,6 +59,9 @@ SIGNATURES = {
                                        ctypes.c_float, _vp, _vp, _vp]),
     "fl_field_params": (_int, [_vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp]),
     "fl_swiglu": (_int, [_vp, _int, _i64, _i64, _vp, _vp]),
+    "fl_block_step_workspace_bytes": (_sz, [_i64] * 3),
+    "fl_block_step": (_int, [_vp, _i64, _i64, _i64] + [_vp] * 9 + [ctypes.c_float, _vp, _vp, _vp, _int,
+                                                                 ctypes.c_float, _vp, _vp, _vp, _vp, _sz, _vp]),
     "fl_mamba_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "fl_mamba_prefill": (_int, [_vp, _int] + [_i64] * 5 + [_vp, _vp, _int] + [_vp] * 4 +
                          [_int, ctypes.c_float, _vp, _int, _vp, _vp, _sz, _vp]),

@@ -27,7 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _native as nat
-from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_linear
+from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_call, plain_linear
 
 VAC_MAX = 0.90  # canon:68
 BACKENDS = ("reference", "triton", "hip")
@@ -724,6 +724,16 @@ def _linear_residual(x: torch.Tensor, layer: nn.Module, h: torch.Tensor) -> torc
     return x + layer(h)
 
 
+# the mixer's methods that one launch sequence stands for (an instance attribute may replace them)
+_MIXER_METHODS = frozenset(("in_proj", "normed_step", "step", "decode_params", "transition", "_raw", "_fused",
+                            "_read_dtype", "_project"))
+
+
+def _ff_layers(ff: nn.Module) -> Tuple[nn.Module, nn.Module]:
+    """The input and output products of either feed-forward layout."""
+    return (ff.w12, ff.w3) if hasattr(ff, "w12") else (ff.gate_up, ff.down)
+
+
 class FieldBlock(nn.Module):
     """canon:1198-1221: x = mixer(x) (residual inside); x + ff(ff_norm(x))."""
 
@@ -749,7 +759,7 @@ class FieldBlock(nn.Module):
     def _tail(self, x: torch.Tensor, normed: torch.Tensor, gate_pre: torch.Tensor) -> torch.Tensor:
         m = self.mixer
         x1, h = gate_residual_norm(x, m.out_proj(normed), gate_pre, self.ff_norm.weight, self.ff_norm.eps)
-        first, second = (self.ff.w12, self.ff.w3) if hasattr(self.ff, "w12") else (self.ff.gate_up, self.ff.down)
+        first, second = _ff_layers(self.ff)
         return _linear_residual(x1, second, swiglu(first(h)))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -768,7 +778,55 @@ class FieldBlock(nn.Module):
         x, state = self.mixer.prefill(x, state)
         return x + self.ff(self.ff_norm(x)), state
 
+    def _native_step(self, x_t: torch.Tensor, state: torch.Tensor, params) -> bool:
+        """``fl_block_step`` takes this token: bf16, up to 128 rows (past them the library's products
+        are as fast), plain layers, nothing of the mixer replaced, no gradient."""
+        m, ff, dim = self.mixer, self.ff, x_t.shape[-1]
+        if not (free_rounding() and not torch.is_grad_enabled() and x_t.dtype == torch.bfloat16 and x_t.ndim == 2
+                and 0 < x_t.shape[0] <= 128 and dim == m.dim and dim % 8 == 0 and dim <= 8192
+                and type(self) is FieldBlock and type(m) is IndependentVacancyField and params is not None
+                and m.fuse_in_proj and m.fuse_read_norm and m.read_dtype in ("auto", torch.bfloat16)
+                and _MIXER_METHODS.isdisjoint(m.__dict__) and len(params) > 3 and state is not None
+                and plain_call(m.read_norm, RMSNorm) and plain_call(self.ff_norm, RMSNorm) and self.fuse_tail):
+            return False
+        first, second = _ff_layers(ff)
+        layers = (m.write_proj, m.gate_proj, m.out_proj, first, second)
+        if not (all(plain_linear(layer) for layer in layers) and first.bias is None and second.bias is None):
+            return False
+        weights = [t for layer in layers for t in (layer.weight, layer.bias) if t is not None]
+        hidden = second.weight.shape[1]
+        shapes = ((3 * m.channels, dim), (dim, dim), (dim, 2 * dim), (2 * hidden, dim), (dim, hidden))
+        vectors = (params[0], params[1], params[2], params[3], state)
+        return (all(layer.weight.shape == s for layer, s in zip(layers, shapes)) and hidden % 8 == 0
+                and 0 < hidden <= 65536 and dim == 2 * m.channels
+                and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in weights)
+                and all(t.dtype == torch.float32 and t.is_contiguous() for t in vectors)
+                and all(t.numel() == m.channels for t in vectors[:3]) and vectors[3].numel() == 2 * dim
+                and state.shape == (x_t.shape[0], dim) and self.ff_norm.weight.dtype in KERNEL_DTYPES
+                and self.ff_norm.weight.data_ptr() % 16 == 0 and x_t.is_contiguous() and x_t.data_ptr() % 16 == 0
+                and eager(x_t, self.ff_norm.weight, *vectors, *weights))
+
+    def _run_native_step(self, x_t: torch.Tensor, state: torch.Tensor, params) -> torch.Tensor:
+        lib, m = nat.load(), self.mixer
+        rows, dim = x_t.shape
+        first, second = _ff_layers(self.ff)
+        hidden = second.weight.shape[1]
+        out = torch.empty_like(x_t)
+        ws = torch.empty(int(lib.fl_block_step_workspace_bytes(rows, dim, hidden)), device=x_t.device,
+                         dtype=torch.uint8)
+        p = nat.ptr
+        code = lib.fl_block_step(
+            p(x_t), rows, dim, hidden, p(m.write_proj.weight), p(m.write_proj.bias), p(m.gate_proj.weight),
+            p(m.gate_proj.bias), p(params[0]), p(params[1]), p(params[2]), p(state), p(params[3]), m.read_norm.eps,
+            p(m.out_proj.weight), p(m.out_proj.bias), p(self.ff_norm.weight),
+            nat.dtype_code(self.ff_norm.weight.dtype), self.ff_norm.eps, p(first.weight), p(second.weight), p(out),
+            p(ws), ws.numel(), nat.stream_handle(x_t.device))
+        nat.check(code, "fl_block_step")
+        return out
+
     def step(self, x_t: torch.Tensor, state: torch.Tensor, params=None) -> torch.Tensor:
+        if self._native_step(x_t, state, params):
+            return self._run_native_step(x_t, state, params)
         if self._fused_tail(x_t):
             raw_t, gate_pre = self.mixer.in_proj(x_t)
             return self._tail(x_t, self.mixer.normed_step(x_t, state, params, raw_t), gate_pre)

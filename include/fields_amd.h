@@ -269,6 +269,24 @@ int fl_gate_residual_norm_w(const void* x, int x_dtype, const void* out, const v
                             void* normed, void* stream);
 
 /*
+ * One token of a whole Field block for up to 128 rows (FieldBlock.forward of one position,
+ * field_only_v4_chunked_triton_wiki100.py:1167-1221), bf16 weights and activations, fp32 sums:
+ *   [raw | g] = x [write_w | gate_w]^T + bias,  normed = fl_decode_norm_step(raw, state),
+ *   x1 = x + (normed out_w^T + out_b) * sigmoid(g),  h = RMSNorm(x1) ff_norm_w,
+ *   out = x1 + (silu(h gate^T) * (h up^T)) down_w^T  with up_w = [gate; up] [2 hidden, dim].
+ * x, out [rows, dim] contiguous; weights as their layers hold them ([out features, in features]),
+ * 16-byte aligned; dim and hidden multiples of 8; biases may be NULL; tr, ti, gamma, read_norm_w
+ * fp32, ff_norm_w of ff_norm_dtype; state [rows, dim] fp32 advances in place. Rounded to bf16 where the
+ * separate ops round, except that the RMSNorm's row scale is applied to the fp32 sums.
+ */
+size_t fl_block_step_workspace_bytes(int64_t rows, int64_t dim, int64_t hidden);
+int fl_block_step(const void* x, int64_t rows, int64_t dim, int64_t hidden, const void* write_w, const void* write_b,
+                  const void* gate_w, const void* gate_b, const float* tr, const float* ti, const float* gamma,
+                  float* state, const float* read_norm_w, float read_eps, const void* out_w, const void* out_b,
+                  const void* ff_norm_w, int ff_norm_dtype, float ff_eps, const void* up_w, const void* down_w,
+                  void* out, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Transition parameters of the Field mixer (field_only_v4_chunked_triton_wiki100.py:1169-1173),
  * fp32 [C] each: radius = clamp(sigmoid(radius_logit), 0.5, 0.99995), tr = radius cos(theta),
  * ti = radius sin(theta), gamma = sqrt(max(1 - radius^2, 1e-4)). With n_weight > 0, weight32
