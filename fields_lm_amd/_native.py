@@ -62,6 +62,13 @@ SIGNATURES = {
     "fl_block_step_workspace_bytes": (_sz, [_i64] * 3),
     "fl_block_step": (_int, [_vp, _i64, _i64, _i64] + [_vp] * 9 + [ctypes.c_float, _vp, _vp, _vp, _int,
                                                                  ctypes.c_float, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "fl_train_workspace_bytes": (_sz, [_i64]),
+    "fl_train_norm": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _int, _vp, _vp]),
+    "fl_train_norm_backward": (_int, [_vp, _int, _vp, _i64, _i64] + [_vp] * 5 + [_sz, _vp]),
+    "fl_train_gate_norm": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _int, _vp, _vp]),
+    "fl_train_gate_norm_backward": (_int, [_vp, _vp, _int, _vp, _vp, _vp, _int, _i64, _i64] + [_vp] * 7 + [_sz, _vp]),
+    "fl_swiglu_backward": (_int, [_vp, _vp, _int, _i64, _i64, _vp, _vp]),
+    "fl_field_params_backward": (_int, [_vp, _vp, _i64] + [_vp] * 6),
     "fl_mamba_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "fl_mamba_prefill": (_int, [_vp, _int] + [_i64] * 5 + [_vp, _vp, _int] + [_vp] * 4 +
                          [_int, ctypes.c_float, _vp, _int, _vp, _vp, _sz, _vp]),

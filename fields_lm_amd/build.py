@@ -20,7 +20,7 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
 SOURCES = [PKG_DIR / "csrc" / name for name in ("field_scan.hip", "block_tail.hip", "field_params.hip", "mamba.hip",
-                                                 "attention.hip", "boundary.hip", "linear.hip")]
+                                                 "attention.hip", "boundary.hip", "linear.hip", "train.hip")]
 # what a source needs beside HIP_FLAGS (a later flag of a kind replaces an earlier one)
 SOURCE_FLAGS = {"field_params.hip": ["-ffp-contract=on"]}
 INCLUDE_DIR = REPO_DIR / "include"

@@ -27,6 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _native as nat
+from . import _train as train
 from ._dispatch import KERNEL_DTYPES, eager, free_rounding, no_grad_needed, plain_call, plain_linear
 
 VAC_MAX = 0.90  # canon:68
@@ -491,6 +492,8 @@ class RMSNorm(nn.Module):
 class PackedSwiGLU(nn.Module):
     """canon:312-325: w12 packs (gate, value); out = w3(silu(gate) * value)."""
 
+    packed_swiglu = True  # forward is second(silu(gate) * value) of [gate | value] = first(x)
+
     def __init__(self, dim: int, hidden: Optional[int] = None):
         super().__init__()
         self.hidden = int(hidden) if hidden is not None else ((int(8 * dim / 3) + 63) // 64) * 64
@@ -549,12 +552,7 @@ class IndependentVacancyField(nn.Module):
         """(tr, ti, gamma) fp32 [C] (canon:1169-1173), computed in the parameters' dtype."""
         if self._native_params():
             return self._scan_params()[:3]
-        radius = torch.sigmoid(self.radius_logit).clamp(0.50, 0.99995).float()
-        theta = self.theta.float()
-        tr = radius * torch.cos(theta)
-        ti = radius * torch.sin(theta)
-        gamma = torch.sqrt((1.0 - radius.square()).clamp_min(1e-4))
-        return tr.contiguous(), ti.contiguous(), gamma.contiguous()
+        return train.transition_ops(self.radius_logit, self.theta)
 
     def _native_params(self) -> bool:
         """The transition parameters from one launch (fl_field_params): fp32 parameters on the
@@ -726,7 +724,7 @@ def _linear_residual(x: torch.Tensor, layer: nn.Module, h: torch.Tensor) -> torc
 
 # the mixer's methods that one launch sequence stands for (an instance attribute may replace them)
 _MIXER_METHODS = frozenset(("in_proj", "normed_step", "step", "decode_params", "transition", "_raw", "_fused",
-                            "_read_dtype", "_project"))
+                            "_read_dtype", "_project", "normed_read", "_unfused_read_dtype"))
 
 
 def _ff_layers(ff: nn.Module) -> Tuple[nn.Module, nn.Module]:
@@ -762,10 +760,48 @@ class FieldBlock(nn.Module):
         first, second = _ff_layers(self.ff)
         return _linear_residual(x1, second, swiglu(first(h)))
 
+    def _native_training(self, x: torch.Tensor) -> bool:
+        """The forward and backward kernels of ``csrc/train.hip`` take the block's elementwise work: an
+        fp32 residual stream and fp32 parameters (under bf16 autocast or none), and every module between
+        the products its own class, called without hooks."""
+        m, ff, dim = self.mixer, self.ff, x.shape[-1]
+        if not (torch.is_grad_enabled() and x.dtype == torch.float32 and x.numel() > 0 and x.ndim == 3
+                and dim == m.dim and dim % 8 == 0 and dim <= 2048 and x.numel() // dim < 1 << 31
+                and type(self) is FieldBlock and plain_call(m, IndependentVacancyField)
+                and plain_call(self.ff_norm, RMSNorm) and plain_call(m.read_norm, RMSNorm)
+                and type(ff).__dict__.get("packed_swiglu") and plain_call(ff, type(ff))
+                and _MIXER_METHODS.isdisjoint(m.__dict__) and m.read_dtype == "auto" and self.fuse_tail
+                and (not torch.is_autocast_enabled() or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
+            return False
+        norms = (m.read_norm.weight, self.ff_norm.weight)
+        ring = (m.radius_logit, m.theta)
+        return (all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in norms)
+                and all(t.dtype == torch.float32 and t.is_contiguous() and t.shape == (m.channels,) for t in ring)
+                and eager(x, *norms, *ring))
+
+    def _train_forward(self, x: torch.Tensor) -> torch.Tensor:
+        m = self.mixer
+        dtype = torch.bfloat16 if torch.is_autocast_enabled() else torch.float32  # what a product reads
+        raw, gate_pre = m.write_proj(x), m.gate_proj(x)
+        tr, ti, gamma = train.Transition.apply(m.radius_logit, m.theta)
+        read = fused_field_read(m._raw(x, raw), tr, ti, gamma, m.triton_block_c, m.triton_chunk_t)
+        out = m.out_proj(train.Norm.apply(read, m.read_norm.weight, m.read_norm.eps, dtype))
+        if out.dtype != gate_pre.dtype or out.dtype not in KERNEL_DTYPES:
+            x = x + (out * torch.sigmoid(gate_pre)).to(x.dtype)
+            return x + self.ff(self.ff_norm(x))
+        x, h = train.GateNorm.apply(x, out, gate_pre, self.ff_norm.weight, self.ff_norm.eps, dtype)
+        first, second = _ff_layers(self.ff)
+        gu = first(h)
+        if gu.dtype in KERNEL_DTYPES and gu.shape[-1] % 16 == 0 and gu.numel() < 1 << 34:
+            return x + second(train.Swiglu.apply(gu))
+        return x + second(train._swiglu_ops(gu))
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._fused_tail(x):
             raw, gate_pre = self.mixer.in_proj(x)
             return self._tail(x, self.mixer.normed_read(x, raw), gate_pre)
+        if self._native_training(x):
+            return self._train_forward(x)
         x = self.mixer(x)
         return x + self.ff(self.ff_norm(x))
 

@@ -90,6 +90,8 @@ class GateUpSwiGLU(nn.Module):
     """v20:107-117 (``PackedSwiGLU`` of the refresh blocks and of the R1-resized Field FFNs):
     down(silu(gate) * up) with gate, up = gate_up(x).chunk(2)."""
 
+    packed_swiglu = True  # as PackedSwiGLU
+
     def __init__(self, dim: int, hidden: int) -> None:
         super().__init__()
         self.gate_up = nn.Linear(dim, 2 * hidden, bias=False)

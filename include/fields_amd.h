@@ -372,6 +372,36 @@ int fl_latent_mean(const void* latent, int64_t stride_b, int64_t stride_t, int64
 int fl_rms_norm(const void* x, int64_t rows, int64_t dim, const void* weight, int w_dtype, float eps, void* out,
                 void* stream);
 
+/*
+ * The Field block's elementwise work in training (field_only_v4_chunked_triton_wiki100.py:300-325,
+ * 1169-1173, 1193-1195, 1219-1221), fp32 residual stream and maths; rows of dim (a multiple of 8, at
+ * most 4,096), every [rows, dim] operand contiguous and 16-byte aligned:
+ * fl_train_norm: out = x rstd weight, rstd = (mean x^2 + eps)^-1/2 per row (kept for the backward);
+ * fl_train_gate_norm: x_new = x + out * sigmoid(gate) (rounded in g_dtype as the stock ops round), and
+ *   its norm;
+ * the backwards give the gradients of every input; gw [dim] is summed over the rows in a fixed order
+ *   through workspace (fl_train_workspace_bytes(dim));
+ * fl_swiglu_backward: gradient of fl_swiglu (hidden a multiple of 8);
+ * fl_field_params_backward: gradients of fl_field_params' tr, ti, gamma.
+ */
+size_t fl_train_workspace_bytes(int64_t dim);
+int fl_train_norm(const float* x, int64_t rows, int64_t dim, const float* weight, float eps, void* out, int out_dtype,
+                  float* rstd, void* stream);
+int fl_train_norm_backward(const void* gy, int gy_dtype, const float* x, int64_t rows, int64_t dim,
+                           const float* weight, const float* rstd, float* gx, float* gw, void* workspace,
+                           size_t workspace_bytes, void* stream);
+int fl_train_gate_norm(const float* x, const void* out, const void* gate, int g_dtype, int64_t rows, int64_t dim,
+                       const float* weight, float eps, float* x_new, void* normed, int normed_dtype, float* rstd,
+                       void* stream);
+int fl_train_gate_norm_backward(const float* g_x_new, const void* g_normed, int normed_dtype, const float* x_new,
+                                const void* out, const void* gate, int g_dtype, int64_t rows, int64_t dim,
+                                const float* weight, const float* rstd, float* gx, void* g_out, void* g_gate,
+                                float* gw, void* workspace, size_t workspace_bytes, void* stream);
+int fl_swiglu_backward(const void* gate_up, const void* gy, int dtype, int64_t rows, int64_t hidden, void* g_gate_up,
+                       void* stream);
+int fl_field_params_backward(const float* radius_logit, const float* theta, int64_t C, const float* gtr,
+                             const float* gti, const float* ggamma, float* g_logit, float* g_theta, void* stream);
+
 /* Library version string (host function). No counterpart in the reference. */
 const char* fl_version(void);
 
