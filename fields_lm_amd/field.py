@@ -63,6 +63,14 @@ def _read_code(read_dtype: torch.dtype) -> int:
     raise TypeError(f"read must be float32 or bfloat16, got {read_dtype}")
 
 
+def _fp32(t: torch.Tensor, device) -> torch.Tensor:
+    """``t`` as the kernels read it: contiguous fp32 on ``device`` (itself where it is that already; only
+    its address is used)."""
+    if t.dtype == torch.float32 and t.device == device and t.is_contiguous():
+        return t
+    return t.detach().to(device=device, dtype=torch.float32).contiguous()
+
+
 def _scan_call(raw, transition_r, transition_i, gamma, state_in, return_state, out_dtype, launch):
     """Shared argument handling of the scan entry points; ``launch(lib, args)`` makes the call.
 
@@ -72,9 +80,7 @@ def _scan_call(raw, transition_r, transition_i, gamma, state_in, return_state, o
     if raw.stride(2) != 1:
         raw = raw.contiguous()
     dev = raw.device
-    tr = transition_r.detach().to(device=dev, dtype=torch.float32).contiguous()
-    ti = transition_i.detach().to(device=dev, dtype=torch.float32).contiguous()
-    gm = gamma.detach().to(device=dev, dtype=torch.float32).contiguous()
+    tr, ti, gm = _fp32(transition_r, dev), _fp32(transition_i, dev), _fp32(gamma, dev)
     if ti.numel() != channels or gm.numel() != channels:
         raise ValueError((raw.shape, transition_i.shape, gamma.shape))
     _read_code(out_dtype)
@@ -83,7 +89,7 @@ def _scan_call(raw, transition_r, transition_i, gamma, state_in, return_state, o
     if state_in is not None:
         if state_in.shape != (batch, 2 * channels):
             raise ValueError(f"state_in must be [B, 2C] = {(batch, 2 * channels)}, got {tuple(state_in.shape)}")
-        sin = state_in.detach().to(device=dev, dtype=torch.float32).contiguous()
+        sin = _fp32(state_in, dev)
     sout = torch.empty((batch, 2 * channels), device=dev, dtype=torch.float32) if return_state else None
     if batch == 0 or length == 0 or channels == 0:
         if sout is not None:
@@ -121,7 +127,7 @@ def field_scan(raw: torch.Tensor, transition_r: torch.Tensor, transition_i: torc
 
 
 def _norm_weight(weight: torch.Tensor, channels: int, device) -> torch.Tensor:
-    w = weight.detach().to(device=device, dtype=torch.float32).contiguous()
+    w = _fp32(weight, device)
     if w.numel() != 4 * channels:
         raise ValueError(f"norm weight must have 4C = {4 * channels} entries, got {w.numel()}")
     return w
@@ -173,12 +179,11 @@ def field_scan_backward(raw: torch.Tensor, transition_r: torch.Tensor, transitio
         raise ValueError("read must be the forward's fp32 [B, T, 4C] output")
     if grad_read.shape != read.shape:
         raise ValueError("grad_read must match read")
-    tr, ti, gm = (t.detach().to(device=dev, dtype=torch.float32).contiguous()
-                  for t in (transition_r, transition_i, gamma))
-    read = read.detach().contiguous()
-    grad_read = grad_read.detach().to(dtype=torch.float32).contiguous()
-    sin = None if state_in is None else state_in.detach().to(device=dev, dtype=torch.float32).contiguous()
-    gso = None if grad_state_out is None else grad_state_out.detach().to(device=dev, dtype=torch.float32).contiguous()
+    tr, ti, gm = _fp32(transition_r, dev), _fp32(transition_i, dev), _fp32(gamma, dev)
+    read = read.contiguous()
+    grad_read = _fp32(grad_read, grad_read.device)
+    sin = None if state_in is None else _fp32(state_in, dev)
+    gso = None if grad_state_out is None else _fp32(grad_state_out, dev)
     for name, t in (("state_in", sin), ("grad_state_out", gso)):
         if t is not None and t.shape != (batch, 2 * channels):
             raise ValueError(f"{name} must be [B, 2C]")
@@ -814,55 +819,74 @@ class FieldBlock(nn.Module):
         x, state = self.mixer.prefill(x, state)
         return x + self.ff(self.ff_norm(x)), state
 
-    def _native_step(self, x_t: torch.Tensor, state: torch.Tensor, params) -> bool:
-        """``fl_block_step`` takes this token: bf16, up to 128 rows (past them the library's products
-        are as fast), plain layers, nothing of the mixer replaced, no gradient."""
-        m, ff, dim = self.mixer, self.ff, x_t.shape[-1]
-        if not (free_rounding() and not torch.is_grad_enabled() and x_t.dtype == torch.bfloat16 and x_t.ndim == 2
-                and 0 < x_t.shape[0] <= 128 and dim == m.dim and dim % 8 == 0 and dim <= 8192
-                and type(self) is FieldBlock and type(m) is IndependentVacancyField and params is not None
-                and m.fuse_in_proj and m.fuse_read_norm and m.read_dtype in ("auto", torch.bfloat16)
-                and _MIXER_METHODS.isdisjoint(m.__dict__) and len(params) > 3 and state is not None
-                and plain_call(m.read_norm, RMSNorm) and plain_call(self.ff_norm, RMSNorm) and self.fuse_tail):
-            return False
-        first, second = _ff_layers(ff)
-        layers = (m.write_proj, m.gate_proj, m.out_proj, first, second)
-        if not (all(plain_linear(layer) for layer in layers) and first.bias is None and second.bias is None):
-            return False
-        weights = [t for layer in layers for t in (layer.weight, layer.bias) if t is not None]
-        hidden = second.weight.shape[1]
-        shapes = ((3 * m.channels, dim), (dim, dim), (dim, 2 * dim), (2 * hidden, dim), (dim, hidden))
-        vectors = (params[0], params[1], params[2], params[3], state)
-        return (all(layer.weight.shape == s for layer, s in zip(layers, shapes)) and hidden % 8 == 0
-                and 0 < hidden <= 65536 and dim == 2 * m.channels
-                and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in weights)
-                and all(t.dtype == torch.float32 and t.is_contiguous() for t in vectors)
-                and all(t.numel() == m.channels for t in vectors[:3]) and vectors[3].numel() == 2 * dim
-                and state.shape == (x_t.shape[0], dim) and self.ff_norm.weight.dtype in KERNEL_DTYPES
-                and self.ff_norm.weight.data_ptr() % 16 == 0 and x_t.is_contiguous() and x_t.data_ptr() % 16 == 0
-                and eager(x_t, self.ff_norm.weight, *vectors, *weights))
-
-    def _run_native_step(self, x_t: torch.Tensor, state: torch.Tensor, params) -> torch.Tensor:
-        lib, m = nat.load(), self.mixer
+    def _native_step(self, x_t: torch.Tensor, state: torch.Tensor, params):
+        """The tensors that ``fl_block_step`` reads where it takes this token, else None: bf16, up to 128
+        rows (past them the library's products are as fast), plain layers, nothing of the mixer
+        replaced, no gradient."""
+        if (torch.is_grad_enabled() or not free_rounding() or x_t.dtype != torch.bfloat16 or x_t.ndim != 2
+                or not 0 < x_t.shape[0] <= 128 or params is None or len(params) < 4 or state is None):
+            return None
+        parts = self._modules
+        m, ff, ff_norm = parts["mixer"], parts["ff"], parts["ff_norm"]
         rows, dim = x_t.shape
-        first, second = _ff_layers(self.ff)
-        hidden = second.weight.shape[1]
+        if not (type(self) is FieldBlock and type(m) is IndependentVacancyField and dim == m.dim == 2 * m.channels
+                and dim % 8 == 0 and dim <= 8192 and self.fuse_tail and m.fuse_in_proj and m.fuse_read_norm
+                and m.read_dtype in ("auto", torch.bfloat16) and _MIXER_METHODS.isdisjoint(m.__dict__)):
+            return None
+        inner = m._modules
+        first, second = _ff_layers(ff)
+        layers = (inner["write_proj"], inner["gate_proj"], inner["out_proj"], first, second)
+        if not (plain_call(inner["read_norm"], RMSNorm) and plain_call(ff_norm, RMSNorm)
+                and all(plain_linear(layer) for layer in layers)):
+            return None
+        tensors = [(p["weight"], p["bias"]) for p in (layer._parameters for layer in layers)]
+        (ww, wb), (gw, gb), (ow, ob), (uw, ub), (dw, db) = tensors
+        hidden = dw.shape[1]
+        norm = ff_norm.weight
+        tr, ti, gamma, read_w = params[:4]
+        matrices = (ww, gw, ow, uw, dw)
+        vectors = tuple(t for t in (wb, gb, ob) if t is not None)
+        fp32 = (tr, ti, gamma, read_w, state)
+        if not (ub is None and db is None and hidden % 8 == 0 and 0 < hidden <= 65536
+                and [t.shape for t in matrices] == [(3 * m.channels, dim), (dim, dim), (dim, 2 * dim),
+                                                    (2 * hidden, dim), (dim, hidden)]
+                and tr.numel() == ti.numel() == gamma.numel() == m.channels and read_w.numel() == 2 * dim
+                and state.shape == (rows, dim) and norm.dtype in KERNEL_DTYPES
+                and eager(x_t, norm, *fp32, *matrices, *vectors)):
+            return None
+        for t in (x_t, *matrices):
+            if t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16:
+                return None
+        for t in vectors:
+            if t.dtype != torch.bfloat16 or not t.is_contiguous():
+                return None
+        for t in fp32:
+            if t.dtype != torch.float32 or not t.is_contiguous():
+                return None
+        if not norm.is_contiguous() or norm.data_ptr() % 16:
+            return None
+        return hidden, ww, wb, gw, gb, tr, ti, gamma, read_w, inner["read_norm"].eps, ow, ob, norm, ff_norm.eps, uw, dw
+
+    @staticmethod
+    def _run_native_step(x_t: torch.Tensor, state: torch.Tensor, args) -> torch.Tensor:
+        hidden, ww, wb, gw, gb, tr, ti, gamma, read_w, read_eps, ow, ob, norm, ff_eps, uw, dw = args
+        lib, p = nat.load(), nat.ptr
+        rows, dim = x_t.shape
         out = torch.empty_like(x_t)
-        ws = torch.empty(int(lib.fl_block_step_workspace_bytes(rows, dim, hidden)), device=x_t.device,
-                         dtype=torch.uint8)
-        p = nat.ptr
+        n = lib.fl_block_step_workspace_bytes(rows, dim, hidden)
+        ws = torch.empty(n, device=x_t.device, dtype=torch.uint8)
         code = lib.fl_block_step(
-            p(x_t), rows, dim, hidden, p(m.write_proj.weight), p(m.write_proj.bias), p(m.gate_proj.weight),
-            p(m.gate_proj.bias), p(params[0]), p(params[1]), p(params[2]), p(state), p(params[3]), m.read_norm.eps,
-            p(m.out_proj.weight), p(m.out_proj.bias), p(self.ff_norm.weight),
-            nat.dtype_code(self.ff_norm.weight.dtype), self.ff_norm.eps, p(first.weight), p(second.weight), p(out),
-            p(ws), ws.numel(), nat.stream_handle(x_t.device))
+            x_t.data_ptr(), rows, dim, hidden, ww.data_ptr(), p(wb), gw.data_ptr(), p(gb), tr.data_ptr(),
+            ti.data_ptr(), gamma.data_ptr(), state.data_ptr(), read_w.data_ptr(), read_eps, ow.data_ptr(), p(ob),
+            norm.data_ptr(), nat.dtype_code(norm.dtype), ff_eps, uw.data_ptr(), dw.data_ptr(), out.data_ptr(),
+            ws.data_ptr(), n, nat.stream_handle(x_t.device))
         nat.check(code, "fl_block_step")
         return out
 
     def step(self, x_t: torch.Tensor, state: torch.Tensor, params=None) -> torch.Tensor:
-        if self._native_step(x_t, state, params):
-            return self._run_native_step(x_t, state, params)
+        native = self._native_step(x_t, state, params)
+        if native is not None:
+            return self._run_native_step(x_t, state, native)
         if self._fused_tail(x_t):
             raw_t, gate_pre = self.mixer.in_proj(x_t)
             return self._tail(x_t, self.mixer.normed_step(x_t, state, params, raw_t), gate_pre)

@@ -707,15 +707,16 @@ class BoundaryStateMixer(nn.Module):
 
     def _native(self, x: torch.Tensor, tokens: torch.Tensor) -> bool:
         """The kernels of ``fl_softpatch_norm`` / ``fl_softpatch_scan`` take this call."""
-        score, norm, lut = self.score, self.norm, self._boundary_lut
-        return (free_rounding() and type(self) is BoundaryStateMixer and self.learned and x.ndim == 3
+        score, norm, up, lut = self.score, self.norm, self.up, self._boundary_lut
+        if not (free_rounding() and type(self) is BoundaryStateMixer and self.learned and x.ndim == 3
                 and plain_call(norm, RMSNorm) and plain_linear(score) and score.bias is not None
-                and plain_linear(self.up) and self.up.bias is None and x.is_contiguous()
-                and rms_norm_takes(x, norm.weight) and x.data_ptr() % 16 == 0
-                and no_grad_needed(*self.parameters()) and eager(x, tokens, lut, *self.parameters())
+                and plain_linear(up) and up.bias is None and x.is_contiguous() and x.data_ptr() % 16 == 0):
+            return False
+        params = (norm.weight, score.weight, score.bias, up.weight)
+        return (rms_norm_takes(x, norm.weight) and no_grad_needed(*params, self.down.weight)
+                and eager(x, tokens, lut, *params)
                 and lut.dtype == torch.float32 and tokens.shape == x.shape[:2]
-                and all(t.dtype == x.dtype and t.is_contiguous()
-                        for t in (norm.weight, score.weight, score.bias, self.up.weight))
+                and all(t.dtype == x.dtype and t.is_contiguous() for t in params)
                 and score.weight.data_ptr() % 16 == 0 and x.shape[0] <= 65535 and x.shape[1] <= 1 << 26)
 
     def _native_forward(self, x: torch.Tensor, tokens: torch.Tensor):

@@ -51,7 +51,7 @@ def test_block_step_kernels(dev, dim, hidden, B):
     s0 = torch.randn(B, dim, device=dev, generator=g)
     with torch.no_grad():
         params, rparams = b.mixer.decode_params(), ref.mixer.decode_params()
-        assert b._native_step(xs[0], s0, params)
+        assert b._native_step(xs[0], s0, params) is not None
         st, st_stock, st_ref = s0.clone(), s0.clone(), s0.clone()
         y = torch.stack([b.step(x, st, params) for x in xs])
         b.mixer.fuse_in_proj = False  # the separate ops
@@ -91,12 +91,12 @@ def test_block_step_in_hip_graph_and_replaced_parts(dev):
         calls = []
         for part in (b.mixer.out_proj, b.ff.w3, b.mixer.read_norm):
             handle = part.register_forward_pre_hook(lambda mod, args: calls.append(mod))
-            assert not b._native_step(x, st2, params)
+            assert b._native_step(x, st2, params) is None
             handle.remove()
         b.mixer.normed_step = b.mixer.normed_step
-        assert not b._native_step(x, st2, params)
+        assert b._native_step(x, st2, params) is None
         del b.mixer.normed_step
-        assert b._native_step(x, st2, params)
+        assert b._native_step(x, st2, params) is not None
         with torch.autocast("cuda", dtype=torch.bfloat16):
-            assert not b._native_step(x, st2, params)
-    assert not b._native_step(x, st2, params)  # gradients enabled
+            assert b._native_step(x, st2, params) is None
+    assert b._native_step(x, st2, params) is None  # gradients enabled
