@@ -78,6 +78,10 @@ SIGNATURES = {
     "fl_refresh_attention": (_int, [_vp, _i64, _i64, _vp, _vp] + [_i64] * 7 + [_vp, _vp, _vp, _int, _vp, _vp, _sz,
                                                                              _vp]),
     "fl_refresh_state": (_int, [_vp] * 3 + [_i64] * 6 + [_vp] * 5),
+    "fl_refresh_step_in": (_int, [_vp] * 5 + [_i64] * 7 + [_vp] * 6),
+    "fl_refresh_step_out": (_int, [_vp] * 4 + [_i64] * 5 + [_vp] * 3),
+    "fl_mask_scores": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _i64, ctypes.c_float, _vp, _vp]),
+    "fl_mix": (_int, [_vp, _vp, _vp, _int, _i64, _vp, _vp]),
     "fl_latent_mean": (_int, [_vp] + [_i64] * 6 + [_vp, _vp, _vp]),
     "fl_rms_norm": (_int, [_vp, _i64, _i64, _vp, _int, ctypes.c_float, _vp, _vp]),
     "fl_softpatch_norm": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float] + [_vp] * 5),

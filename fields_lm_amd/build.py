@@ -20,9 +20,9 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
 SOURCES = [PKG_DIR / "csrc" / name for name in ("field_scan.hip", "block_tail.hip", "field_params.hip", "mamba.hip",
-                                                 "attention.hip", "boundary.hip", "linear.hip", "train.hip")]
+                                                 "attention.hip", "boundary.hip", "linear.hip", "train.hip", "exact.hip")]
 # what a source needs beside HIP_FLAGS (a later flag of a kind replaces an earlier one)
-SOURCE_FLAGS = {"field_params.hip": ["-ffp-contract=on"]}
+SOURCE_FLAGS = {"field_params.hip": ["-ffp-contract=on"], "exact.hip": ["-ffp-contract=on"]}
 INCLUDE_DIR = REPO_DIR / "include"
 LIB_PATH = PKG_DIR / "libfields_amd.so"
 # measurement kernels for bench.py (the scan's access pattern without its arithmetic), kept out of

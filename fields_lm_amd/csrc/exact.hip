@@ -1,0 +1,208 @@
+// exact.hip — elementwise work of the refresh blocks in the stock ops' own roundings, bit for bit, so
+// that it may run under autocast too, where a generation loop keeps its bits (reference: src/
+// fields_official/reference/official_source/field_fusion_system_smoke_v21.py:131-253). bf16 values are
+// rounded after every operation, as an op on bf16 tensors does; sums and products with an order of
+// their own (the matrix products, softmax) stay with the stock ops.
+//
+// Built with -ffp-contract=on: products and sums of separate statements stay separate.
+#include "fl_common.h"
+
+#pragma clang fp contract(off)
+
+namespace {
+
+using namespace fl;
+
+constexpr int kHd = 64;
+
+__device__ __forceinline__ float bf(const bf16_bits* p) { return load_as<bf16_bits>(p); }
+
+// (a, b) -> (a cos - b sin, b cos + a sin), each product and each sum rounded
+__device__ __forceinline__ void rope_pair(float a, float b, float c, float s, bf16_bits* first, bf16_bits* second) {
+  const float ac = bf16_round(a * c), bs = bf16_round(b * s), bc = bf16_round(b * c), as = bf16_round(a * s);
+  *first = (bf16_bits)bf16_bits_of(ac - bs);
+  *second = (bf16_bits)bf16_bits_of(bc + as);
+}
+
+struct StepArgs {
+  const bf16_bits* qlat;  // [B, q_heads * 64 + latent]
+  const bf16_bits* kv;    // [B, 2 * kv_heads * 64]
+  const bf16_bits* cos;   // [rope_len, 32]
+  const bf16_bits* sin;
+  const int64_t* pos;
+  int q_heads, kv_heads, latent, rope_len, window, chunk, slots;
+};
+
+// One token's rotations and state writes before the attention: some 40 stock launches of 4 us in one.
+// q [B, q_heads * 64] rotated; keys and values into the window's slot; the chunk's running latent sum
+// (restarted on a chunk's first token) and its mean.
+__global__ __launch_bounds__(256) void fl_refresh_step_in_kernel(StepArgs a, bf16_bits* __restrict__ q,
+                                                                 bf16_bits* __restrict__ kt,
+                                                                 bf16_bits* __restrict__ v,
+                                                                 float* __restrict__ lat_sum,
+                                                                 bf16_bits* __restrict__ mean) {
+  const int64_t b = blockIdx.x, p = *a.pos;
+  const int64_t at = p < a.rope_len - 1 ? (p < 0 ? 0 : p) : a.rope_len - 1;
+  const int slot = (int)(((p % a.window) + a.window) % a.window);
+  const bf16_bits *c = a.cos + at * 32, *s = a.sin + at * 32;
+  const int qw = a.q_heads * kHd;
+  const bf16_bits* x = a.qlat + b * (qw + a.latent);
+  const bf16_bits* kv = a.kv + b * 2 * a.kv_heads * kHd;
+  for (int i = threadIdx.x; i < a.q_heads * 32; i += 256) {
+    const int o = (i >> 5) * kHd + (i & 31);
+    rope_pair(bf(x + o), bf(x + o + 32), bf(c + (i & 31)), bf(s + (i & 31)), q + b * qw + o, q + b * qw + o + 32);
+  }
+  for (int i = threadIdx.x; i < a.kv_heads * 32; i += 256) {
+    const int h = i >> 5, d = i & 31;
+    bf16_bits* k = kt + ((b * a.kv_heads + h) * kHd + d) * a.window + slot;
+    rope_pair(bf(kv + h * kHd + d), bf(kv + h * kHd + d + 32), bf(c + d), bf(s + d), k, k + (int64_t)32 * a.window);
+  }
+  for (int i = threadIdx.x; i < a.kv_heads * kHd; i += 256)
+    v[((b * a.kv_heads + (i >> 6)) * a.window + slot) * kHd + (i & 63)] = kv[a.kv_heads * kHd + i];
+  const float keep = ((p % a.chunk) + a.chunk) % a.chunk == 0 ? 0.f : 1.f, inv = 1.0f / (float)a.chunk;
+  for (int i = threadIdx.x; i < a.latent; i += 256) {
+    float t = lat_sum[b * a.latent + i] * keep;
+    t = t + bf(x + qw + i);
+    lat_sum[b * a.latent + i] = t;
+    mean[b * a.latent + i] = (bf16_bits)bf16_bits_of(t * inv);  // a power of two: exact
+  }
+}
+
+// The chunk's landmark of one token's running mean into its slot (clamped into the buffer).
+__global__ __launch_bounds__(256) void fl_refresh_step_out_kernel(StepArgs a, bf16_bits* __restrict__ lkt,
+                                                                  bf16_bits* __restrict__ lv) {
+  const int64_t b = blockIdx.x, p = *a.pos;
+  const int64_t at = p < a.rope_len - 1 ? (p < 0 ? 0 : p) : a.rope_len - 1;
+  const int64_t chunk = p < 0 ? -1 : p / a.chunk;
+  const int slot = (int)(chunk + 1 < a.slots - 1 ? chunk + 1 : a.slots - 1);
+  const bf16_bits *c = a.cos + at * 32, *s = a.sin + at * 32;
+  const bf16_bits* kv = a.kv + b * 2 * a.kv_heads * kHd;
+  for (int i = threadIdx.x; i < a.kv_heads * 32; i += 256) {
+    const int h = i >> 5, d = i & 31;
+    bf16_bits* k = lkt + ((b * a.kv_heads + h) * kHd + d) * a.slots + slot;
+    rope_pair(bf(kv + h * kHd + d), bf(kv + h * kHd + d + 32), bf(c + d), bf(s + d), k, k + (int64_t)32 * a.slots);
+  }
+  for (int i = threadIdx.x; i < a.kv_heads * kHd; i += 256)
+    lv[((b * a.kv_heads + (i >> 6)) * a.slots + slot) * kHd + (i & 63)] = kv[a.kv_heads * kHd + i];
+}
+
+// out = float(scores) * scale where column j is visible, else -inf. Visible: j <= limit, with limit the
+// token's window slot or its chunk (read from pos, period and step), or the row's index within lq
+// (causal), or any. Four passes of the stock ops over the fp32 scores in one, bound by memory.
+__global__ __launch_bounds__(256) void fl_mask_scores_kernel(const bf16_bits* __restrict__ scores, uint64_t n,
+                                                             uint32_t lk, uint32_t lq, int mode,
+                                                             const int64_t* __restrict__ pos, int period,
+                                                             float scale, float* __restrict__ out) {
+  const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  const uint64_t row = i / lk;
+  const uint32_t j = (uint32_t)(i - row * lk);  // lk is a multiple of 4: one row per thread
+  int64_t limit = lk;
+  if (mode == 0) limit = row % lq;
+  else if (mode == 1) limit = ((*pos % period) + period) % period;
+  else limit = *pos / period;
+  const u32x2 w = *reinterpret_cast<const u32x2*>(scores + i);
+  const float s[4] = {bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y)};
+  f32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (int64_t)j + e <= limit ? s[e] * scale : -INFINITY;
+  *reinterpret_cast<f32x4*>(out + i) = o;
+}
+
+__global__ __launch_bounds__(256) void fl_mask_scores_any_kernel(const bf16_bits* __restrict__ scores, uint64_t n,
+                                                                 uint32_t lk, uint32_t lq, int mode,
+                                                                 const int64_t* __restrict__ pos, int period,
+                                                                 float scale, float* __restrict__ out) {
+  const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const uint64_t row = i / lk;
+  const int64_t j = (int64_t)(i - row * lk);
+  const int64_t limit = mode == 0 ? (int64_t)(row % lq)
+                                  : mode == 1 ? ((*pos % period) + period) % period : *pos / period;
+  out[i] = j <= limit ? bf(scores + i) * scale : -INFINITY;
+}
+
+// out = y + round(sigmoid(mix)) * g, rounded after each operation
+__global__ __launch_bounds__(256) void fl_mix_kernel(const bf16_bits* __restrict__ y, const bf16_bits* __restrict__ g,
+                                                     const void* mix, int mix16, uint32_t n,
+                                                     bf16_bits* __restrict__ out) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const float x = mix16 ? bf(static_cast<const bf16_bits*>(mix)) : *static_cast<const float*>(mix);
+  const float s = bf16_round(1.0f / (1.0f + expf(-x)));
+  const float t = bf16_round(s * bf(g + i));
+  out[i] = (bf16_bits)bf16_bits_of(bf(y + i) + t);
+}
+
+bool step_ok(const StepArgs& a, int64_t B) {
+  return B > 0 && B <= (1 << 20) && a.q_heads > 0 && a.q_heads <= 4096 && a.kv_heads > 0 && a.kv_heads <= 4096 &&
+         a.latent > 0 && a.latent <= (1 << 16) && a.rope_len > 0 && a.window > 0 && a.chunk > 0 &&
+         (a.chunk & (a.chunk - 1)) == 0 && a.slots > 0 && a.kv && a.cos && a.sin && a.pos;
+}
+
+StepArgs step_args(const void* qlat, const void* kv, const void* cos, const void* sin, const int64_t* pos,
+                   int64_t q_heads, int64_t kv_heads, int64_t latent, int64_t rope_len, int64_t window, int64_t chunk,
+                   int64_t slots) {
+  auto p = [](const void* t) { return static_cast<const bf16_bits*>(t); };
+  return {p(qlat), p(kv), p(cos), p(sin), pos, (int)q_heads, (int)kv_heads, (int)latent, (int)rope_len,
+          (int)window, (int)chunk, (int)slots};
+}
+
+}  // namespace
+
+extern "C" {
+
+int fl_refresh_step_in(const void* qlat, const void* kv, const void* cos, const void* sin, const int64_t* pos,
+                       int64_t B, int64_t q_heads, int64_t kv_heads, int64_t latent, int64_t rope_len, int64_t window,
+                       int64_t chunk, void* q, void* kt, void* v, float* lat_sum, void* mean, void* stream) {
+  const StepArgs a = step_args(qlat, kv, cos, sin, pos, q_heads, kv_heads, latent, rope_len, window, chunk, 1);
+  if (rope_len > (1 << 28) || window > (1 << 28) || chunk > (1 << 28) || !step_ok(a, B) || !qlat || !q || !kt || !v ||
+      !lat_sum || !mean)
+    return FL_ERR_INVALID_ARGUMENT;
+  fl_refresh_step_in_kernel<<<(unsigned)B, 256, 0, static_cast<hipStream_t>(stream)>>>(
+      a, static_cast<bf16_bits*>(q), static_cast<bf16_bits*>(kt), static_cast<bf16_bits*>(v), lat_sum,
+      static_cast<bf16_bits*>(mean));
+  return hip_status(hipGetLastError());
+}
+
+int fl_refresh_step_out(const void* kv, const void* cos, const void* sin, const int64_t* pos, int64_t B,
+                        int64_t kv_heads, int64_t rope_len, int64_t chunk, int64_t slots, void* lkt, void* lv,
+                        void* stream) {
+  const StepArgs a = step_args(nullptr, kv, cos, sin, pos, 1, kv_heads, 1, rope_len, 1, chunk, slots);
+  if (rope_len > (1 << 28) || chunk > (1 << 28) || slots > (1 << 28) || !step_ok(a, B) || !lkt || !lv)
+    return FL_ERR_INVALID_ARGUMENT;
+  fl_refresh_step_out_kernel<<<(unsigned)B, 256, 0, static_cast<hipStream_t>(stream)>>>(
+      a, static_cast<bf16_bits*>(lkt), static_cast<bf16_bits*>(lv));
+  return hip_status(hipGetLastError());
+}
+
+int fl_mask_scores(const void* scores, int64_t rows, int64_t lk, int64_t lq, int mode, const int64_t* pos,
+                   int64_t period, float scale, float* out, void* stream) {
+  if (rows <= 0 || lk <= 0 || lq <= 0 || rows > ((int64_t)1 << 40) / lk || lk > (1 << 30) || lq > (1 << 30) ||
+      mode < 0 || mode > 2 || (mode > 0 && (!pos || period <= 0 || period > (1 << 30))) || !scores || !out)
+    return FL_ERR_INVALID_ARGUMENT;
+  const int64_t n = rows * lk;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bf16_bits* p = static_cast<const bf16_bits*>(scores);
+  const bool vec = lk % 4 == 0 && aligned(scores, 8) && aligned(out, 16);
+  if (cdiv(n, vec ? 1024 : 256) >= ((int64_t)1 << 31)) return FL_ERR_INVALID_ARGUMENT;
+  if (vec) {
+    fl_mask_scores_kernel<<<(unsigned)cdiv(n, 1024), 256, 0, s>>>(p, (uint64_t)n, (uint32_t)lk, (uint32_t)lq, mode, pos,
+                                                                  (int)period, scale, out);
+  } else {
+    fl_mask_scores_any_kernel<<<(unsigned)cdiv(n, 256), 256, 0, s>>>(p, (uint64_t)n, (uint32_t)lk, (uint32_t)lq, mode,
+                                                                     pos, (int)period, scale, out);
+  }
+  return hip_status(hipGetLastError());
+}
+
+int fl_mix(const void* y, const void* g, const void* mix_logit, int mix_dtype, int64_t n, void* out, void* stream) {
+  if (!dtype_ok(mix_dtype)) return FL_ERR_DTYPE;
+  if (n <= 0 || n > ((int64_t)1 << 31) - 1 || !y || !g || !mix_logit || !out) return FL_ERR_INVALID_ARGUMENT;
+  fl_mix_kernel<<<(unsigned)cdiv(n, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+      static_cast<const bf16_bits*>(y), static_cast<const bf16_bits*>(g), mix_logit, mix_dtype == FL_DTYPE_BF16,
+      (uint32_t)n, static_cast<bf16_bits*>(out));
+  return hip_status(hipGetLastError());
+}
+
+}  // extern "C"

@@ -125,6 +125,22 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     return torch.cat((a * cos - b * sin, b * cos + a * sin), dim=-1)
 
 
+def _mask_scores_takes(raw: torch.Tensor) -> bool:
+    return (raw.dtype == torch.bfloat16 and no_grad_needed(raw) and raw.is_contiguous()
+            and 0 < raw.numel() < 1 << 39 and raw.data_ptr() % 2 == 0 and eager(raw))
+
+
+def mask_scores(raw: torch.Tensor, lq: int, mode: int, pos: Optional[torch.Tensor], period: int,
+                hd: int) -> torch.Tensor:
+    """``raw * hd ** -0.5`` in fp32, -inf where a row's limit hides the column (``fl_mask_scores``): the
+    bits of ``raw.float() * hd ** -0.5`` with a mask filled in, in one pass."""
+    out = torch.empty(raw.shape, device=raw.device, dtype=torch.float32)
+    lk = raw.shape[-1]
+    nat.check(nat.load().fl_mask_scores(nat.ptr(raw), raw.numel() // lk, lk, lq, mode, nat.ptr(pos), period,
+                                        hd ** -0.5, nat.ptr(out), nat.stream_handle(raw.device)), "fl_mask_scores")
+    return out
+
+
 def gqa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                   allowed: Optional[torch.Tensor], causal: bool) -> torch.Tensor:
     """softmax(q k^T / sqrt(hd) + mask) v with grouped KV heads (query head h reads KV head
@@ -139,7 +155,12 @@ def gqa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     rep = hq // hkv
     qg = q.reshape(n, hkv, rep * lq, hd)
     kt = k.transpose(-1, -2).contiguous()
-    scores = torch.matmul(qg, kt).float().view(n, hkv, rep, lq, lk) * (hd ** -0.5)
+    raw = torch.matmul(qg, kt)
+    if causal and allowed is None and lq == lk and _mask_scores_takes(raw):
+        scores = mask_scores(raw, lq, 0, None, 0, hd).view(n, hkv, rep, lq, lk)
+        p = torch.softmax(scores, dim=-1).to(v.dtype).view(n, hkv, rep * lq, lk)
+        return torch.matmul(p, v.contiguous()).view(n, hq, lq, hd)
+    scores = raw.float().view(n, hkv, rep, lq, lk) * (hd ** -0.5)
     if causal:
         i = torch.arange(lq, device=q.device)
         mask = i[:, None] >= torch.arange(lk, device=q.device)[None, :]
@@ -337,6 +358,55 @@ class LandmarkAttention(nn.Module):
         st["lat_sum"] = latent[:, full * c:].float().sum(1)
         return out, st
 
+    def _native_step(self, qlat: torch.Tensor, pos: torch.Tensor, st: Dict[str, torch.Tensor]) -> bool:
+        """The kernels of ``fl_refresh_step_in`` / ``_out`` take this token's projection [B, q | latent].
+        They give the stock ops' bits, so they run under autocast too."""
+        b, h, hd, w, c = qlat.shape[0], self.kv_heads, self.head_dim, self.local_window, self.landmark_chunk
+        state = tuple(st[k] for k in ("kt", "v", "lkt", "lv", "lat_sum"))
+        mix = self.global_mix_logit
+        return (type(self) is LandmarkAttention and qlat.dtype == torch.bfloat16 and qlat.ndim == 2 and hd == 64
+                and c & (c - 1) == 0 and 0 < b <= 1 << 20 and max(w, c, self._rope_len) < 1 << 28
+                and self.q_heads <= 4096 and self.latent_dim <= 1 << 16 and mix.dtype in KERNEL_DTYPES
+                and no_grad_needed(qlat, mix, *self.kv_up.parameters()) and eager(qlat, pos, mix, *state)
+                and qlat.is_contiguous() and pos.dtype == torch.int64 and pos.numel() == 1
+                and all(t.is_contiguous() for t in state) and st["lat_sum"].dtype == torch.float32
+                and all(t.dtype == qlat.dtype for t in state[:4])
+                and st["kt"].shape == (b, h, hd, w) and st["v"].shape == (b, h, w, hd)
+                and st["lat_sum"].shape == (b, self.latent_dim) and 0 < st["lv"].shape[2] < 1 << 28
+                and st["lkt"].shape == (b, h, hd, st["lv"].shape[2]) and st["lv"].shape == (b, h, st["lv"].shape[2], hd))
+
+    def _run_native_step(self, qlat: torch.Tensor, pos: torch.Tensor, st: Dict[str, torch.Tensor]) -> torch.Tensor:
+        lib, stream = nat.load(), nat.stream_handle(qlat.device)
+        b, hd, hq, hkv, c = qlat.shape[0], self.head_dim, self.q_heads, self.kv_heads, self.landmark_chunk
+        dev, dt = qlat.device, qlat.dtype
+        kv = self.kv_up(qlat[:, self.q_width:]).contiguous()
+        cos, sin = rope_cos_sin(dev, dt, self._rope_len, hd)
+        q = torch.empty((b, self.q_width), device=dev, dtype=dt)
+        mean = torch.empty((b, self.latent_dim), device=dev, dtype=dt)
+        nat.check(lib.fl_refresh_step_in(
+            nat.ptr(qlat), nat.ptr(kv), nat.ptr(cos), nat.ptr(sin), nat.ptr(pos), b, hq, hkv, self.latent_dim,
+            self._rope_len, self.local_window, c, nat.ptr(q), nat.ptr(st["kt"]), nat.ptr(st["v"]),
+            nat.ptr(st["lat_sum"]), nat.ptr(mean), stream), "fl_refresh_step_in")
+        qg = q.view(b, hkv, hq // hkv, hd)
+
+        def attend(keys, values, mode, period):
+            s = mask_scores(torch.matmul(qg, keys).contiguous(), 1, mode, pos, period, hd)
+            return torch.matmul(torch.softmax(s, -1).to(dt), values).contiguous()
+
+        # window slots written so far, and the null slot with the landmarks of completed chunks
+        local = attend(st["kt"], st["v"], 1, self.local_window)
+        landmarks = attend(st["lkt"], st["lv"], 2, c)
+        y = torch.empty((b, self.dim), device=dev, dtype=dt)
+        nat.check(lib.fl_mix(nat.ptr(local), nat.ptr(landmarks), nat.ptr(self.global_mix_logit),
+                             nat.dtype_code(self.global_mix_logit.dtype), y.numel(), nat.ptr(y), stream), "fl_mix")
+        # the running mean's landmark is (re)written every step and becomes visible once its chunk is
+        # complete (slot chunk + 1 <= chunk of later tokens)
+        land = self.kv_up(mean).contiguous()
+        nat.check(lib.fl_refresh_step_out(
+            nat.ptr(land), nat.ptr(cos), nat.ptr(sin), nat.ptr(pos), b, hkv, self._rope_len, c, st["lv"].shape[2],
+            nat.ptr(st["lkt"]), nat.ptr(st["lv"]), stream), "fl_refresh_step_out")
+        return self.out_proj(y)
+
     def step(self, x_t: torch.Tensor, pos: torch.Tensor, st: Dict[str, torch.Tensor]) -> torch.Tensor:
         """One token at position ``pos`` (0-d int64 device tensor): x_t [B, dim] -> [B, dim].
 
@@ -346,7 +416,10 @@ class LandmarkAttention(nn.Module):
         b = x_t.shape[0]
         hd, hq, hkv = self.head_dim, self.q_heads, self.kv_heads
         w, c = self.local_window, self.landmark_chunk
-        qraw, latent = self.q_latent_proj(x_t).split((self.q_width, self.latent_dim), dim=-1)
+        qlat = self.q_latent_proj(x_t)
+        if self._native_step(qlat, pos, st) and x_t.dtype == qlat.dtype:
+            return self._run_native_step(qlat, pos, st)
+        qraw, latent = qlat.split((self.q_width, self.latent_dim), dim=-1)
         kraw, vraw = self.kv_up(latent).split(hkv * hd, dim=-1)
         cos, sin = rope_cos_sin(x_t.device, x_t.dtype, self._rope_len, hd)
         # gathered on the device (no host read of the position); clamped to the table, so a

@@ -402,6 +402,29 @@ int fl_swiglu_backward(const void* gate_up, const void* gy, int dtype, int64_t r
 int fl_field_params_backward(const float* radius_logit, const float* theta, int64_t C, const float* gtr,
                              const float* gti, const float* ggamma, float* g_logit, float* g_theta, void* stream);
 
+/*
+ * Elementwise work of the refresh blocks in the stock ops' own roundings (same file, 131-253), bf16:
+ * fl_refresh_step_in: one token at *pos (a device int64): q [B, q_heads * 64] = rotated queries of
+ *   qlat [B, q_heads * 64 + latent]; rotated keys and values of kv [B, 2 * kv_heads * 64] into slot
+ *   *pos % window of kt [B, kv_heads, 64, window] and v [B, kv_heads, window, 64]; lat_sum [B, latent]
+ *   (fp32) += latent, restarted where *pos % chunk is 0 (chunk a power of two); mean = lat_sum / chunk;
+ * fl_refresh_step_out: the rotated key and the value of kv into slot min(*pos / chunk + 1, slots - 1) of
+ *   lkt [B, kv_heads, 64, slots] and lv [B, kv_heads, slots, 64];
+ *   positions are clamped to the tables cos / sin [rope_len, 32];
+ * fl_mask_scores: out [rows, lk] fp32 = scale * scores where column j <= the row's limit, else -inf; limit:
+ *   mode 0 row % lq (causal), 1 *pos % period, 2 *pos / period;
+ * fl_mix: out = y + sigmoid(mix_logit[0]) * g over n values.
+ */
+int fl_refresh_step_in(const void* qlat, const void* kv, const void* cos, const void* sin, const int64_t* pos,
+                       int64_t B, int64_t q_heads, int64_t kv_heads, int64_t latent, int64_t rope_len, int64_t window,
+                       int64_t chunk, void* q, void* kt, void* v, float* lat_sum, void* mean, void* stream);
+int fl_refresh_step_out(const void* kv, const void* cos, const void* sin, const int64_t* pos, int64_t B,
+                        int64_t kv_heads, int64_t rope_len, int64_t chunk, int64_t slots, void* lkt, void* lv,
+                        void* stream);
+int fl_mask_scores(const void* scores, int64_t rows, int64_t lk, int64_t lq, int mode, const int64_t* pos,
+                   int64_t period, float scale, float* out, void* stream);
+int fl_mix(const void* y, const void* g, const void* mix_logit, int mix_dtype, int64_t n, void* out, void* stream);
+
 /* Library version string (host function). No counterpart in the reference. */
 const char* fl_version(void);
 

@@ -130,3 +130,44 @@ def test_softpatch_against_fp32(dev, dim, rank, B, T):
     print(f"[case] softpatch native {e:.2e} stock {e_stock:.2e}", flush=True)
     assert e <= 1.1 * e_stock + 1e-4 and e <= 1e-2
     assert _norm(last, last_exp) <= 2e-2  # z rounded to bf16, boundaries from a bf16 score
+
+
+class _Stock(M.LandmarkAttention):
+    """The same attention through the stock ops (the kernels take the class itself only)."""
+
+
+@pytest.mark.parametrize("heads,kv,window,chunk,B,prompt", [(16, 4, 256, 256, 5, 250), (8, 2, 64, 32, 1, 60), (8, 8, 100, 16, 3, 95),
+                                                            (4, 1, 33, 4, 2, 30)])
+@pytest.mark.parametrize("autocast", [False, True], ids=["plain", "autocast"])
+def test_attention_step_gives_the_stock_bits(dev, heads, kv, window, chunk, B, prompt, autocast):
+    """Tokens across the end of a window and of a chunk, to the last position the state is sized for:
+    outputs and every state equal the stock ops' bit for bit."""
+    print(f"[case] refresh step bits heads={heads}/{kv} window={window} chunk={chunk} B={B}", flush=True)
+    att = _block(dev, heads, kv, window, chunk, seed=window).attn
+    stock = copy.deepcopy(att)
+    stock.__class__ = _Stock
+    n = 12
+    x = torch.randn(B, prompt + n, 64 * heads, device=dev, generator=torch.Generator(device=dev).manual_seed(B)).to(torch.bfloat16)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        _, st = stock.prefill(x[:, :prompt], prompt + n)
+        att._rope_len = stock._rope_len
+        mine = {k: v.clone() for k, v in st.items()}
+        for i in range(n):
+            pos = torch.tensor(prompt + i, device=dev)
+            assert att._native_step(att.q_latent_proj(x[:, prompt + i]), pos, mine)
+            a, b = att.step(x[:, prompt + i], pos, mine), stock.step(x[:, prompt + i], pos, st)
+            assert torch.equal(a, b), i
+            for k in st:
+                assert torch.equal(mine[k], st[k]), (i, k)
+
+
+@pytest.mark.parametrize("B,T,window", [(2, 300, 64), (1, 77, 128), (3, 130, 256)])
+def test_causal_scores_under_autocast_give_the_stock_bits(dev, B, T, window):
+    """Prompts under autocast: the scaled, masked scores in one pass leave every bit as it was."""
+    print(f"[case] masked scores B={B} T={T} window={window}", flush=True)
+    att = _block(dev, 8, 2, window, 32, seed=T).attn
+    x = torch.randn(B, T, 512, device=dev, generator=torch.Generator(device=dev).manual_seed(T)).to(torch.bfloat16)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        stock = att(x).detach()  # gradients enabled: the stock ops
+        with torch.no_grad():
+            assert torch.equal(att(x), stock)
