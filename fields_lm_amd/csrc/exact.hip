@@ -1,6 +1,7 @@
-// exact.hip — elementwise work of the refresh blocks in the stock ops' own roundings, bit for bit, so
-// that it may run under autocast too, where a generation loop keeps its bits (reference: src/
-// fields_official/reference/official_source/field_fusion_system_smoke_v21.py:131-253). bf16 values are
+// exact.hip — elementwise work of the refresh and Mamba-2 blocks in the stock ops' own roundings, bit
+// for bit, so that it may run under autocast too, where a generation loop keeps its bits (reference:
+// src/fields_official/reference/official_source/field_fusion_system_smoke_v21.py:131-253,
+// field_fusion_wiki100_mamba2_v25.py:73-91). bf16 values are
 // rounded after every operation, as an op on bf16 tensors does; sums and products with an order of
 // their own (the matrix products, softmax) stay with the stock ops.
 //
@@ -134,6 +135,97 @@ __global__ __launch_bounds__(256) void fl_mix_kernel(const bf16_bits* __restrict
   out[i] = (bf16_bits)bf16_bits_of(bf(y + i) + t);
 }
 
+// ---- Mamba-2 ----
+
+// silu(bias + sum_k w[k] in[t - 3 + k]) of bf16 rows in fp32, each product and each sum rounded, in the
+// stock order: a chain of five fp32 passes (75 MB each at 8,192 tokens) in one.
+__global__ __launch_bounds__(256) void fl_conv_silu_kernel(const bf16_bits* __restrict__ x, int64_t sb, int64_t st,
+                                                           int L, int channels, const void* w, const void* bias,
+                                                           int is16, float* __restrict__ out) {
+  const int c = blockIdx.x * 256 + threadIdx.x, t0 = blockIdx.y * 16;
+  const int64_t b = blockIdx.z;
+  if (c >= channels) return;
+  float wt[4], bs;
+  if (is16) {
+    for (int k = 0; k < 4; ++k) wt[k] = bf(static_cast<const bf16_bits*>(w) + 4 * c + k);
+    bs = bf(static_cast<const bf16_bits*>(bias) + c);
+  } else {
+    for (int k = 0; k < 4; ++k) wt[k] = static_cast<const float*>(w)[4 * c + k];
+    bs = static_cast<const float*>(bias)[c];
+  }
+  const bf16_bits* p = x + b * sb + c;
+  float in[19];
+#pragma unroll
+  for (int i = 0; i < 19; ++i) {
+    const int t = t0 - 3 + i;
+    in[i] = bf(p + (int64_t)min(max(t, 0), L - 1) * st);
+    if (t < 0) in[i] = 0.f;
+  }
+  float* o = out + (b * L + t0) * channels + c;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    if (t0 + i >= L) break;
+    float v = in[i] * wt[0];
+    v = bs + v;
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+      const float m = in[i + k] * wt[k];
+      v = v + m;
+    }
+    o[(int64_t)i * channels] = v / (1.0f + expf(-v));
+  }
+}
+
+// [b, h, c, s, s] = cb[b, c] * exp(acs_i - acs_j) for j <= i, times 0 above, rounded to the bf16 operand
+// that autocast makes of it: six fp32 passes over the largest tensor of the block in one.
+__global__ __launch_bounds__(256) void fl_decay_product_kernel(const bf16_bits* __restrict__ cb,
+                                                               const float* __restrict__ acs, int H, int n_chunks,
+                                                               int s, bf16_bits* __restrict__ out) {
+  const int row_vecs = s / 8;
+  const int idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= s * row_vecs) return;
+  const int i = idx / row_vecs, j0 = 8 * (idx - i * row_vecs), c = blockIdx.y;
+  const int64_t bh = blockIdx.z, b = bh / H;
+  const float* a = acs + (bh * n_chunks + c) * s;
+  float v[8], o[8];
+  Vec<bf16_bits, 8>::load(cb + ((b * n_chunks + c) * s + i) * s + j0, v);
+  const float ai = a[i];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float d = j0 + e <= i ? expf(ai - a[j0 + e]) : 0.f;
+    o[e] = v[e] * d;
+  }
+  Vec<bf16_bits, 8>::store(out + (((bh * n_chunks + c) * s + i) * s + j0), o);
+}
+
+// One token's state update, s = s * decay then s + xdt * b, each rounded, and the bf16 operand that
+// autocast makes of the state for its product with C: 500 MB of traffic in 168 MB at 64 x 32 heads.
+__global__ __launch_bounds__(256) void fl_state_update_kernel(const float* __restrict__ decay,
+                                                              const float* __restrict__ xdt,
+                                                              const float* __restrict__ bm, int64_t bm_stride,
+                                                              int H, int P, int N, float* __restrict__ ssm,
+                                                              bf16_bits* __restrict__ ssm16) {
+  const int64_t bh = blockIdx.x, b = bh / H;
+  const float d = decay[bh];
+  for (int i = threadIdx.x; i < P * N / 4; i += 256) {
+    const int p = 4 * i / N, n = 4 * i - p * N;
+    float* at = ssm + bh * P * N + 4 * (int64_t)i;
+    f32x4 v = *reinterpret_cast<const f32x4*>(at);
+    const float x = xdt[bh * P + p];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float t = x * bm[b * bm_stride + n + e];
+      const float q = v[e] * d;
+      v[e] = q + t;
+    }
+    *reinterpret_cast<f32x4*>(at) = v;
+    u32x2 w;
+    w.x = bf16_pair(v[0], v[1]);
+    w.y = bf16_pair(v[2], v[3]);
+    *reinterpret_cast<u32x2*>(ssm16 + bh * P * N + 4 * (int64_t)i) = w;
+  }
+}
+
 bool step_ok(const StepArgs& a, int64_t B) {
   return B > 0 && B <= (1 << 20) && a.q_heads > 0 && a.q_heads <= 4096 && a.kv_heads > 0 && a.kv_heads <= 4096 &&
          a.latent > 0 && a.latent <= (1 << 16) && a.rope_len > 0 && a.window > 0 && a.chunk > 0 &&
@@ -193,6 +285,39 @@ int fl_mask_scores(const void* scores, int64_t rows, int64_t lk, int64_t lq, int
     fl_mask_scores_any_kernel<<<(unsigned)cdiv(n, 256), 256, 0, s>>>(p, (uint64_t)n, (uint32_t)lk, (uint32_t)lq, mode,
                                                                      pos, (int)period, scale, out);
   }
+  return hip_status(hipGetLastError());
+}
+
+int fl_conv_silu(const void* x, int64_t stride_b, int64_t stride_t, int64_t B, int64_t L, int64_t channels,
+                 const void* w, const void* bias, int w_dtype, float* out, void* stream) {
+  if (!dtype_ok(w_dtype)) return FL_ERR_DTYPE;
+  if (B <= 0 || B > 65535 || L <= 0 || L > 65535 * 16 || channels <= 0 || channels > (1 << 24) ||
+      stride_t < channels || stride_b < 0 || !x || !w || !bias || !out)
+    return FL_ERR_INVALID_ARGUMENT;
+  fl_conv_silu_kernel<<<dim3((unsigned)cdiv(channels, 256), (unsigned)cdiv(L, 16), (unsigned)B), 256, 0,
+                        static_cast<hipStream_t>(stream)>>>(static_cast<const bf16_bits*>(x), stride_b, stride_t, (int)L,
+                                                            (int)channels, w, bias, w_dtype == FL_DTYPE_BF16, out);
+  return hip_status(hipGetLastError());
+}
+
+int fl_decay_product(const void* cb, const float* acs, int64_t B, int64_t heads, int64_t n_chunks, int64_t s,
+                     void* out, void* stream) {
+  if (B <= 0 || heads <= 0 || B * heads > 65535 || n_chunks <= 0 || n_chunks > 65535 || s <= 0 || s % 8 || s > 4096 ||
+      !cb || !acs || !out || !aligned(cb, 16) || !aligned(out, 16))
+    return FL_ERR_INVALID_ARGUMENT;
+  fl_decay_product_kernel<<<dim3((unsigned)cdiv(s * (s / 8), 256), (unsigned)n_chunks, (unsigned)(B * heads)), 256, 0,
+                            static_cast<hipStream_t>(stream)>>>(static_cast<const bf16_bits*>(cb), acs, (int)heads,
+                                                                (int)n_chunks, (int)s, static_cast<bf16_bits*>(out));
+  return hip_status(hipGetLastError());
+}
+
+int fl_state_update(const float* decay, const float* xdt, const float* bm, int64_t bm_stride, int64_t B, int64_t heads,
+                    int64_t P, int64_t N, float* ssm, void* ssm16, void* stream) {
+  if (B <= 0 || heads <= 0 || B * heads > (1 << 30) || P <= 0 || N <= 0 || N % 4 || P * N > (1 << 24) ||
+      bm_stride < N || !decay || !xdt || !bm || !ssm || !ssm16 || !aligned(ssm, 16) || !aligned(ssm16, 8))
+    return FL_ERR_INVALID_ARGUMENT;
+  fl_state_update_kernel<<<(unsigned)(B * heads), 256, 0, static_cast<hipStream_t>(stream)>>>(
+      decay, xdt, bm, bm_stride, (int)heads, (int)P, (int)N, ssm, static_cast<bf16_bits*>(ssm16));
   return hip_status(hipGetLastError());
 }
 

@@ -535,6 +535,15 @@ class GatedRMSNorm(nn.Module):
         return y * self.weight.float()
 
 
+def _autocast_operands(product: torch.Tensor, *others: torch.Tensor) -> bool:
+    """Under bf16 autocast without gradients, the state of affairs in which the Mamba-2 blocks' fp32
+    intermediates become bf16 operands: ``product`` came out of one such product. The kernels of
+    ``csrc/exact.hip`` then form those operands with the stock ops' bits."""
+    return (torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16
+            and product.dtype == torch.bfloat16 and product.numel() > 0 and no_grad_needed(product, *others)
+            and eager(product, *others) and all(t.dtype == torch.float32 for t in others))
+
+
 def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None):
     """State-space-duality scan of Mamba-2 in fp32 (the chunked algorithm of Dao & Gu, 2024):
 
@@ -557,11 +566,18 @@ def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None):
     Bc = Bm.float().view(b, c, chunk, n)
     Cc = Cm.float().view(b, c, chunk, n)
     # intra-chunk: y_i = sum_{j<=i} (C_i.B_j) exp(acs_i - acs_j) xdt_j
-    seg = acs[..., :, None] - acs[..., None, :]                                        # [b,h,c,s,s]
-    causal = torch.ones(chunk, chunk, device=x.device, dtype=torch.bool).tril()
-    decay = torch.exp(seg.masked_fill(~causal, float("-inf")))
     cb = torch.matmul(Cc, Bc.transpose(-1, -2).contiguous())                            # [b,c,s,s]
-    y = torch.matmul(cb[:, None] * decay, xdt)                                          # [b,h,c,s,p]
+    if _autocast_operands(cb, acs) and chunk % 8 == 0 and chunk <= 4096 and b * h <= 65535 and 0 < c <= 65535 \
+            and cb.is_contiguous() and cb.data_ptr() % 16 == 0:
+        acs = acs.contiguous()
+        weights = torch.empty((b, h, c, chunk, chunk), device=x.device, dtype=cb.dtype)
+        nat.check(nat.load().fl_decay_product(nat.ptr(cb), nat.ptr(acs), b, h, c, chunk, nat.ptr(weights),
+                                              nat.stream_handle(x.device)), "fl_decay_product")
+    else:
+        seg = acs[..., :, None] - acs[..., None, :]                                    # [b,h,c,s,s]
+        causal = torch.ones(chunk, chunk, device=x.device, dtype=torch.bool).tril()
+        weights = cb[:, None] * torch.exp(seg.masked_fill(~causal, float("-inf")))
+    y = torch.matmul(weights, xdt)                                                      # [b,h,c,s,p]
     # chunk states from 0: sum_j exp(acs_end - acs_j) xdt_j B_j^T
     w_end = torch.exp(acs[..., -1:] - acs)                                              # [b,h,c,s]
     states = torch.matmul((xdt * w_end[..., None]).transpose(-1, -2).contiguous(), Bc[:, None])  # [b,h,c,p,n]
@@ -669,20 +685,35 @@ class Mamba2Mixer(nn.Module):
                 "fl_mamba_prefill", zxbcdt, l, (b, l, self.nheads), (zxbcdt.stride(0), zxbcdt.stride(1)), u.dtype,
                 state))
             return (out, self._new_state(xbc_raw, state)) if return_state else out
-        # causal depthwise convolution as d_conv shifted multiply-adds in the channel-last
-        # layout: out[t] = bias + sum_k w[k] * in[t - (d_conv-1) + k]
-        w = self.conv1d.weight.float()[:, 0]                                           # [C, K]
-        xp = F.pad(xbc_raw.float(), (0, 0, self.d_conv - 1, 0))
-        xbc = self.conv1d.bias.float() + xp[:, :l] * w[:, 0]
-        for k in range(1, self.d_conv):
-            xbc = torch.addcmul(xbc, xp[:, k:k + l], w[:, k])
-        x, bm, cm, dt = self._ssm_in(F.silu(xbc), dt)
+        x, bm, cm, dt = self._ssm_in(self._conv_silu(xbc_raw), dt)
         A = -torch.exp(self.A_log.float())
         xh = x.reshape(b, l, self.nheads, self.headdim)
         y, state = ssd_chunked(xh, dt, A, bm, cm, self.chunk_size)
         y = y + self.D.float()[:, None] * xh
         out = self.out_proj(self.norm(y.reshape(b, l, self.d_inner), z).to(u.dtype))
         return (out, self._new_state(xbc_raw, state)) if return_state else out
+
+    def _conv_silu(self, xbc_raw: torch.Tensor) -> torch.Tensor:
+        """silu of the causal depthwise convolution, fp32 [b, l, channels]: d_conv shifted multiply-adds in
+        the channel-last layout, out[t] = bias + sum_k w[k] * in[t - (d_conv-1) + k]."""
+        b, l, channels = xbc_raw.shape
+        weight, bias = self.conv1d.weight, self.conv1d.bias
+        if (xbc_raw.dtype == torch.bfloat16 and self.d_conv == 4 and no_grad_needed(xbc_raw, weight, bias)
+                and eager(xbc_raw, weight, bias) and xbc_raw.stride(-1) == 1 and 0 < b <= 65535 and 0 < l <= 1 << 19
+                and xbc_raw.stride(1) >= channels and xbc_raw.stride(0) >= 0 and weight.dtype == bias.dtype
+                and weight.dtype in KERNEL_DTYPES and weight.is_contiguous() and bias.is_contiguous()):
+            out = torch.empty((b, l, channels), device=xbc_raw.device, dtype=torch.float32)
+            nat.check(nat.load().fl_conv_silu(
+                nat.ptr(xbc_raw), xbc_raw.stride(0), xbc_raw.stride(1), b, l, channels, nat.ptr(weight),
+                nat.ptr(bias), nat.dtype_code(weight.dtype), nat.ptr(out), nat.stream_handle(xbc_raw.device)),
+                "fl_conv_silu")
+            return out
+        w = weight.float()[:, 0]                                                        # [C, K]
+        xp = F.pad(xbc_raw.float(), (0, 0, self.d_conv - 1, 0))
+        xbc = bias.float() + xp[:, :l] * w[:, 0]
+        for k in range(1, self.d_conv):
+            xbc = torch.addcmul(xbc, xp[:, k:k + l], w[:, k])
+        return F.silu(xbc)
 
     def _new_state(self, xbc_raw: torch.Tensor, ssm: torch.Tensor) -> Dict[str, torch.Tensor]:
         """Decode state after a sequence: the last d_conv convolution inputs and the SSM state."""
@@ -716,8 +747,20 @@ class Mamba2Mixer(nn.Module):
         A = -torch.exp(self.A_log.float())
         xh = x.view(b, self.nheads, self.headdim)
         decay = torch.exp(dt * A)                                                       # [B,H]
-        ssm.mul_(decay[:, :, None, None]).add_((xh * dt[..., None])[..., None] * bm[:, None, None, :])
-        y = torch.matmul(ssm, cm[:, None, :, None]).squeeze(-1) + self.D.float()[:, None] * xh
+        xdt = xh * dt[..., None]
+        if (_autocast_operands(zxbcdt, ssm, decay, xdt, bm) and ssm.is_contiguous() and decay.is_contiguous()
+                and xdt.is_contiguous() and bm.stride(-1) == 1 and self.d_state % 4 == 0
+                and bm.stride(0) >= self.d_state and ssm.data_ptr() % 16 == 0
+                and ssm.shape == (b, self.nheads, self.headdim, self.d_state)
+                and b * self.nheads <= 1 << 30 and self.headdim * self.d_state <= 1 << 24):
+            operand = torch.empty(ssm.shape, device=ssm.device, dtype=torch.bfloat16)  # what the product reads
+            nat.check(nat.load().fl_state_update(
+                nat.ptr(decay), nat.ptr(xdt), nat.ptr(bm), bm.stride(0), b, self.nheads, self.headdim, self.d_state,
+                nat.ptr(ssm), nat.ptr(operand), nat.stream_handle(ssm.device)), "fl_state_update")
+        else:
+            ssm.mul_(decay[:, :, None, None]).add_(xdt[..., None] * bm[:, None, None, :])
+            operand = ssm
+        y = torch.matmul(operand, cm[:, None, :, None]).squeeze(-1) + self.D.float()[:, None] * xh
         return self.out_proj(self.norm(y.reshape(b, self.d_inner), z).to(u_t.dtype))
 
 

@@ -413,7 +413,13 @@ int fl_field_params_backward(const float* radius_logit, const float* theta, int6
  *   positions are clamped to the tables cos / sin [rope_len, 32];
  * fl_mask_scores: out [rows, lk] fp32 = scale * scores where column j <= the row's limit, else -inf; limit:
  *   mode 0 row % lq (causal), 1 *pos % period, 2 *pos / period;
- * fl_mix: out = y + sigmoid(mix_logit[0]) * g over n values.
+ * fl_mix: out = y + sigmoid(mix_logit[0]) * g over n values;
+ * and of the Mamba-2 blocks as they run under bf16 autocast (field_fusion_wiki100_mamba2_v25.py:73-91):
+ * fl_conv_silu: out [B, L, channels] fp32 = silu(causal depthwise conv of width 4), x bf16 with strides;
+ * fl_decay_product: out [B, heads, n_chunks, s, s] bf16 = cb [B, n_chunks, s, s] exp(acs_i - acs_j) for
+ *   j <= i and cb * 0 above, acs [B, heads, n_chunks, s] fp32, s a multiple of 8;
+ * fl_state_update: ssm [B, heads, P, N] = ssm decay [B, heads] + xdt [B, heads, P] bm [B, N] in place
+ *   (rows of bm bm_stride apart), and ssm16 its bf16 copy; N a multiple of 4.
  */
 int fl_refresh_step_in(const void* qlat, const void* kv, const void* cos, const void* sin, const int64_t* pos,
                        int64_t B, int64_t q_heads, int64_t kv_heads, int64_t latent, int64_t rope_len, int64_t window,
@@ -423,6 +429,12 @@ int fl_refresh_step_out(const void* kv, const void* cos, const void* sin, const 
                         void* stream);
 int fl_mask_scores(const void* scores, int64_t rows, int64_t lk, int64_t lq, int mode, const int64_t* pos,
                    int64_t period, float scale, float* out, void* stream);
+int fl_conv_silu(const void* x, int64_t stride_b, int64_t stride_t, int64_t B, int64_t L, int64_t channels,
+                 const void* w, const void* bias, int w_dtype, float* out, void* stream);
+int fl_decay_product(const void* cb, const float* acs, int64_t B, int64_t heads, int64_t n_chunks, int64_t s,
+                     void* out, void* stream);
+int fl_state_update(const float* decay, const float* xdt, const float* bm, int64_t bm_stride, int64_t B, int64_t heads,
+                    int64_t P, int64_t N, float* ssm, void* ssm16, void* stream);
 int fl_mix(const void* y, const void* g, const void* mix_logit, int mix_dtype, int64_t n, void* out, void* stream);
 
 /* Library version string (host function). No counterpart in the reference. */

@@ -135,3 +135,26 @@ def test_mamba_other_geometries_and_modes_keep_the_stock_ops(dev):
         both = torch.stack([m(x), m(2 * x)])
     assert oracle.rel_err(tangent.cpu(), slope.cpu()) <= 1e-2
     assert oracle.rel_err(batched.cpu(), both.cpu()) <= 1e-5
+
+
+@pytest.mark.parametrize("dim,B,L,weights", [(128, 2, 70, "bf16"), (512, 1, 300, "bf16"), (128, 1, 3, "fp32"), (1024, 2, 257, "fp32")])
+def test_mamba_under_autocast_gives_the_stock_bits(dev, dim, B, L, weights):
+    """Under autocast the convolution, the decayed products and the state update run in kernels that keep
+    every bit of the stock ops (which run whenever a gradient is needed, and in a subclass's step)."""
+    print(f"[case] mamba autocast bits dim={dim} B={B} L={L} {weights}", flush=True)
+    m = _mixer(dev, dim, seed=L)
+    if weights == "bf16":
+        m = M.cast_for_inference(m)
+    u = torch.randn(B, L + 3, dim, device=dev, generator=torch.Generator(device=dev).manual_seed(L))
+    u = u.to(torch.bfloat16) if weights == "bf16" else u
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        stock, st_stock = m(u[:, :L], return_state=True)
+        with torch.no_grad():
+            y, st = m(u[:, :L], return_state=True)
+            assert torch.equal(y, stock.detach())
+            for k in st:
+                assert torch.equal(st[k], st_stock[k].detach()), k
+            other = {"conv": st["conv"].clone(), "ssm": st["ssm"].transpose(2, 3).contiguous().transpose(2, 3)}
+            for i in range(3):  # a transposed state takes the stock ops
+                a, b = m.step(u[:, L + i], st), m.step(u[:, L + i], other)
+                assert torch.equal(a, b) and torch.equal(st["ssm"], other["ssm"]) and torch.equal(st["conv"], other["conv"])
