@@ -141,13 +141,29 @@ def mask_scores(raw: torch.Tensor, lq: int, mode: int, pos: Optional[torch.Tenso
     return out
 
 
+def masked_softmax(raw: torch.Tensor, lq: int, mode: int, pos: Optional[torch.Tensor], period: int,
+                   hd: int) -> torch.Tensor:
+    """bf16 softmax over the visible columns of ``raw * hd ** -0.5``, with the bits of the stock ops in
+    fp32. Up to 1,024 columns one kernel holds a row (``fl_masked_softmax``); a longer row's sum is the
+    stock softmax's own affair."""
+    lk = raw.shape[-1]
+    if lk > 1024 or raw.numel() // lk >= 1 << 32:
+        return torch.softmax(mask_scores(raw, lq, mode, pos, period, hd), -1).to(raw.dtype)
+    out = torch.empty_like(raw)
+    nat.check(nat.load().fl_masked_softmax(nat.ptr(raw), raw.numel() // lk, lk, lq, mode, nat.ptr(pos), period,
+                                           hd ** -0.5, nat.ptr(out), nat.stream_handle(raw.device)),
+              "fl_masked_softmax")
+    return out
+
+
 def gqa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
-                  allowed: Optional[torch.Tensor], causal: bool) -> torch.Tensor:
+                  allowed: Optional[torch.Tensor], causal: bool, *, chunk: int = 0) -> torch.Tensor:
     """softmax(q k^T / sqrt(hd) + mask) v with grouped KV heads (query head h reads KV head
     h // (Hq / Hkv), the grouping of v20:147-163's ``enable_gqa``).
 
     q [N, Hq, Lq, hd], k/v [N, Hkv, Lk, hd]; ``allowed`` a bool mask broadcastable to
-    [N, Hkv, Lq, Lk] (True = visible) or None; ``causal`` adds j <= i (Lq == Lk). The products run
+    [N, Hkv, Lq, Lk] (True = visible) or None; ``causal`` adds j <= i (Lq == Lk); ``chunk`` hides the
+    columns past i // chunk (a null slot and the landmarks of the completed chunks). The products run
     as plain matmuls on contiguous operands with an fp32 softmax.
     """
     n, hq, lq, hd = q.shape
@@ -156,15 +172,18 @@ def gqa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     qg = q.reshape(n, hkv, rep * lq, hd)
     kt = k.transpose(-1, -2).contiguous()
     raw = torch.matmul(qg, kt)
-    if causal and allowed is None and lq == lk and _mask_scores_takes(raw):
-        scores = mask_scores(raw, lq, 0, None, 0, hd).view(n, hkv, rep, lq, lk)
-        p = torch.softmax(scores, dim=-1).to(v.dtype).view(n, hkv, rep * lq, lk)
+    if ((chunk > 0 and lk <= 1024 and raw.numel() < 1 << 32) if not causal else lq == lk and chunk == 0) and allowed is None \
+            and v.dtype == raw.dtype and _mask_scores_takes(raw):
+        p = masked_softmax(raw, lq, 0 if causal else 3, None, chunk, hd)
         return torch.matmul(p, v.contiguous()).view(n, hq, lq, hd)
     scores = raw.float().view(n, hkv, rep, lq, lk) * (hd ** -0.5)
     if causal:
         i = torch.arange(lq, device=q.device)
         mask = i[:, None] >= torch.arange(lk, device=q.device)[None, :]
         scores = scores.masked_fill(~mask, float("-inf"))
+    if chunk > 0:
+        last = torch.arange(lq, device=q.device) // chunk
+        scores = scores.masked_fill(torch.arange(lk, device=q.device)[None, :] > last[:, None], float("-inf"))
     if allowed is not None:
         scores = scores.masked_fill(~allowed.unsqueeze(-3), float("-inf"))
     p = torch.softmax(scores, dim=-1).to(v.dtype).view(n, hkv, rep * lq, lk)
@@ -242,10 +261,7 @@ class LandmarkAttention(nn.Module):
         lk, lv = self._landmarks(latent, full, cos, sin)
         zero = lk.new_zeros((b, self.kv_heads, 1, hd))
         lk, lv = torch.cat((zero, lk), 2), torch.cat((zero, lv), 2)
-        chunk_of = torch.arange(length, device=q.device) // c
-        allowed = torch.cat((torch.ones(length, 1, device=q.device, dtype=torch.bool),
-                             torch.arange(full, device=q.device)[None, :] < chunk_of[:, None]), 1)
-        return gqa_attention(q, lk, lv, allowed, False)
+        return gqa_attention(q, lk, lv, None, False, chunk=c)
 
     def _native(self, qlat: torch.Tensor) -> bool:
         """The kernels of ``fl_refresh_attention`` take this projection [B, T, q | latent]."""
@@ -390,8 +406,8 @@ class LandmarkAttention(nn.Module):
         qg = q.view(b, hkv, hq // hkv, hd)
 
         def attend(keys, values, mode, period):
-            s = mask_scores(torch.matmul(qg, keys).contiguous(), 1, mode, pos, period, hd)
-            return torch.matmul(torch.softmax(s, -1).to(dt), values).contiguous()
+            p = masked_softmax(torch.matmul(qg, keys).contiguous(), 1, mode, pos, period, hd)
+            return torch.matmul(p, values).contiguous()
 
         # window slots written so far, and the null slot with the landmarks of completed chunks
         local = attend(st["kt"], st["v"], 1, self.local_window)

@@ -413,6 +413,8 @@ int fl_field_params_backward(const float* radius_logit, const float* theta, int6
  *   positions are clamped to the tables cos / sin [rope_len, 32];
  * fl_mask_scores: out [rows, lk] fp32 = scale * scores where column j <= the row's limit, else -inf; limit:
  *   mode 0 row % lq (causal), 1 *pos % period, 2 *pos / period;
+ * fl_masked_softmax: out [rows, lk] bf16 = softmax of the scores fl_mask_scores forms, lk <= 1024; mode 3:
+ *   limit (row % lq) / period;
  * fl_mix: out = y + sigmoid(mix_logit[0]) * g over n values;
  * and of the Mamba-2 blocks as they run under bf16 autocast (field_fusion_wiki100_mamba2_v25.py:73-91):
  * fl_conv_silu: out [B, L, channels] fp32 = silu(causal depthwise conv of width 4), x bf16 with strides;
@@ -429,6 +431,8 @@ int fl_refresh_step_out(const void* kv, const void* cos, const void* sin, const 
                         void* stream);
 int fl_mask_scores(const void* scores, int64_t rows, int64_t lk, int64_t lq, int mode, const int64_t* pos,
                    int64_t period, float scale, float* out, void* stream);
+int fl_masked_softmax(const void* scores, int64_t rows, int64_t lk, int64_t lq, int mode, const int64_t* pos,
+                      int64_t period, float scale, void* out, void* stream);
 int fl_conv_silu(const void* x, int64_t stride_b, int64_t stride_t, int64_t B, int64_t L, int64_t channels,
                  const void* w, const void* bias, int w_dtype, float* out, void* stream);
 int fl_decay_product(const void* cb, const float* acs, int64_t B, int64_t heads, int64_t n_chunks, int64_t s,

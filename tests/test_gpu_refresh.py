@@ -171,3 +171,40 @@ def test_causal_scores_under_autocast_give_the_stock_bits(dev, B, T, window):
         stock = att(x).detach()  # gradients enabled: the stock ops
         with torch.no_grad():
             assert torch.equal(att(x), stock)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("lk", [1, 5, 16, 17, 32, 33, 63, 64, 65, 127, 128, 200, 257, 512, 777, 1023, 1024, 1025])
+def test_masked_softmax_gives_the_stock_bits(dev, lk, mode):
+    """Every unroll of the row at its edges, spread scores, equal scores, a row of -inf and one infinity."""
+    if mode == 3 and lk > 1024:
+        pytest.skip("longer landmark rows take the stock ops")
+    print(f"[case] masked softmax lk={lk} mode={mode}", flush=True)
+    lq = lk if mode == 0 else 7
+    rows, period = 6 * lq, max(1, (lk + 1) // 2) if mode else 0
+    g = torch.Generator(device=dev).manual_seed(lk)
+    raw = (torch.randn(rows, lk, device=dev, generator=g) * 40).to(torch.bfloat16)
+    raw[0] = 3.0
+    raw[1] = raw[1] * 1e4
+    raw[2] = float("-inf")
+    raw[3, -1] = float("inf")
+    pos = torch.tensor(period + lk // 3, device=dev, dtype=torch.int64)
+    row = torch.arange(rows, device=dev) % lq
+    limit = {0: row, 1: (pos % max(period, 1)).expand(rows), 2: (pos // max(period, 1)).expand(rows),
+             3: row // max(period, 1)}[mode]
+    scores = (raw.float() * 64 ** -0.5).masked_fill(torch.arange(lk, device=dev)[None] > limit[:, None], float("-inf"))
+    stock = torch.softmax(scores, -1).to(torch.bfloat16)
+    got = M.masked_softmax(raw, lq, mode, pos if mode in (1, 2) else None, period, 64)
+    assert torch.equal(got.isnan(), stock.isnan())
+    assert torch.equal(got.nan_to_num(7.0), stock.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("T,window", [(1300, 512), (1100, 1024), (40, 64)])
+def test_landmark_scores_under_autocast_give_the_stock_bits(dev, T, window):
+    print(f"[case] landmark scores T={T} window={window}", flush=True)
+    att = _block(dev, 8, 2, window, 32, seed=T).attn
+    x = torch.randn(2, T, 512, device=dev, generator=torch.Generator(device=dev).manual_seed(T)).to(torch.bfloat16)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        stock = att(x).detach()  # gradients enabled: the stock ops
+        with torch.no_grad():
+            assert torch.equal(att(x), stock)
