@@ -259,15 +259,25 @@ class LandmarkAttention(nn.Module):
         if full == 0:
             return q.new_zeros(q.shape)
         lk, lv = self._landmarks(latent, full, cos, sin)
-        zero = lk.new_zeros((b, self.kv_heads, 1, hd))
+        return self._null_slot_attend(q, lk, lv)
+
+    def _null_slot_attend(self, q, lk, lv) -> torch.Tensor:
+        zero = lk.new_zeros((lk.shape[0], self.kv_heads, 1, self.head_dim))
         lk, lv = torch.cat((zero, lk), 2), torch.cat((zero, lv), 2)
-        return gqa_attention(q, lk, lv, None, False, chunk=c)
+        return gqa_attention(q, lk, lv, None, False, chunk=self.landmark_chunk)
+
+    def _plain(self, qlat: torch.Tensor) -> bool:
+        """``kv_up`` and the projection are what the kernels take their outputs for."""
+        up = self.kv_up
+        return (plain_linear(up) and up.weight.shape == (2 * self.kv_heads * self.head_dim, self.latent_dim)
+                and qlat.shape[-1] == self.q_width + self.latent_dim)
 
     def _native(self, qlat: torch.Tensor) -> bool:
         """The kernels of ``fl_refresh_attention`` take this projection [B, T, q | latent]."""
         params = (*self.kv_up.parameters(), self.global_mix_logit)
         rep = self.q_heads // self.kv_heads
-        return (free_rounding() and type(self) is LandmarkAttention and qlat.dtype == torch.bfloat16
+        return (free_rounding() and type(self) is LandmarkAttention and self._plain(qlat)
+                and qlat.dtype == torch.bfloat16
                 and self.head_dim == 64 and rep in (1, 2, 4, 8) and self.kv_heads <= 4096
                 and self.local_window % 64 == 0 and self.local_window <= 1 << 20
                 and self.landmark_chunk % 32 == 0 and self.latent_dim % 8 == 0
@@ -307,12 +317,59 @@ class LandmarkAttention(nn.Module):
         st["lat_sum"] = tail
         return y, st
 
+    def _exact(self, x: torch.Tensor, qlat: torch.Tensor) -> bool:
+        """The kernels of ``fl_rope_heads`` / ``fl_mix_heads`` take this projection [B, T, q | latent]. They
+        give the stock ops' bits, so they run under autocast too."""
+        params = (*self.kv_up.parameters(), self.global_mix_logit)
+        b, length, _ = qlat.shape
+        w = min(self.local_window, length)
+        return (type(self) is LandmarkAttention and self._plain(qlat) and x.dtype == qlat.dtype == torch.bfloat16
+                and self.head_dim == 64 and self.q_width == self.dim
+                and max(self.q_heads, self.kv_heads) <= 4096 and self.latent_dim % 8 == 0
+                and self.global_mix_logit.dtype in KERNEL_DTYPES and no_grad_needed(qlat, *params)
+                and eager(qlat, *params) and qlat.is_contiguous() and qlat.data_ptr() % 16 == 0
+                and 0 < b <= 65535 and 0 < length <= 1 << 26
+                and b * (length + w) * self.q_heads * 8 < 1 << 31 and b * (length + w) * self.q_heads * w < 1 << 39)
+
+    def _exact_attend(self, qlat: torch.Tensor, cos, sin):
+        """What out_proj reads, [B, T, dim]; the windows' keys (transposed) and values; the landmarks'."""
+        lib, stream = nat.load(), nat.stream_handle(qlat.device)
+        b, length, _ = qlat.shape
+        hq, hkv, hd, c = self.q_heads, self.kv_heads, self.head_dim, self.landmark_chunk
+        w = min(self.local_window, length)
+        groups, full = -(-length // w), length // c
+        latent = qlat[..., self.q_width:]
+        kv = self.kv_up(latent).contiguous()
+
+        def new(*shape):
+            return torch.empty(shape, device=qlat.device, dtype=qlat.dtype)
+
+        q, local = new(b, hq, length, hd), new(b * groups, hkv, hq // hkv * w, hd)
+        kt, v = new(b * groups, hkv, hd, w), new(b * groups, hkv, w, hd)
+        nat.check(lib.fl_rope_heads(
+            nat.ptr(qlat), qlat.stride(0), qlat.stride(1), nat.ptr(kv), kv.stride(0), kv.stride(1), nat.ptr(cos),
+            nat.ptr(sin), b, length, hq, hkv, w, nat.ptr(q), nat.ptr(local), nat.ptr(kt), nat.ptr(v), stream),
+            "fl_rope_heads")
+        p = masked_softmax(torch.matmul(local, kt).contiguous(), w, 0, None, 0, hd)
+        local = torch.matmul(p, v).contiguous()
+        land, attended = None, None
+        if full:
+            land = lk, lv = self._landmarks(latent, full, cos, sin)
+            attended = self._null_slot_attend(q, lk, lv).contiguous()
+        y = new(b, length, self.dim)
+        nat.check(lib.fl_mix_heads(nat.ptr(local), nat.ptr(attended), nat.ptr(self.global_mix_logit),
+                                   nat.dtype_code(self.global_mix_logit.dtype), b, length, hq, w, nat.ptr(y), stream),
+                  "fl_mix_heads")
+        return y, kt.view(b, groups, hkv, hd, w), v.view(b, groups, hkv, w, hd), land
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         b, length, _ = x.shape
         qlat = self.q_latent_proj(x)
         if self._native(qlat):
             cos, sin = rope_cos_sin(x.device, qlat.dtype, length, self.head_dim)
             return self.out_proj(self._native_attend(qlat, cos, sin)[0])
+        if self._exact(x, qlat):
+            return self.out_proj(self._exact_attend(qlat, *rope_cos_sin(x.device, x.dtype, length, self.head_dim))[0])
         qraw, latent = qlat.split((self.q_width, self.latent_dim), dim=-1)
         kraw, vraw = self.kv_up(latent).split(self.kv_heads * self.head_dim, dim=-1)
         q, k, v = self._heads(qraw, self.q_heads), self._heads(kraw, self.kv_heads), self._heads(vraw, self.kv_heads)
@@ -350,25 +407,32 @@ class LandmarkAttention(nn.Module):
         if x.dtype == qlat.dtype and b * self.kv_heads <= 65535 and max_len < 1 << 24 and self._native(qlat):
             y, st = self._native_attend(qlat, cos, sin, max_len)
             return self.out_proj(y), st
-        qraw, latent = qlat.split((self.q_width, self.latent_dim), dim=-1)
-        kraw, vraw = self.kv_up(latent).split(self.kv_heads * self.head_dim, dim=-1)
-        q, k, v = self._heads(qraw, self.q_heads), self._heads(kraw, self.kv_heads), self._heads(vraw, self.kv_heads)
-        cl, sl = cos[:, :, :length], sin[:, :, :length]
-        q, k = apply_rope(q, cl, sl), apply_rope(k, cl, sl)
-        y = self._local(q, k, v)
-        y = y + torch.sigmoid(self.global_mix_logit).to(y.dtype) * self._global(q, latent, cl, sl)
-        out = self.out_proj(y.transpose(1, 2).reshape(b, length, self.dim))
+        if self._exact(x, qlat):
+            y, kt, v, land = self._exact_attend(qlat, cos, sin)
+            out, latent = self.out_proj(y), qlat[..., self.q_width:]
+            kt, v = kt[:, -1], v[:, -1]  # the last window
+        else:
+            qraw, latent = qlat.split((self.q_width, self.latent_dim), dim=-1)
+            kraw, vraw = self.kv_up(latent).split(self.kv_heads * self.head_dim, dim=-1)
+            q, k, v = self._heads(qraw, self.q_heads), self._heads(kraw, self.kv_heads), self._heads(vraw, self.kv_heads)
+            cl, sl = cos[:, :, :length], sin[:, :, :length]
+            q, k = apply_rope(q, cl, sl), apply_rope(k, cl, sl)
+            y = self._local(q, k, v)
+            y = y + torch.sigmoid(self.global_mix_logit).to(y.dtype) * self._global(q, latent, cl, sl)
+            out = self.out_proj(y.transpose(1, 2).reshape(b, length, self.dim))
+            land = None
+            g0 = length // self.local_window * self.local_window
+            kt, v = k[:, :, g0:].transpose(-1, -2), v[:, :, g0:]
         st = self.new_state(b, max_len, x.device, x.dtype)
         self._rope_len = int(max_len)
-        w, c = self.local_window, self.landmark_chunk
-        g0 = (length // w) * w  # the next token opens a window at g0 or continues it
-        n = length - g0
+        c = self.landmark_chunk
+        n = length % self.local_window  # the next token opens a window or continues the last one
         if n:
-            st["kt"][..., :n] = k[:, :, g0:].transpose(-1, -2)
-            st["v"][:, :, :n] = v[:, :, g0:]
+            st["kt"][..., :n] = kt[..., :n]
+            st["v"][:, :, :n] = v[:, :, :n]
         full = length // c
         if full:
-            lk, lv = self._landmarks(latent, full, cos, sin)
+            lk, lv = self._landmarks(latent, full, cos, sin) if land is None else land
             st["lkt"][..., 1:1 + full] = lk.transpose(-1, -2)
             st["lv"][:, :, 1:1 + full] = lv
         st["lat_sum"] = latent[:, full * c:].float().sum(1)
@@ -380,7 +444,8 @@ class LandmarkAttention(nn.Module):
         b, h, hd, w, c = qlat.shape[0], self.kv_heads, self.head_dim, self.local_window, self.landmark_chunk
         state = tuple(st[k] for k in ("kt", "v", "lkt", "lv", "lat_sum"))
         mix = self.global_mix_logit
-        return (type(self) is LandmarkAttention and qlat.dtype == torch.bfloat16 and qlat.ndim == 2 and hd == 64
+        return (type(self) is LandmarkAttention and self._plain(qlat) and qlat.dtype == torch.bfloat16
+                and qlat.ndim == 2 and hd == 64
                 and c & (c - 1) == 0 and 0 < b <= 1 << 20 and max(w, c, self._rope_len) < 1 << 28
                 and self.q_heads <= 4096 and self.latent_dim <= 1 << 16 and mix.dtype in KERNEL_DTYPES
                 and no_grad_needed(qlat, mix, *self.kv_up.parameters()) and eager(qlat, pos, mix, *state)

@@ -415,6 +415,12 @@ int fl_field_params_backward(const float* radius_logit, const float* theta, int6
  *   mode 0 row % lq (causal), 1 *pos % period, 2 *pos / period;
  * fl_masked_softmax: out [rows, lk] bf16 = softmax of the scores fl_mask_scores forms, lk <= 1024; mode 3:
  *   limit (row % lq) / period;
+ * fl_rope_heads: a prompt's heads of 64 for the products, windows = ceil(T / window), window <= T, zeros past
+ *   T: rotated queries of x [B, T, q_heads * 64] (strides in elements, multiples of 8) to q [B, q_heads, T, 64]
+ *   and local [B, windows, q_heads, window, 64]; of kv [B, T, 2 * kv_heads * 64] the rotated keys to
+ *   kt [B, windows, kv_heads, 64, window] and the values to v [B, windows, kv_heads, window, 64];
+ * fl_mix_heads: out [B, T, heads * 64] = local (as above) + sigmoid(mix_logit[0]) * g [B, heads, T, 64], g
+ *   null for zeros;
  * fl_mix: out = y + sigmoid(mix_logit[0]) * g over n values;
  * and of the Mamba-2 blocks as they run under bf16 autocast (field_fusion_wiki100_mamba2_v25.py:73-91):
  * fl_conv_silu: out [B, L, channels] fp32 = silu(causal depthwise conv of width 4), x bf16 with strides;
@@ -433,6 +439,11 @@ int fl_mask_scores(const void* scores, int64_t rows, int64_t lk, int64_t lq, int
                    int64_t period, float scale, float* out, void* stream);
 int fl_masked_softmax(const void* scores, int64_t rows, int64_t lk, int64_t lq, int mode, const int64_t* pos,
                       int64_t period, float scale, void* out, void* stream);
+int fl_rope_heads(const void* x, int64_t x_stride_b, int64_t x_stride_t, const void* kv, int64_t kv_stride_b,
+                  int64_t kv_stride_t, const void* cos, const void* sin, int64_t B, int64_t T, int64_t q_heads,
+                  int64_t kv_heads, int64_t window, void* q, void* local, void* kt, void* v, void* stream);
+int fl_mix_heads(const void* local, const void* g, const void* mix_logit, int mix_dtype, int64_t B, int64_t T,
+                 int64_t heads, int64_t window, void* out, void* stream);
 int fl_conv_silu(const void* x, int64_t stride_b, int64_t stride_t, int64_t B, int64_t L, int64_t channels,
                  const void* w, const void* bias, int w_dtype, float* out, void* stream);
 int fl_decay_product(const void* cb, const float* acs, int64_t B, int64_t heads, int64_t n_chunks, int64_t s,

@@ -208,3 +208,19 @@ def test_landmark_scores_under_autocast_give_the_stock_bits(dev, T, window):
         stock = att(x).detach()  # gradients enabled: the stock ops
         with torch.no_grad():
             assert torch.equal(att(x), stock)
+
+
+@pytest.mark.parametrize("heads,kv,B,T,window", [(8, 2, 2, 20, 64), (4, 4, 3, 130, 64), (6, 3, 1, 77, 20),
+                                                 (8, 2, 2, 128, 64), (16, 4, 1, 1111, 512)])
+def test_prompt_state_under_autocast_gives_the_stock_bits(dev, heads, kv, B, T, window):
+    """Rotated, padded and transposed heads, no landmark yet, odd windows: output and decode state."""
+    print(f"[case] prompt heads={heads}/{kv} B={B} T={T} window={window}", flush=True)
+    att = _block(dev, heads, kv, window, 32, seed=T).attn
+    x = torch.randn(B, T, 64 * heads, device=dev, generator=torch.Generator(device=dev).manual_seed(T)).to(torch.bfloat16)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        stock, st_stock = att.prefill(x, T + 9)  # gradients enabled: the stock ops
+        with torch.no_grad():
+            y, st = att.prefill(x, T + 9)
+    assert torch.equal(y, stock)
+    for k in st:
+        assert torch.equal(st[k], st_stock[k]), k
