@@ -86,6 +86,8 @@ SIGNATURES = {
     "fl_mix_heads": (_int, [_vp, _vp, _vp, _int] + [_i64] * 4 + [_vp, _vp]),
     "fl_conv_silu": (_int, [_vp] + [_i64] * 5 + [_vp, _vp, _int, _vp, _vp]),
     "fl_decay_product": (_int, [_vp, _vp] + [_i64] * 4 + [_vp, _vp]),
+    "fl_ssd_operands": (_int, [_vp, _i64, _i64, _vp, _i64, _vp] + [_i64] * 6 + [_vp] * 3),
+    "fl_ssd_finish": (_int, [_vp] * 4 + [_i64, _i64, _vp, _vp, _i64, _i64] + [_i64] * 6 + [_vp, _vp]),
     "fl_state_update": (_int, [_vp] * 3 + [_i64] * 5 + [_vp] * 3),
     "fl_mix": (_int, [_vp, _vp, _vp, _int, _i64, _vp, _vp]),
     "fl_latent_mean": (_int, [_vp] + [_i64] * 6 + [_vp, _vp, _vp]),

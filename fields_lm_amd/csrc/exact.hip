@@ -364,6 +364,70 @@ __global__ __launch_bounds__(256) void fl_decay_product_kernel(const bf16_bits* 
   Vec<bf16_bits, 8>::store(out + (((bh * n_chunks + c) * s + i) * s + j0), o);
 }
 
+// The two operands autocast makes of x dt, each bf16 of fp32 products: xdt [B, H, chunks, s, P] and, times
+// w_end (the decay to the chunk's end), xw [B, H, chunks, P, s], zeros past L. A tile of 64 tokens by 64
+// dimensions goes through LDS, so that both orders are read and written in rows. Two products, two
+// reorderings and two conversions of the stock ops in fp32 (67 MB each way at 8,192 tokens) in one pass.
+__global__ __launch_bounds__(256) void fl_ssd_operands_kernel(const float* __restrict__ x, int64_t sb, int64_t st,
+                                                              const float* __restrict__ dt, int64_t dt_sb,
+                                                              const float* __restrict__ w_end, int H, int n_chunks,
+                                                              int s, int P, int64_t L, bf16_bits* __restrict__ xdt,
+                                                              bf16_bits* __restrict__ xw) {
+  __shared__ bf16_bits tile[64][66];
+  const int s_tiles = (s + 63) / 64, t0 = (int)(blockIdx.x % s_tiles) * 64, p0 = (int)(blockIdx.x / s_tiles) * 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = (int)(blockIdx.z % H);
+  const int64_t b = blockIdx.z / H, bhc = (int64_t)blockIdx.z * n_chunks + blockIdx.y;
+  const int64_t first = (int64_t)blockIdx.y * s + t0;  // the tile's first token
+  const bool has = p0 + lane < P;
+  for (int t = wave; t < 64 && t0 + t < s; t += 4) {
+    float v = 0.f;
+    if (has && first + t < L)
+      v = x[b * sb + (first + t) * st + (int64_t)h * P + p0 + lane] * dt[b * dt_sb + (first + t) * H + h];
+    if (has) xdt[(bhc * s + t0 + t) * P + p0 + lane] = (bf16_bits)bf16_bits_of(v);
+    const float w = v * w_end[bhc * s + t0 + t];
+    tile[lane][t] = (bf16_bits)bf16_bits_of(w);
+  }
+  __syncthreads();
+  if (t0 + lane < s)
+    for (int d = wave; d < 64 && p0 + d < P; d += 4) xw[(bhc * P + p0 + d) * s + t0 + lane] = tile[d][lane];
+}
+
+// What the gated norm takes the mean square of: ((y + y_off exp(acs)) + D x) silu(z), each operation rounded
+// in fp32, [B, L, H P] from y and y_off [B, H, chunks, s, P]: eight fp32 passes in one, bound by memory.
+__global__ __launch_bounds__(256) void fl_ssd_finish_kernel(const bf16_bits* __restrict__ y,
+                                                            const bf16_bits* __restrict__ y_off,
+                                                            const float* __restrict__ acs,
+                                                            const float* __restrict__ x, int64_t x_sb, int64_t x_st,
+                                                            const float* __restrict__ D,
+                                                            const bf16_bits* __restrict__ z, int64_t z_sb, int64_t z_st,
+                                                            uint32_t n, int H, int n_chunks, int s, int P, int L,
+                                                            float* __restrict__ out) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t width = (uint32_t)(H * P / 4), row = i / width, col = (i - row * width) * 4;
+  const uint32_t b = row / (uint32_t)L, t = row - b * (uint32_t)L, h = col / (uint32_t)P, p = col - h * (uint32_t)P;
+  const uint32_t c = t / (uint32_t)s;
+  const int64_t at = (((int64_t)b * H + h) * n_chunks + c) * s + (t - c * (uint32_t)s);
+  auto load4 = [](const bf16_bits* q, float* o) {
+    const u32x2 w = *reinterpret_cast<const u32x2*>(q);
+    o[0] = bf16_lo(w.x), o[1] = bf16_hi(w.x), o[2] = bf16_lo(w.y), o[3] = bf16_hi(w.y);
+  };
+  float a[4], off[4], g[4];
+  load4(y + at * P + p, a);
+  load4(y_off + at * P + p, off);
+  load4(z + (int64_t)b * z_sb + (int64_t)t * z_st + col, g);
+  const f32x4 xv = *reinterpret_cast<const f32x4*>(x + (int64_t)b * x_sb + (int64_t)t * x_st + col);
+  const float e = expf(acs[at]), d = D[h];
+  f32x4 o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float m = off[k] * e, u = a[k] + m, dx = d * xv[k], v = u + dx;
+    const float silu = g[k] / (1.0f + expf(-g[k]));
+    o[k] = v * silu;
+  }
+  *reinterpret_cast<f32x4*>(out + (int64_t)i * 4) = o;
+}
+
 // One token's state update, s = s * decay then s + xdt * b, each rounded, and the bf16 operand that
 // autocast makes of the state for its product with C: 500 MB of traffic in 168 MB at 64 x 32 heads.
 __global__ __launch_bounds__(256) void fl_state_update_kernel(const float* __restrict__ decay,
@@ -535,6 +599,38 @@ int fl_decay_product(const void* cb, const float* acs, int64_t B, int64_t heads,
   fl_decay_product_kernel<<<dim3((unsigned)cdiv(s * (s / 8), 256), (unsigned)n_chunks, (unsigned)(B * heads)), 256, 0,
                             static_cast<hipStream_t>(stream)>>>(static_cast<const bf16_bits*>(cb), acs, (int)heads,
                                                                 (int)n_chunks, (int)s, static_cast<bf16_bits*>(out));
+  return hip_status(hipGetLastError());
+}
+
+int fl_ssd_operands(const float* x, int64_t x_stride_b, int64_t x_stride_t, const float* dt, int64_t dt_stride_b,
+                    const float* w_end, int64_t B, int64_t heads, int64_t n_chunks, int64_t s, int64_t P, int64_t L,
+                    void* xdt, void* xw, void* stream) {
+  if (B <= 0 || heads <= 0 || B * heads > 65535 || n_chunks <= 0 || n_chunks > 65535 || s <= 0 || s > 4096 || P <= 0 ||
+      P > 4096 || L <= 0 || L > n_chunks * s || x_stride_t < heads * P || x_stride_b < 0 || dt_stride_b < 0 || !x ||
+      !dt || !w_end || !xdt || !xw)
+    return FL_ERR_INVALID_ARGUMENT;
+  fl_ssd_operands_kernel<<<dim3((unsigned)(cdiv(s, 64) * cdiv(P, 64)), (unsigned)n_chunks, (unsigned)(B * heads)), 256,
+                           0, static_cast<hipStream_t>(stream)>>>(
+      x, x_stride_b, x_stride_t, dt, dt_stride_b, w_end, (int)heads, (int)n_chunks, (int)s, (int)P, L,
+      static_cast<bf16_bits*>(xdt), static_cast<bf16_bits*>(xw));
+  return hip_status(hipGetLastError());
+}
+
+int fl_ssd_finish(const void* y, const void* y_off, const float* acs, const float* x, int64_t x_stride_b,
+                  int64_t x_stride_t, const float* D, const void* z, int64_t z_stride_b, int64_t z_stride_t, int64_t B,
+                  int64_t heads, int64_t n_chunks, int64_t s, int64_t P, int64_t L, float* out, void* stream) {
+  if (B <= 0 || heads <= 0 || B * heads > 65535 || n_chunks <= 0 || n_chunks > 65535 || s <= 0 || s > 4096 || P <= 0 ||
+      P > 4096 || P % 4 || L <= 0 || L > n_chunks * s || x_stride_t < heads * P || z_stride_t < heads * P ||
+      x_stride_b < 0 || z_stride_b < 0 || (x_stride_b | x_stride_t | z_stride_b | z_stride_t) % 4 || !y || !y_off ||
+      !acs || !x || !D || !z || !out || !aligned(y, 8) || !aligned(y_off, 8) || !aligned(x, 16) || !aligned(z, 8) ||
+      !aligned(out, 16))
+    return FL_ERR_INVALID_ARGUMENT;
+  if (L > (((int64_t)1 << 32) - 256) / (heads * P / 4) / B) return FL_ERR_INVALID_ARGUMENT;
+  const int64_t n = B * L * (heads * P / 4);
+  fl_ssd_finish_kernel<<<(unsigned)cdiv(n, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+      static_cast<const bf16_bits*>(y), static_cast<const bf16_bits*>(y_off), acs, x, x_stride_b, x_stride_t, D,
+      static_cast<const bf16_bits*>(z), z_stride_b, z_stride_t, (uint32_t)n, (int)heads, (int)n_chunks, (int)s, (int)P,
+      (int)L, out);
   return hip_status(hipGetLastError());
 }
 

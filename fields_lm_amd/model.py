@@ -611,7 +611,9 @@ class GatedRMSNorm(nn.Module):
         self.eps = float(eps)
 
     def forward(self, x: torch.Tensor, z: torch.Tensor) -> torch.Tensor:
-        y = x.float() * F.silu(z.float())
+        return self.scaled(x.float() * F.silu(z.float()))
+
+    def scaled(self, y: torch.Tensor) -> torch.Tensor:
         y = y * torch.rsqrt(y.square().mean(-1, keepdim=True) + self.eps)
         return y * self.weight.float()
 
@@ -625,23 +627,24 @@ def _autocast_operands(product: torch.Tensor, *others: torch.Tensor) -> bool:
             and eager(product, *others) and all(t.dtype == torch.float32 for t in others))
 
 
-def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None):
+def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None, *, finish=None):
     """State-space-duality scan of Mamba-2 in fp32 (the chunked algorithm of Dao & Gu, 2024):
 
         h_t = exp(dt_t A) h_{t-1} + dt_t x_t B_t^T,   y_t = h_t C_t       (per head)
 
     x [b,l,h,p], dt [b,l,h] (after softplus), A [h] (negative), Bm/Cm [b,l,n] (one group).
     Within a chunk the output is a masked (C B^T ∘ decay) product; chunk states are carried by
-    a short sequential loop. Returns (y [b,l,h,p], final state [b,h,p,n]).
+    a short sequential loop. Returns (y [b,l,h,p], final state [b,h,p,n]); ``finish`` may make something
+    else of (the product within chunks, C h from before them, log-decay sums), or None for y.
     """
     b, l, h, p = x.shape
     n = Bm.shape[-1]
     pad = (-l) % chunk
+    given = x, dt  # before padding
     if pad:  # dt = 0 on padded steps: decay 1, input 0 (identity)
-        x, dt, Bm, Cm = (F.pad(t, (0, 0) * (t.dim() - 2) + (0, pad)) for t in (x, dt, Bm, Cm))
-    L = x.shape[1]
+        dt, Bm, Cm = (F.pad(t, (0, 0) * (t.dim() - 2) + (0, pad)) for t in (dt, Bm, Cm))
+    L = dt.shape[1]
     c = L // chunk
-    xdt = (x.float() * dt.float()[..., None]).view(b, c, chunk, h, p).permute(0, 3, 1, 2, 4).contiguous()
     adt = (dt.float() * A.float()).view(b, c, chunk, h).permute(0, 3, 1, 2)          # [b,h,c,s]
     acs = torch.cumsum(adt, -1)
     Bc = Bm.float().view(b, c, chunk, n)
@@ -658,10 +661,22 @@ def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None):
         seg = acs[..., :, None] - acs[..., None, :]                                    # [b,h,c,s,s]
         causal = torch.ones(chunk, chunk, device=x.device, dtype=torch.bool).tril()
         weights = cb[:, None] * torch.exp(seg.masked_fill(~causal, float("-inf")))
+    w_end = torch.exp(acs[..., -1:] - acs)                                              # [b,h,c,s]
+    if (_autocast_operands(cb, w_end, *given) and b * h <= 65535 and 0 < c <= 65535 and chunk <= 4096
+            and 0 < p <= 4096 and l > 0 and x.stride(-1) == 1 and x.stride(-2) == p and x.stride(0) >= 0
+            and x.stride(1) >= h * p and dt.is_contiguous() and w_end.is_contiguous()):
+        xdt = torch.empty((b, h, c, chunk, p), device=x.device, dtype=cb.dtype)
+        xw = torch.empty((b, h, c, p, chunk), device=x.device, dtype=cb.dtype)
+        nat.check(nat.load().fl_ssd_operands(nat.ptr(x), x.stride(0), x.stride(1), nat.ptr(dt), dt.stride(0),
+                                             nat.ptr(w_end), b, h, c, chunk, p, l, nat.ptr(xdt), nat.ptr(xw),
+                                             nat.stream_handle(x.device)), "fl_ssd_operands")
+    else:
+        x = F.pad(x, (0, 0, 0, 0, 0, pad)) if pad else x
+        xdt = (x.float() * dt.float()[..., None]).view(b, c, chunk, h, p).permute(0, 3, 1, 2, 4).contiguous()
+        xw = (xdt * w_end[..., None]).transpose(-1, -2).contiguous()
     y = torch.matmul(weights, xdt)                                                      # [b,h,c,s,p]
     # chunk states from 0: sum_j exp(acs_end - acs_j) xdt_j B_j^T
-    w_end = torch.exp(acs[..., -1:] - acs)                                              # [b,h,c,s]
-    states = torch.matmul((xdt * w_end[..., None]).transpose(-1, -2).contiguous(), Bc[:, None])  # [b,h,c,p,n]
+    states = torch.matmul(xw, Bc[:, None])                                              # [b,h,c,p,n]
     chunk_decay = torch.exp(acs[..., -1])                                               # [b,h,c]
     s = (initial_state.float() if initial_state is not None
          else torch.zeros(b, h, p, n, device=x.device, dtype=torch.float32))
@@ -672,6 +687,9 @@ def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None):
     carry = torch.stack(carries, 2)                                                     # [b,h,c,p,n]
     # inter-chunk: y_i += exp(acs_i) C_i carry
     y_off = torch.matmul(Cc[:, None], carry.transpose(-1, -2).contiguous())             # [b,h,c,s,p]
+    done = finish(y, y_off, acs) if finish is not None else None
+    if done is not None:
+        return done, s
     y = y + y_off * torch.exp(acs)[..., None]
     y = y.permute(0, 2, 3, 1, 4).reshape(b, L, h, p)[:, :l]
     return y, s
@@ -769,10 +787,35 @@ class Mamba2Mixer(nn.Module):
         x, bm, cm, dt = self._ssm_in(self._conv_silu(xbc_raw), dt)
         A = -torch.exp(self.A_log.float())
         xh = x.reshape(b, l, self.nheads, self.headdim)
-        y, state = ssd_chunked(xh, dt, A, bm, cm, self.chunk_size)
-        y = y + self.D.float()[:, None] * xh
-        out = self.out_proj(self.norm(y.reshape(b, l, self.d_inner), z).to(u.dtype))
+        y, state = ssd_chunked(xh, dt, A, bm, cm, self.chunk_size,
+                               finish=lambda y, y_off, acs: self._finish(y, y_off, acs, xh, z))
+        if y.ndim == 3:
+            y = self.norm.scaled(y)
+        else:
+            y = y + self.D.float()[:, None] * xh
+            y = self.norm(y.reshape(b, l, self.d_inner), z)
+        out = self.out_proj(y.to(u.dtype))
         return (out, self._new_state(xbc_raw, state)) if return_state else out
+
+    def _finish(self, y, y_off, acs, xh, z) -> Optional[torch.Tensor]:
+        """(y + y_off exp(acs) + D x) silu(z), fp32 [b, l, d_inner], with the stock ops' bits."""
+        b, l, h, p = xh.shape
+        c, s = y.shape[2:4]
+        if not (plain_call(self.norm, GatedRMSNorm) and _autocast_operands(y, acs, xh)
+                and no_grad_needed(y_off, z, self.D) and eager(y_off, z, self.D) and z.dtype == y_off.dtype == y.dtype
+                and y.is_contiguous() and y_off.is_contiguous() and y_off.shape == y.shape and acs.is_contiguous()
+                and p % 4 == 0 and p <= 4096 and s <= 4096 and b * h <= 65535 and 0 < c <= 65535
+                and xh.stride(-1) == z.stride(-1) == 1 and xh.stride(-2) == p and xh.stride(1) >= h * p
+                and z.stride(1) >= h * p and xh.data_ptr() % 16 == 0 and z.data_ptr() % 8 == 0
+                and all(n >= 0 and n % 4 == 0 for t in (xh, z) for n in t.stride()[:2])
+                and b * l * (h * p // 4) <= (1 << 32) - 256):
+            return None
+        out = torch.empty((b, l, self.d_inner), device=y.device, dtype=torch.float32)
+        d = self.D.detach().float().contiguous()
+        nat.check(nat.load().fl_ssd_finish(
+            nat.ptr(y), nat.ptr(y_off), nat.ptr(acs), nat.ptr(xh), xh.stride(0), xh.stride(1), nat.ptr(d), nat.ptr(z),
+            z.stride(0), z.stride(1), b, h, c, s, p, l, nat.ptr(out), nat.stream_handle(y.device)), "fl_ssd_finish")
+        return out
 
     def _conv_silu(self, xbc_raw: torch.Tensor) -> torch.Tensor:
         """silu of the causal depthwise convolution, fp32 [b, l, channels]: d_conv shifted multiply-adds in

@@ -426,6 +426,10 @@ int fl_field_params_backward(const float* radius_logit, const float* theta, int6
  * fl_conv_silu: out [B, L, channels] fp32 = silu(causal depthwise conv of width 4), x bf16 with strides;
  * fl_decay_product: out [B, heads, n_chunks, s, s] bf16 = cb [B, n_chunks, s, s] exp(acs_i - acs_j) for
  *   j <= i and cb * 0 above, acs [B, heads, n_chunks, s] fp32, s a multiple of 8;
+ * fl_ssd_operands: bf16 xdt [B, heads, n_chunks, s, P] = x dt and xw [B, heads, n_chunks, P, s] = x dt w_end,
+ *   zeros past L; x [B, L, heads * P], dt [B, >= L, heads] with strides in elements, w_end [B, heads, n_chunks, s];
+ * fl_ssd_finish: out [B, L, heads * P] fp32 = ((y + y_off exp(acs)) + D x) silu(z), y, y_off bf16
+ *   [B, heads, n_chunks, s, P], x fp32 and z bf16 with strides in elements, multiples of 4; P a multiple of 4;
  * fl_state_update: ssm [B, heads, P, N] = ssm decay [B, heads] + xdt [B, heads, P] bm [B, N] in place
  *   (rows of bm bm_stride apart), and ssm16 its bf16 copy; N a multiple of 4.
  */
@@ -448,6 +452,12 @@ int fl_conv_silu(const void* x, int64_t stride_b, int64_t stride_t, int64_t B, i
                  const void* w, const void* bias, int w_dtype, float* out, void* stream);
 int fl_decay_product(const void* cb, const float* acs, int64_t B, int64_t heads, int64_t n_chunks, int64_t s,
                      void* out, void* stream);
+int fl_ssd_operands(const float* x, int64_t x_stride_b, int64_t x_stride_t, const float* dt, int64_t dt_stride_b,
+                    const float* w_end, int64_t B, int64_t heads, int64_t n_chunks, int64_t s, int64_t P, int64_t L,
+                    void* xdt, void* xw, void* stream);
+int fl_ssd_finish(const void* y, const void* y_off, const float* acs, const float* x, int64_t x_stride_b,
+                  int64_t x_stride_t, const float* D, const void* z, int64_t z_stride_b, int64_t z_stride_t, int64_t B,
+                  int64_t heads, int64_t n_chunks, int64_t s, int64_t P, int64_t L, float* out, void* stream);
 int fl_state_update(const float* decay, const float* xdt, const float* bm, int64_t bm_stride, int64_t B, int64_t heads,
                     int64_t P, int64_t N, float* ssm, void* ssm16, void* stream);
 int fl_mix(const void* y, const void* g, const void* mix_logit, int mix_dtype, int64_t n, void* out, void* stream);

@@ -158,3 +158,20 @@ def test_mamba_under_autocast_gives_the_stock_bits(dev, dim, B, L, weights):
             for i in range(3):  # a transposed state takes the stock ops
                 a, b = m.step(u[:, L + i], st), m.step(u[:, L + i], other)
                 assert torch.equal(a, b) and torch.equal(st["ssm"], other["ssm"]) and torch.equal(st["conv"], other["conv"])
+
+
+@pytest.mark.parametrize("headdim,chunk,B,L", [(24, 24, 2, 50), (32, 72, 1, 72), (96, 136, 2, 300), (6, 16, 1, 33),
+                                               (48, 20, 1, 45)])
+def test_mamba_under_autocast_odd_geometry_gives_the_stock_bits(dev, headdim, chunk, B, L):
+    """Tiles of the products' operands with remainders in tokens and dimensions, and what they do not take."""
+    print(f"[case] mamba operands headdim={headdim} chunk={chunk} B={B} L={L}", flush=True)
+    torch.manual_seed(L)
+    m = M.Mamba2Mixer(headdim * 2, d_state=16, d_conv=4, expand=2, headdim=headdim, ngroups=1, chunk_size=chunk).to(dev)
+    u = torch.randn(B, L, headdim * 2, device=dev, generator=torch.Generator(device=dev).manual_seed(L))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        stock, st_stock = m(u, return_state=True)
+        with torch.no_grad():
+            y, st = m(u, return_state=True)
+    assert torch.equal(y, stock.detach())
+    for k in st:
+        assert torch.equal(st[k], st_stock[k].detach()), k
