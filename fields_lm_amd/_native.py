@@ -84,6 +84,7 @@ SIGNATURES = {
     "fl_masked_softmax": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _i64, ctypes.c_float, _vp, _vp]),
     "fl_rope_heads": (_int, [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp] + [_i64] * 5 + [_vp] * 5),
     "fl_mix_heads": (_int, [_vp, _vp, _vp, _int] + [_i64] * 4 + [_vp, _vp]),
+    "fl_gate_add": (_int, [_vp, _vp, _vp, _i64, _vp, _vp]),
     "fl_conv_silu": (_int, [_vp] + [_i64] * 5 + [_vp, _vp, _int, _vp, _vp]),
     "fl_decay_product": (_int, [_vp, _vp] + [_i64] * 4 + [_vp, _vp]),
     "fl_ssd_operands": (_int, [_vp, _i64, _i64, _vp, _i64, _vp] + [_i64] * 6 + [_vp] * 3),

@@ -197,6 +197,27 @@ __global__ __launch_bounds__(256) void fl_mix_kernel(const bf16_bits* __restrict
   out[i] = (bf16_bits)bf16_bits_of(bf(y + i) + t);
 }
 
+// out = x + round(sigmoid(gate)) * a, rounded after each operation: three passes of the stock ops in one,
+// bound by memory in a prompt and by the launch in a step. A multiple of 8 values, 16 bytes each.
+__global__ __launch_bounds__(256) void fl_gate_add_kernel(const bf16_bits* __restrict__ x,
+                                                          const bf16_bits* __restrict__ gate,
+                                                          const bf16_bits* __restrict__ a, uint32_t n8,
+                                                          bf16_bits* __restrict__ out) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  const int64_t at = (int64_t)i * 8;
+  float v[8], g[8], w[8];
+  Vec<bf16_bits, 8>::load(x + at, v);
+  Vec<bf16_bits, 8>::load(gate + at, g);
+  Vec<bf16_bits, 8>::load(a + at, w);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float s = bf16_round(1.0f / (1.0f + expf(-g[e])));
+    v[e] += bf16_round(s * w[e]);
+  }
+  Vec<bf16_bits, 8>::store(out + at, v);
+}
+
 // ---- a prompt's heads ----
 
 // 8 values from element o of each half of a head, rotated (8 pairs); zeros past the prompt
@@ -576,6 +597,16 @@ int fl_mix_heads(const void* local, const void* g, const void* mix_logit, int mi
   fl_mix_heads_kernel<<<(unsigned)cdiv(n, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const bf16_bits*>(local), static_cast<const bf16_bits*>(g), mix_logit, mix_dtype == FL_DTYPE_BF16,
       (uint32_t)n, (int)T, (int)heads, (int)window, (int)cdiv(T, window), static_cast<bf16_bits*>(out));
+  return hip_status(hipGetLastError());
+}
+
+int fl_gate_add(const void* x, const void* gate, const void* a, int64_t n, void* out, void* stream) {
+  if (n <= 0 || n % 8 || n / 8 > ((int64_t)1 << 32) - 256 || !x || !gate || !a || !out || !aligned(x, 16) ||
+      !aligned(gate, 16) || !aligned(a, 16) || !aligned(out, 16))
+    return FL_ERR_INVALID_ARGUMENT;
+  fl_gate_add_kernel<<<(unsigned)cdiv(n / 8, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+      static_cast<const bf16_bits*>(x), static_cast<const bf16_bits*>(gate), static_cast<const bf16_bits*>(a),
+      (uint32_t)(n / 8), static_cast<bf16_bits*>(out));
   return hip_status(hipGetLastError());
 }
 

@@ -98,7 +98,10 @@ class GateUpSwiGLU(nn.Module):
         self.down = nn.Linear(hidden, dim, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gate, up = self.gate_up(x).chunk(2, dim=-1)
+        h = self.gate_up(x)
+        if (h.dtype == torch.bfloat16 and no_grad_needed(h) and eager(h) and h.numel() > 0 and h.shape[-1] % 2 == 0):
+            return self.down(swiglu(h))  # the stock ops' bits
+        gate, up = h.chunk(2, dim=-1)
         return self.down(F.silu(gate) * up)
 
 
@@ -579,8 +582,23 @@ class RefreshBlock(nn.Module):
                 and not torch.is_grad_enabled() and eager(x, a, n2.weight) and x.numel() > 0):
             x, h = gate_residual_norm(x, a, self.residual_gate(z), n2.weight, n2.eps)
             return _linear_residual(x, ff.down, swiglu(ff.gate_up(h)))
-        x = x + self._gate(z) * a
+        x = self._gated(x, z, a)
         return x + ff(n2(x))
+
+    def _gated(self, x: torch.Tensor, z: torch.Tensor, a: torch.Tensor) -> torch.Tensor:
+        """x + gate * a; ``fl_gate_add`` keeps the stock ops' bits."""
+        if self.light_gate or type(self) is not RefreshBlock:
+            return x + self._gate(z) * a
+        g = self.residual_gate(z)
+        if (x.dtype == g.dtype == a.dtype == torch.bfloat16 and x.shape == g.shape == a.shape
+                and no_grad_needed(x, g, a) and eager(x, g, a) and x.is_contiguous() and g.is_contiguous()
+                and a.is_contiguous() and 0 < x.numel() < 1 << 34 and x.numel() % 8 == 0
+                and (x.data_ptr() | g.data_ptr() | a.data_ptr()) % 16 == 0):
+            out = torch.empty_like(x)
+            nat.check(nat.load().fl_gate_add(nat.ptr(x), nat.ptr(g), nat.ptr(a), x.numel(), nat.ptr(out),
+                                             nat.stream_handle(x.device)), "fl_gate_add")
+            return out
+        return x + torch.sigmoid(g) * a
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         z = self.norm1(x)
@@ -593,7 +611,7 @@ class RefreshBlock(nn.Module):
 
     def step(self, x_t: torch.Tensor, pos: torch.Tensor, st) -> torch.Tensor:
         z = self.norm1(x_t)
-        x_t = x_t + self._gate(z) * self.attn.step(z, pos, st)
+        x_t = self._gated(x_t, z, self.attn.step(z, pos, st))
         return x_t + self.ff(self.norm2(x_t))
 
 

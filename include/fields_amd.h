@@ -421,6 +421,7 @@ int fl_field_params_backward(const float* radius_logit, const float* theta, int6
  *   kt [B, windows, kv_heads, 64, window] and the values to v [B, windows, kv_heads, window, 64];
  * fl_mix_heads: out [B, T, heads * 64] = local (as above) + sigmoid(mix_logit[0]) * g [B, heads, T, 64], g
  *   null for zeros;
+ * fl_gate_add: out = x + sigmoid(gate) * a over n values, n a multiple of 8;
  * fl_mix: out = y + sigmoid(mix_logit[0]) * g over n values;
  * and of the Mamba-2 blocks as they run under bf16 autocast (field_fusion_wiki100_mamba2_v25.py:73-91):
  * fl_conv_silu: out [B, L, channels] fp32 = silu(causal depthwise conv of width 4), x bf16 with strides;
@@ -448,6 +449,7 @@ int fl_rope_heads(const void* x, int64_t x_stride_b, int64_t x_stride_t, const v
                   int64_t kv_heads, int64_t window, void* q, void* local, void* kt, void* v, void* stream);
 int fl_mix_heads(const void* local, const void* g, const void* mix_logit, int mix_dtype, int64_t B, int64_t T,
                  int64_t heads, int64_t window, void* out, void* stream);
+int fl_gate_add(const void* x, const void* gate, const void* a, int64_t n, void* out, void* stream);
 int fl_conv_silu(const void* x, int64_t stride_b, int64_t stride_t, int64_t B, int64_t L, int64_t channels,
                  const void* w, const void* bias, int w_dtype, float* out, void* stream);
 int fl_decay_product(const void* cb, const float* acs, int64_t B, int64_t heads, int64_t n_chunks, int64_t s,

@@ -224,3 +224,23 @@ def test_prompt_state_under_autocast_gives_the_stock_bits(dev, heads, kv, B, T, 
     assert torch.equal(y, stock)
     for k in st:
         assert torch.equal(st[k], st_stock[k]), k
+
+
+@pytest.mark.parametrize("heads,ff,B,T", [(8, 96, 2, 70), (4, 44, 1, 33), (1, 8, 3, 1)])
+def test_block_under_autocast_gives_the_stock_bits(dev, heads, ff, B, T):
+    """The gated residual and the feed-forward's activation, rows that take 16 bytes and rows that do not."""
+    print(f"[case] refresh block heads={heads} ff={ff} B={B} T={T}", flush=True)
+    torch.manual_seed(T)
+    blk = M.RefreshBlock(64 * heads, heads, 1, 64, 64, 32, ff).to(dev)
+    with torch.no_grad():
+        blk.residual_gate.weight.normal_(0, 2.0)  # sigmoids over their whole range
+        blk.ff.gate_up.weight.mul_(20.0)
+    blk = M.cast_for_inference(blk).eval()
+    x = torch.randn(B, T, 64 * heads, device=dev, generator=torch.Generator(device=dev).manual_seed(T)).to(torch.bfloat16)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        stock, st_stock = blk.prefill(x, T + 9)  # gradients enabled: the stock ops
+        step_stock = blk.step(x[:, 0], torch.tensor(T, device=dev), {k: v.detach().clone() for k, v in st_stock.items()})
+        with torch.no_grad():
+            y, st = blk.prefill(x, T + 9)
+            step = blk.step(x[:, 0], torch.tensor(T, device=dev), st)
+    assert torch.equal(y, stock) and torch.equal(step, step_stock)
