@@ -670,7 +670,7 @@ def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None, *, finish=None
     # intra-chunk: y_i = sum_{j<=i} (C_i.B_j) exp(acs_i - acs_j) xdt_j
     cb = torch.matmul(Cc, Bc.transpose(-1, -2).contiguous())                            # [b,c,s,s]
     if _autocast_operands(cb, acs) and chunk % 8 == 0 and chunk <= 4096 and b * h <= 65535 and 0 < c <= 65535 \
-            and cb.is_contiguous() and cb.data_ptr() % 16 == 0:
+            and cb.is_contiguous() and (cb.data_ptr() | acs.data_ptr()) % 16 == 0:
         acs = acs.contiguous()
         weights = torch.empty((b, h, c, chunk, chunk), device=x.device, dtype=cb.dtype)
         nat.check(nat.load().fl_decay_product(nat.ptr(cb), nat.ptr(acs), b, h, c, chunk, nat.ptr(weights),
