@@ -10,18 +10,15 @@ namespace {
 
 using namespace fl;
 
-// sigmoid and silu of a loaded T. Of a bf16 value the sigmoid is one v_exp_f32 and one v_rcp_f32:
-// compared over all 65,536 inputs, its bf16 rounding is the library form's except at -87.5, -88 and
-// -88.5, where that is a denormal (below 1.1e-38) and this is 0. The plain form of silu would miss one
-// more (5.9375), so it takes the residual step. fp32 keeps the library exponential and division.
+// sigmoid and silu of a loaded T: of a bf16 value the forms of fl_common.h, whose bf16 roundings are the
+// library forms' for every input (a plain quotient of silu would miss 5.9375, so it takes the residual
+// step); fp32 keeps the library exponential and division.
 template <typename T>
 __device__ __forceinline__ float sigmoid(float x);
 template <>
 __device__ __forceinline__ float sigmoid<float>(float x) { return 1.0f / (1.0f + expf(-x)); }
 template <>
-__device__ __forceinline__ float sigmoid<bf16_bits>(float x) {
-  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -kLog2e));
-}
+__device__ __forceinline__ float sigmoid<bf16_bits>(float x) { return sigmoid_bf16(x); }
 template <typename T>
 __device__ __forceinline__ float silu(float x);
 template <>

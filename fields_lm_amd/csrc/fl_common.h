@@ -118,22 +118,34 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __uint_as_float(b.x) + __uint_as_float(b.y);
 }
 
+// 1 / (1 + e), subnormal results included: v_rcp_f32 gives 0 for those, so it takes a quarter of the
+// divisor, and the scale back is exact up to the subnormal's own rounding.
+__device__ __forceinline__ float rcp_one_plus(float e) {
+  return __builtin_amdgcn_rcpf(fmaf(e, 0.25f, 0.25f)) * 0.25f;
+}
+
+// 1 / (1 + e^-x) of a bf16 x: one v_exp_f32 and one v_rcp_f32, whose bf16 rounding is the library form's for
+// all 65,536 inputs.
+__device__ __forceinline__ float sigmoid_bf16(float x) {
+  return rcp_one_plus(__builtin_amdgcn_exp2f(x * -kLog2e));
+}
+
 // x / (1 + e^-x) to about an ulp: v_exp_f32 of the rounded product x log2(e) with the product's
-// rounding error put back (first order), and one residual step on v_rcp_f32's quotient. The
-// exponent is held within +-88, where e^-x is finite (its reciprocal is 0 there). Where the residual
-// is NaN (an infinite x) the plain quotient stands: inf, and NaN for -inf, as in the stock op. For
-// every bf16 x the result rounds to the stock op's bf16 value, but for 0 below -87.4, where that is
-// under 1e-36.
+// rounding error put back (first order), and one residual step on the reciprocal's quotient. The
+// exponent is held within +-88.7, where e^-x is finite; below, the result is -0 (NaN for -inf). Where the
+// residual is 0 or NaN (an infinite x) the plain quotient stands. For every bf16 x the result rounds to
+// the stock op's bf16 value.
 __device__ __forceinline__ float silu_precise(float x) {
   constexpr float kL = -kLog2e, kLlo = -1.9259629911266175e-8f;  // -log2(e) = kL + kLlo
-  const float xc = __builtin_amdgcn_fmed3f(x, -88.0f, 88.0f);
+  const float xc = __builtin_amdgcn_fmed3f(x, -88.7f, 88.7f);
   const float hi = xc * kL;
   const float lo = fmaf(xc, kLlo, fmaf(xc, kL, -hi));
   const float e0 = __builtin_amdgcn_exp2f(hi);
   const float corr = fmaf(e0, lo * 0.6931471805599453f, e0);
-  const float d = 1.0f + corr, r = __builtin_amdgcn_rcpf(d), q = x * r;
+  const float d = 1.0f + corr, r = rcp_one_plus(corr), q = x * r;
   const float res = fmaf(-q, d, x);
-  return res == res ? fmaf(res, r, q) : q;
+  const float y = __builtin_fabsf(res) > 0.0f ? fmaf(res, r, q) : q;
+  return x < -88.7f ? x * 0.0f : y;
 }
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -162,7 +162,7 @@ __global__ __launch_bounds__(W * 64, W / 4) void fl_linear_rows_kernel(LinearArg
       }
       if constexpr (EPI == kGatedResidual) {
         const float g = load_as<bf16_bits>(a.gate + (int64_t)m * a.gate_stride + col);
-        const float sg = bf16_round(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -kLog2e)));
+        const float sg = bf16_round(sigmoid_bf16(g));
         o = load_as<bf16_bits>(a.res + at) + bf16_round(bf16_round(o) * sg);
       } else if constexpr (EPI == kNormSwiglu) {
         o = bf16_round(silu_precise(bf16_round(o * scale))) * bf16_round(v[1][e] * scale);

@@ -23,9 +23,7 @@ __device__ __forceinline__ float sigmoid(float x);
 template <>
 __device__ __forceinline__ float sigmoid<float>(float x) { return 1.0f / (1.0f + expf(-x)); }
 template <>
-__device__ __forceinline__ float sigmoid<bf16_bits>(float x) {
-  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -kLog2e));
-}
+__device__ __forceinline__ float sigmoid<bf16_bits>(float x) { return sigmoid_bf16(x); }
 
 // out = (x rsqrt(mean x^2 + eps)) w; GATED: x_new = x + round(out_in * round(sigmoid(g))) first (in the
 // products' type G) and its norm. rstd is kept for the backward.
