@@ -569,11 +569,12 @@ class IndependentVacancyField(nn.Module):
 
     def _scan_params(self) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         """(tr, ti, gamma, read_norm weight), all fp32: what the fused scan and step read. One
-        launch where :meth:`_native_params` holds, a bf16 norm weight widened in the same one."""
-        w = self.read_norm.weight.detach()
+        launch where :meth:`_native_params` holds, a bf16 norm weight widened in the same one; the stock
+        ops otherwise, so that a forward-mode tangent reaches the scan, which refuses it."""
+        w = self.read_norm.weight
         if not self._native_params():
             return (*self.transition(), w.float().contiguous())
-        lib, c, p = nat.load(), self.radius_logit.numel(), self.radius_logit
+        lib, c, p, w = nat.load(), self.radius_logit.numel(), self.radius_logit, w.detach()
         widen = w.dtype == torch.bfloat16 and w.device == p.device and w.is_contiguous()
         n_w = w.numel() if widen else 0
         buf = torch.empty(3 * c + n_w, device=p.device, dtype=torch.float32)
@@ -687,7 +688,8 @@ class IndependentVacancyField(nn.Module):
     def decode_params(self) -> Tuple[torch.Tensor, ...]:
         """(tr, ti, gamma, read_norm weight in fp32): what :meth:`step` reads, cached once per
         decode loop."""
-        return self._scan_params()
+        *params, weight = self._scan_params()
+        return (*params, weight.detach())
 
     def step(self, x_t: torch.Tensor, state: torch.Tensor,
              params: Optional[Tuple[torch.Tensor, ...]] = None) -> torch.Tensor:

@@ -72,3 +72,24 @@ def test_transition_params_match_oracle():
     torch.testing.assert_close(ti, eti, rtol=0, atol=0)
     torch.testing.assert_close(gamma, egm, rtol=0, atol=0)
     assert float(gamma.min()) >= 0.01 - 1e-9 and float(tr.abs().max()) <= 0.99995
+
+
+def test_forward_mode_through_the_fused_norm_is_refused(monkeypatch):
+    """The fused scan has no forward-mode derivative: a dual read_norm.weight raises, it does not lose its
+    tangent (the scan itself replaced by its shape: only the routing is under test)."""
+    import torch.autograd.forward_ad as fwad
+
+    from fields_lm_amd import field
+
+    monkeypatch.setattr(field, "field_scan_norm", lambda raw, tr, ti, gamma, weight, eps, **kw:
+                        torch.ones(*raw.shape[:2], 4 * tr.numel()) * weight.detach())
+    m = field.IndependentVacancyField(16, "triton", 8, 8, 16)
+    x = torch.randn(1, 3, 16)
+    w = m.read_norm.weight.detach()
+    del m.read_norm.weight
+    with torch.no_grad(), fwad.dual_level():
+        m.read_norm.weight = fwad.make_dual(w, torch.ones_like(w))
+        with pytest.raises(NotImplementedError):
+            m.normed_read(x)
+        m.read_norm.weight = w
+        assert m.normed_read(x).shape == (1, 3, 32)
