@@ -720,10 +720,11 @@ class IndependentVacancyField(nn.Module):
 def _linear_residual(x: torch.Tensor, layer: nn.Module, h: torch.Tensor) -> torch.Tensor:
     """``x + layer(h)`` for a contiguous ``x`` that the caller owns. A plain bias-free layer of x's
     dtype accumulates onto x inside its GEMM (one rounding instead of two, and no add launch); any
-    other layer is called as it is."""
+    other layer is called as it is, also where something transforms its weight (vmap cannot batch an
+    in-place sum)."""
     if plain_linear(layer) and layer.bias is None and not torch.is_grad_enabled() \
             and x.dtype == h.dtype == layer.weight.dtype and free_rounding() \
-            and layer.weight.shape == (x.shape[-1], h.shape[-1]):
+            and layer.weight.shape == (x.shape[-1], h.shape[-1]) and eager(x, h, layer.weight):
         x.view(-1, x.shape[-1]).addmm_(h.view(-1, h.shape[-1]), layer.weight.t())
         return x
     return x + layer(h)

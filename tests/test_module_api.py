@@ -93,3 +93,32 @@ def test_forward_mode_through_the_fused_norm_is_refused(monkeypatch):
             m.normed_read(x)
         m.read_norm.weight = w
         assert m.normed_read(x).shape == (1, 3, 32)
+
+
+def _host_eager(*tensors):
+    """``eager`` without its device check, so that a route's other conditions decide on the CPU."""
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter)
+               and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
+
+
+class _Call(torch.nn.Module):
+    """A module's method as a forward, for functional_call."""
+
+    def __init__(self, inner, fn):
+        super().__init__()
+        self.inner, self.fn = inner, fn
+
+    def forward(self, *args):
+        return self.fn(self.inner, *args)
+
+
+def test_vmap_over_the_output_layer_of_a_residual(monkeypatch):
+    """Only the layer's weight batched: the residual cannot take its product in place."""
+    from fields_lm_amd import field
+
+    monkeypatch.setattr(field, "eager", _host_eager)
+    call = _Call(torch.nn.Linear(6, 4, bias=False), lambda layer, x, h: field._linear_residual(x, layer, h))
+    x, h, ws = torch.randn(3, 4), torch.randn(3, 6), torch.randn(5, 4, 6)
+    with torch.no_grad():
+        got = torch.func.vmap(lambda w: torch.func.functional_call(call, {"inner.weight": w}, (x.clone(), h)))(ws)
+    torch.testing.assert_close(got, x + torch.matmul(h, ws.transpose(1, 2)))
