@@ -576,11 +576,13 @@ class RefreshBlock(nn.Module):
         """x + gate * a, then its feed-forward. Without gradients the elementwise work runs in the
         Field block's two kernels (gated residual with the next norm, SwiGLU activation), rounded where
         the stock ops round, and the last product accumulates onto the residual."""
-        n2, ff = self.norm2, self.ff
+        n2, ff, gate = self.norm2, self.ff, self.residual_gate
         if (x.dtype == a.dtype == torch.bfloat16 and free_rounding() and type(self) is RefreshBlock
                 and not self.light_gate and plain_call(n2, NativeRMSNorm) and plain_call(ff, GateUpSwiGLU)
-                and not torch.is_grad_enabled() and eager(x, a, n2.weight) and x.numel() > 0):
-            x, h = gate_residual_norm(x, a, self.residual_gate(z), n2.weight, n2.eps)
+                and plain_linear(gate) and gate.weight.shape[0] == x.shape[-1] and plain_linear(ff.gate_up)
+                and not torch.is_grad_enabled() and x.numel() > 0
+                and eager(x, a, n2.weight, ff.gate_up.weight, gate.weight, *(() if gate.bias is None else (gate.bias,)))):
+            x, h = gate_residual_norm(x, a, gate(z), n2.weight, n2.eps)
             return _linear_residual(x, ff.down, swiglu(ff.gate_up(h)))
         x = self._gated(x, z, a)
         return x + ff(n2(x))

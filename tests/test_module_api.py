@@ -122,3 +122,55 @@ def test_vmap_over_the_output_layer_of_a_residual(monkeypatch):
     with torch.no_grad():
         got = torch.func.vmap(lambda w: torch.func.functional_call(call, {"inner.weight": w}, (x.clone(), h)))(ws)
     torch.testing.assert_close(got, x + torch.matmul(h, ws.transpose(1, 2)))
+
+
+@pytest.mark.parametrize("name", ["ff.gate_up.weight", "residual_gate.weight", "residual_gate.bias", "norm2.weight"])
+def test_vmap_over_refresh_block_weights_takes_the_stock_ops(monkeypatch, name):
+    from fields_lm_amd import model as M
+
+    def kernel(*args, **kw):
+        raise AssertionError("a batched tensor on its way to a kernel")
+
+    torch.manual_seed(2)
+    blk = M.RefreshBlock(32, 4, 2, 16, 64, 32, 24).to(torch.bfloat16)
+    call = _Call(blk, M.RefreshBlock._tail)
+    x, z, a = (torch.randn(2, 3, 32).to(torch.bfloat16) for _ in range(3))
+    ws = torch.stack([dict(blk.named_parameters())[name].detach() * k for k in (1, 2, 3)])
+    with torch.no_grad():
+        exp = torch.stack([torch.func.functional_call(call, {"inner." + name: w}, (x.clone(), z, a)) for w in ws])
+        monkeypatch.setattr(M, "eager", _host_eager)
+        monkeypatch.setattr(M, "gate_residual_norm", kernel)
+        monkeypatch.setattr(M.RefreshBlock, "_gated", lambda self, x, z, a: x + self._gate(z) * a)
+        got = torch.func.vmap(lambda w: torch.func.functional_call(call, {"inner." + name: w}, (x.clone(), z, a)))(ws)
+    torch.testing.assert_close(got, exp, rtol=2e-2, atol=2e-2)
+
+
+def test_refresh_block_replaced_layers_take_the_stock_ops(monkeypatch):
+    """A gate or a packed projection that is not a plain layer may return any type or width (a gate of one
+    column broadcasts): nothing that a kernel reads by address."""
+    from fields_lm_amd import model as M
+
+    def kernel(*args, **kw):
+        raise AssertionError("a replaced layer's output on its way to a kernel")
+
+    class Wide(torch.nn.Linear):
+        def forward(self, x):
+            return super().forward(x).float()
+
+    monkeypatch.setattr(M, "eager", _host_eager)
+    monkeypatch.setattr(M, "gate_residual_norm", kernel)
+    monkeypatch.setattr(M.RefreshBlock, "_gated", lambda self, x, z, a: x + self._gate(z) * a)
+    monkeypatch.setattr(M.GateUpSwiGLU, "forward", lambda self, x: self.down(torch.nn.functional.silu(
+        self.gate_up(x).chunk(2, -1)[0].bfloat16())))
+    x, z, a = (torch.randn(2, 3, 32).to(torch.bfloat16) for _ in range(3))
+    parts = [("residual_gate", torch.nn.Linear(32, 1)), ("residual_gate", torch.nn.Sequential(torch.nn.Linear(32, 32))),
+             ("gate_up", Wide(32, 48, bias=False)), ("gate_up", None)]
+    for name, layer in parts:
+        blk = M.RefreshBlock(32, 4, 2, 16, 64, 32, 24).to(torch.bfloat16)
+        owner = blk if name == "residual_gate" else blk.ff
+        if layer is None:  # the plain layer with a hook that changes its output's type
+            owner.gate_up.register_forward_hook(lambda mod, args, out: out.float())
+        else:
+            setattr(owner, name, layer.to(torch.bfloat16))
+        with torch.no_grad():
+            assert blk._tail(x.clone(), z, a).shape == x.shape
