@@ -770,14 +770,16 @@ class FieldBlock(nn.Module):
 
     def _native_training(self, x: torch.Tensor) -> bool:
         """The forward and backward kernels of ``csrc/train.hip`` take the block's elementwise work: an
-        fp32 residual stream and fp32 parameters (under bf16 autocast or none), and every module between
-        the products its own class, called without hooks."""
+        fp32 residual stream and fp32 parameters (under bf16 autocast or none), every module between
+        the products its own class, called without hooks, and plain layers behind the norms, whose bf16 output
+        is the cast such a layer makes of its input."""
         m, ff, dim = self.mixer, self.ff, x.shape[-1]
         if not (torch.is_grad_enabled() and x.dtype == torch.float32 and x.numel() > 0 and x.ndim == 3
                 and dim == m.dim and dim % 8 == 0 and dim <= 2048 and x.numel() // dim < 1 << 31
                 and type(self) is FieldBlock and plain_call(m, IndependentVacancyField)
                 and plain_call(self.ff_norm, RMSNorm) and plain_call(m.read_norm, RMSNorm)
                 and type(ff).__dict__.get("packed_swiglu") and plain_call(ff, type(ff))
+                and plain_linear(m.out_proj) and plain_linear(_ff_layers(ff)[0])
                 and _MIXER_METHODS.isdisjoint(m.__dict__) and m.read_dtype == "auto" and self.fuse_tail
                 and (not torch.is_autocast_enabled() or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
             return False

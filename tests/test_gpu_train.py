@@ -135,3 +135,23 @@ def test_training_replaced_parts_keep_the_stock_ops(dev):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t, lambda t: t):
         b(x)
     assert seen
+
+
+def test_training_replaced_product_sees_fp32_under_autocast(dev):
+    print("[case] block training, a product that computes in fp32", flush=True)
+
+    class Fp32Linear(torch.nn.Linear):
+        def forward(self, x):
+            seen.append(x.dtype)
+            with torch.autocast("cuda", enabled=False):
+                return super().forward(x)
+
+    for owner, name in (("mixer", "out_proj"), ("ff", "w12")):
+        b = _block(dev, 64, 40)
+        layer = getattr(getattr(b, owner), name)
+        layer.__class__ = Fp32Linear
+        x = torch.randn(1, 5, 64, device=dev, requires_grad=True)
+        seen = []
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            b(x).sum().backward()
+        assert seen == [torch.float32] and x.grad.isfinite().all()

@@ -174,3 +174,27 @@ def test_refresh_block_replaced_layers_take_the_stock_ops(monkeypatch):
             setattr(owner, name, layer.to(torch.bfloat16))
         with torch.no_grad():
             assert blk._tail(x.clone(), z, a).shape == x.shape
+
+
+def _training_block(monkeypatch):
+    from fields_lm_amd import field
+
+    monkeypatch.setattr(field, "eager", _host_eager)
+    block = FieldBlock(16, "triton", 8, 8, 16, 24)
+    return block, torch.randn(1, 3, 16)
+
+
+def test_training_route_leaves_replaced_products_their_fp32_input(monkeypatch):
+    """Under autocast the kernels write what a product reads in bf16; a layer that computes otherwise, or a
+    hook that sees the input, gets the stock ops' fp32 values."""
+    block, x = _training_block(monkeypatch)
+    assert block._native_training(x)
+    for owner, name in ((block.mixer, "out_proj"), (block.ff, "w12")):
+        layer = getattr(owner, name)
+        handle = layer.register_forward_pre_hook(lambda mod, args: None)
+        assert not block._native_training(x)
+        handle.remove()
+        setattr(owner, name, torch.nn.Sequential(layer))
+        assert not block._native_training(x)
+        setattr(owner, name, layer)
+    assert block._native_training(x)
