@@ -785,7 +785,8 @@ class FieldBlock(nn.Module):
             return False
         norms = (m.read_norm.weight, self.ff_norm.weight)
         ring = (m.radius_logit, m.theta)
-        return (all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in norms)
+        return (norms[0].shape == (2 * dim,) and norms[1].shape == (dim,)
+                and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in norms)
                 and all(t.dtype == torch.float32 and t.is_contiguous() and t.shape == (m.channels,) for t in ring)
                 and eager(x, *norms, *ring))
 
@@ -796,13 +797,14 @@ class FieldBlock(nn.Module):
         tr, ti, gamma = train.Transition.apply(m.radius_logit, m.theta)
         read = fused_field_read(m._raw(x, raw), tr, ti, gamma, m.triton_block_c, m.triton_chunk_t)
         out = m.out_proj(train.Norm.apply(read, m.read_norm.weight, m.read_norm.eps, dtype))
-        if out.dtype != gate_pre.dtype or out.dtype not in KERNEL_DTYPES:
+        if not (out.dtype == gate_pre.dtype and out.dtype in KERNEL_DTYPES and eager(x, out, gate_pre)
+                and out.shape == gate_pre.shape == x.shape):
             x = x + (out * torch.sigmoid(gate_pre)).to(x.dtype)
             return x + self.ff(self.ff_norm(x))
         x, h = train.GateNorm.apply(x, out, gate_pre, self.ff_norm.weight, self.ff_norm.eps, dtype)
         first, second = _ff_layers(self.ff)
         gu = first(h)
-        if gu.dtype in KERNEL_DTYPES and gu.shape[-1] % 16 == 0 and gu.numel() < 1 << 34:
+        if gu.dtype in KERNEL_DTYPES and gu.shape[-1] % 16 == 0 and 0 < gu.numel() < 1 << 34 and eager(gu):
             return x + second(train.Swiglu.apply(gu))
         return x + second(train._swiglu_ops(gu))
 

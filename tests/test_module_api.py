@@ -198,3 +198,58 @@ def test_training_route_leaves_replaced_products_their_fp32_input(monkeypatch):
         assert not block._native_training(x)
         setattr(owner, name, layer)
     assert block._native_training(x)
+
+
+@pytest.mark.parametrize("case", ["batched gate", "batched out", "batched up", "one gate column", "scalar norm"])
+def test_training_route_checks_what_its_kernels_read(monkeypatch, case):
+    """Outputs of batched or replaced layers, and weights of another shape that broadcast in the stock ops,
+    stay with the stock ops."""
+    from fields_lm_amd import field
+
+    block, x = _training_block(monkeypatch)
+    m = block.mixer
+
+    def scan(raw, tr, ti, gamma, *args, **kw):
+        return torch.cat((raw, raw[..., :raw.shape[-1] // 3]), -1)
+
+    class Kernel:
+        def __getattr__(self, name):
+            raise AssertionError(name)
+
+    def norm(t, w, eps, dtype):
+        assert w.shape == t.shape[-1:] and _host_eager(t, w)
+        return (t * torch.rsqrt(t.square().mean(-1, keepdim=True) + eps) * w).to(dtype)
+
+    def gate_norm(t, out, gate, w, eps, dtype):
+        assert out.shape == gate.shape == t.shape and _host_eager(t, out, gate)
+        t = t + out * torch.sigmoid(gate)
+        return t, norm(t, w, eps, dtype)
+
+    monkeypatch.setattr(field, "fused_field_read", scan)
+    monkeypatch.setattr(field.nat, "load", Kernel)
+    for name, fn in (("Transition", lambda *a: field.train.transition_ops(*a)), ("Norm", norm), ("GateNorm", gate_norm)):
+        monkeypatch.setattr(field.train, name, type(name, (), {"apply": staticmethod(fn)}))
+
+    def swiglu(gu):
+        assert _host_eager(gu)
+        return field.train._swiglu_ops(gu)
+
+    monkeypatch.setattr(field.train, "Swiglu", type("Swiglu", (), {"apply": staticmethod(swiglu)}))
+    monkeypatch.setattr(field.IndependentVacancyField, "normed_read",
+                        lambda self, t, raw=None: self.read_norm(scan(self.write_proj(t) if raw is None else raw, None, None, None)))
+    if case == "one gate column":
+        m.gate_proj = torch.nn.Linear(16, 1)
+    elif case == "scalar norm":
+        block.ff_norm.weight = torch.nn.Parameter(torch.ones(1))
+    name = {"batched gate": "mixer.gate_proj.weight", "batched out": "mixer.out_proj.weight", "batched up": "ff.w12.weight"}.get(case)
+    if name is None:
+        block.fuse_tail = False
+        exp = block(x)
+        block.fuse_tail = True
+        torch.testing.assert_close(block(x), exp)
+        return
+    ws = torch.stack([dict(block.named_parameters())[name].detach() * k for k in (1, 2)])
+    got = torch.func.vmap(lambda w: torch.func.functional_call(block, {name: w}, (x,)))(ws)
+    block.fuse_tail = False
+    exp = torch.stack([torch.func.functional_call(block, {name: w}, (x,)) for w in ws])
+    torch.testing.assert_close(got, exp)
