@@ -740,6 +740,11 @@ def _ff_layers(ff: nn.Module) -> Tuple[nn.Module, nn.Module]:
     return (ff.w12, ff.w3) if hasattr(ff, "w12") else (ff.gate_up, ff.down)
 
 
+def _plain_ff(ff: nn.Module) -> bool:
+    """``ff`` is a packed SwiGLU by its class's own word, and calling it is nothing but its forward."""
+    return bool(type(ff).__dict__.get("packed_swiglu")) and plain_call(ff, type(ff))
+
+
 class FieldBlock(nn.Module):
     """canon:1198-1221: x = mixer(x) (residual inside); x + ff(ff_norm(x))."""
 
@@ -756,9 +761,7 @@ class FieldBlock(nn.Module):
     # The elementwise tail (gated residual, ff_norm, SwiGLU activation) runs in two fused launches
     # on the inference path (no gradient needed); the GEMMs stay stock.
     def _fused_tail(self, x: torch.Tensor) -> bool:
-        if not self.fuse_tail or type(self.ff_norm) is not RMSNorm:
-            return False
-        if not (hasattr(self.ff, "w12") or hasattr(self.ff, "gate_up")):
+        if not self.fuse_tail or type(self.ff_norm) is not RMSNorm or not _plain_ff(self.ff):
             return False
         return not (torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters())))
 
@@ -778,8 +781,7 @@ class FieldBlock(nn.Module):
                 and dim == m.dim and dim % 8 == 0 and dim <= 2048 and x.numel() // dim < 1 << 31
                 and type(self) is FieldBlock and plain_call(m, IndependentVacancyField)
                 and plain_call(self.ff_norm, RMSNorm) and plain_call(m.read_norm, RMSNorm)
-                and type(ff).__dict__.get("packed_swiglu") and plain_call(ff, type(ff))
-                and plain_linear(m.out_proj) and plain_linear(_ff_layers(ff)[0])
+                and _plain_ff(ff) and plain_linear(m.out_proj) and plain_linear(_ff_layers(ff)[0])
                 and _MIXER_METHODS.isdisjoint(m.__dict__) and m.read_dtype == "auto" and self.fuse_tail
                 and (not torch.is_autocast_enabled() or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
             return False
@@ -835,6 +837,8 @@ class FieldBlock(nn.Module):
             return None
         parts = self._modules
         m, ff, ff_norm = parts["mixer"], parts["ff"], parts["ff_norm"]
+        if not _plain_ff(ff):
+            return None
         rows, dim = x_t.shape
         if not (type(self) is FieldBlock and type(m) is IndependentVacancyField and dim == m.dim == 2 * m.channels
                 and dim % 8 == 0 and dim <= 8192 and self.fuse_tail and m.fuse_in_proj and m.fuse_read_norm

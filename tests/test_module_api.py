@@ -253,3 +253,48 @@ def test_training_route_checks_what_its_kernels_read(monkeypatch, case):
     block.fuse_tail = False
     exp = torch.stack([torch.func.functional_call(block, {name: w}, (x,)) for w in ws])
     torch.testing.assert_close(got, exp)
+
+
+def _step_call(monkeypatch):
+    from fields_lm_amd import field
+    from fields_lm_amd import model as M
+
+    torch.manual_seed(4)
+    block = M.cast_for_inference(FieldBlock(16, "triton", 8, 8, 16, 24))
+    x, state = torch.randn(2, 16).to(torch.bfloat16), torch.zeros(2, 16)
+    params = tuple(t.clone() for t in block.mixer.decode_params())  # the stock ops: no device here
+    monkeypatch.setattr(field, "eager", _host_eager)
+    return block, x, state, params
+
+
+class _Gelu(torch.nn.Module):
+    """A feed-forward with the packed layout's names and another activation."""
+
+    def __init__(self):
+        super().__init__()
+        self.gate_up, self.down = torch.nn.Linear(16, 48, bias=False), torch.nn.Linear(24, 16, bias=False)
+
+    def forward(self, x):
+        gate, up = self.gate_up(x).chunk(2, -1)
+        return self.down(torch.nn.functional.gelu(gate) * up)
+
+
+def test_step_and_tail_ask_what_the_feed_forward_is(monkeypatch):
+    """Only this package's SwiGLU classes, called without hooks, run as kernels; any other module is called."""
+    block, x, state, params = _step_call(monkeypatch)
+    with torch.no_grad():
+        assert block._native_step(x, state, params) is not None and block._fused_tail(x)
+        ff = block.ff
+        handle = ff.register_forward_hook(lambda mod, args, out: out * 2)
+        assert block._native_step(x, state, params) is None and not block._fused_tail(x)
+        handle.remove()
+        for other in (_Gelu(), torch.nn.Sequential(torch.nn.Linear(16, 16)), torch.nn.Identity()):
+            block.ff = other.to(torch.bfloat16)
+            assert block._native_step(x, state, params) is None and not block._fused_tail(x)
+        block.ff = ff
+        for owner, name in ((block, "ff_norm"), (block.mixer, "read_norm"), (block.mixer, "write_proj"),
+                            (block.mixer, "gate_proj"), (block.mixer, "out_proj"), (ff, "w12"), (ff, "w3")):
+            handle = getattr(owner, name).register_forward_pre_hook(lambda mod, args: None)
+            assert block._native_step(x, state, params) is None, name
+            handle.remove()
+        assert block._native_step(x, state, params) is not None
