@@ -861,7 +861,9 @@ class FieldBlock(nn.Module):
         if not (ub is None and db is None and hidden % 8 == 0 and 0 < hidden <= 65536
                 and [t.shape for t in matrices] == [(3 * m.channels, dim), (dim, dim), (dim, 2 * dim),
                                                     (2 * hidden, dim), (dim, hidden)]
+                and [t.shape for t in vectors] == [t.shape[:1] for t, b in zip(matrices, (wb, gb, ob)) if b is not None]
                 and tr.numel() == ti.numel() == gamma.numel() == m.channels and read_w.numel() == 2 * dim
+                and norm.shape == (dim,)
                 and state.shape == (rows, dim) and norm.dtype in KERNEL_DTYPES
                 and eager(x_t, norm, *fp32, *matrices, *vectors)):
             return None

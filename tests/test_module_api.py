@@ -298,3 +298,14 @@ def test_step_and_tail_ask_what_the_feed_forward_is(monkeypatch):
             assert block._native_step(x, state, params) is None, name
             handle.remove()
         assert block._native_step(x, state, params) is not None
+
+
+@pytest.mark.parametrize("name,entries", [("write_proj.bias", 1), ("gate_proj.bias", 1), ("out_proj.bias", 1), ("ff_norm.weight", 1)])
+def test_step_checks_the_length_of_vectors(monkeypatch, name, entries):
+    """A bias or norm weight of one entry broadcasts in the stock ops; the kernels read whole vectors."""
+    block, x, state, params = _step_call(monkeypatch)
+    owner, attr = name.split(".")
+    layer = block.ff_norm if owner == "ff_norm" else getattr(block.mixer, owner)
+    setattr(layer, attr, torch.nn.Parameter(torch.ones(entries, dtype=torch.bfloat16)))
+    with torch.no_grad():
+        assert block._native_step(x, state, params) is None
