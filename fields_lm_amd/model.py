@@ -967,15 +967,18 @@ class BoundaryStateMixer(nn.Module):
 
     def _native(self, x: torch.Tensor, tokens: torch.Tensor) -> bool:
         """The kernels of ``fl_softpatch_norm`` / ``fl_softpatch_scan`` take this call."""
-        score, norm, up, lut = self.score, self.norm, self.up, self._boundary_lut
+        score, norm, down, up, lut = self.score, self.norm, self.down, self.up, self._boundary_lut
         if not (free_rounding() and type(self) is BoundaryStateMixer and self.learned and x.ndim == 3
                 and plain_call(norm, RMSNorm) and plain_linear(score) and score.bias is not None
-                and plain_linear(up) and up.bias is None and x.is_contiguous() and x.data_ptr() % 16 == 0):
+                and plain_linear(down) and down.bias is None and plain_linear(up) and up.bias is None
+                and x.is_contiguous() and x.data_ptr() % 16 == 0):
             return False
-        params = (norm.weight, score.weight, score.bias, up.weight)
-        return (rms_norm_takes(x, norm.weight) and no_grad_needed(*params, self.down.weight)
+        params = (norm.weight, score.weight, score.bias, down.weight, up.weight)
+        dim, rank = x.shape[-1], down.weight.shape[0]
+        return (rms_norm_takes(x, norm.weight) and no_grad_needed(*params) and 0 < rank <= 1 << 16
+                and [t.shape for t in params] == [(dim,), (1, dim), (1,), (rank, dim), (dim, 2 * rank)]
                 and eager(x, tokens, lut, *params)
-                and lut.dtype == torch.float32 and tokens.shape == x.shape[:2]
+                and lut.dtype == torch.float32 and lut.ndim == 1 and tokens.shape == x.shape[:2]
                 and all(t.dtype == x.dtype and t.is_contiguous() for t in params)
                 and score.weight.data_ptr() % 16 == 0 and x.shape[0] <= 65535 and x.shape[1] <= 1 << 26)
 

@@ -309,3 +309,33 @@ def test_step_checks_the_length_of_vectors(monkeypatch, name, entries):
     setattr(layer, attr, torch.nn.Parameter(torch.ones(entries, dtype=torch.bfloat16)))
     with torch.no_grad():
         assert block._native_step(x, state, params) is None
+
+
+def test_softpatch_route_asks_what_its_layers_are(monkeypatch):
+    """A down projection, scorer or up projection that is wrapped, hooked or of another width stays with the
+    stock ops: the kernels read bf16 rows of the rank's width by address."""
+    from fields_lm_amd import field
+    from fields_lm_amd import model as M
+
+    monkeypatch.setattr(field, "eager", _host_eager)
+    monkeypatch.setattr(M, "eager", _host_eager)
+    x, tok = torch.randn(1, 3, 32).to(torch.bfloat16), torch.zeros(1, 3, dtype=torch.long)
+
+    def mixer():
+        sp = M.BoundaryStateMixer(32, 8, vocab=5)
+        return M.cast_for_inference(sp)
+
+    with torch.no_grad():
+        assert mixer()._native(x, tok)
+        for edit in (lambda sp: setattr(sp, "down", torch.nn.Sequential(sp.down)),
+                     lambda sp: setattr(sp, "down", torch.nn.Identity()),
+                     lambda sp: sp.down.register_forward_hook(lambda mod, args, out: out.float()),
+                     lambda sp: setattr(sp, "down", torch.nn.Linear(32, 8).to(torch.bfloat16)),
+                     lambda sp: setattr(sp, "down", torch.nn.Linear(32, 6, bias=False).to(torch.bfloat16)),
+                     lambda sp: setattr(sp, "down", torch.nn.Linear(32, 8, bias=False)),
+                     lambda sp: setattr(sp, "score", torch.nn.Linear(16, 1).to(torch.bfloat16)),
+                     lambda sp: setattr(sp, "score", torch.nn.Linear(32, 2).to(torch.bfloat16)),
+                     lambda sp: setattr(sp, "up", torch.nn.Linear(16, 16, bias=False).to(torch.bfloat16))):
+            sp = mixer()
+            edit(sp)
+            assert not sp._native(x, tok)
