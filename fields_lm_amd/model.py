@@ -682,7 +682,8 @@ def ssd_chunked(x, dt, A, Bm, Cm, chunk: int, initial_state=None, *, finish=None
         causal = torch.ones(chunk, chunk, device=x.device, dtype=torch.bool).tril()
         weights = cb[:, None] * torch.exp(seg.masked_fill(~causal, float("-inf")))
     w_end = torch.exp(acs[..., -1:] - acs)                                              # [b,h,c,s]
-    if (_autocast_operands(cb, w_end, *given) and b * h <= 65535 and 0 < c <= 65535 and chunk <= 4096
+    if (_autocast_operands(cb, w_end, *given) and given[1].shape == (b, l, h)
+            and b * h <= 65535 and 0 < c <= 65535 and chunk <= 4096
             and 0 < p <= 4096 and l > 0 and x.stride(-1) == 1 and x.stride(-2) == p and x.stride(0) >= 0
             and x.stride(1) >= h * p and dt.is_contiguous() and w_end.is_contiguous()):
         xdt = torch.empty((b, h, c, chunk, p), device=x.device, dtype=cb.dtype)
@@ -762,8 +763,11 @@ class Mamba2Mixer(nn.Module):
         """The kernels of ``fl_mamba_prefill`` / ``fl_mamba_step`` take this call: the promoted
         geometry, no gradient, every tensor where and what they read."""
         params = (self.conv1d.weight, self.conv1d.bias, self.A_log, self.dt_bias, self.D, self.norm.weight)
+        heads, inner, channels = self.nheads, self.d_inner, self.conv_dim
         return (free_rounding() and type(self) is Mamba2Mixer and plain_call(self.norm, GatedRMSNorm)
-                and (self.headdim, self.d_state, self.d_conv) == (64, 128, 4) and self.nheads <= 1024
+                and (self.headdim, self.d_state, self.d_conv) == (64, 128, 4) and heads <= 1024
+                and inner == 64 * heads and zxbcdt.shape[-1] == inner + channels + heads
+                and [t.shape for t in params] == [(channels, 1, 4), (channels,), (heads,), (heads,), (heads,), (inner,)]
                 and no_grad_needed(zxbcdt, *params) and eager(zxbcdt, *params)
                 and zxbcdt.dtype in KERNEL_DTYPES and zxbcdt.is_contiguous() and zxbcdt.numel() > 0
                 and zxbcdt.shape[-1] % 2 == 0 and zxbcdt.data_ptr() % 8 == 0
@@ -824,6 +828,7 @@ class Mamba2Mixer(nn.Module):
         if not (plain_call(self.norm, GatedRMSNorm) and _autocast_operands(y, acs, xh)
                 and no_grad_needed(y_off, z, self.D) and eager(y_off, z, self.D) and z.dtype == y_off.dtype == y.dtype
                 and y.is_contiguous() and y_off.is_contiguous() and y_off.shape == y.shape and acs.is_contiguous()
+                and self.D.shape == (h,) and z.shape == (b, l, h * p) and self.d_inner == h * p
                 and p % 4 == 0 and p <= 4096 and s <= 4096 and b * h <= 65535 and 0 < c <= 65535
                 and xh.stride(-1) == z.stride(-1) == 1 and xh.stride(-2) == p and xh.stride(1) >= h * p
                 and z.stride(1) >= h * p and xh.data_ptr() % 16 == 0 and z.data_ptr() % 8 == 0
@@ -845,6 +850,7 @@ class Mamba2Mixer(nn.Module):
         if (xbc_raw.dtype == torch.bfloat16 and self.d_conv == 4 and no_grad_needed(xbc_raw, weight, bias)
                 and eager(xbc_raw, weight, bias) and xbc_raw.stride(-1) == 1 and 0 < b <= 65535 and 0 < l <= 1 << 19
                 and xbc_raw.stride(1) >= channels and xbc_raw.stride(0) >= 0 and weight.dtype == bias.dtype
+                and weight.shape == (channels, 1, 4) and bias.shape == (channels,)
                 and weight.dtype in KERNEL_DTYPES and weight.is_contiguous() and bias.is_contiguous()):
             out = torch.empty((b, l, channels), device=xbc_raw.device, dtype=torch.float32)
             nat.check(nat.load().fl_conv_silu(

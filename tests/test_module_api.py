@@ -339,3 +339,52 @@ def test_softpatch_route_asks_what_its_layers_are(monkeypatch):
             sp = mixer()
             edit(sp)
             assert not sp._native(x, tok)
+
+
+def test_mamba_routes_check_what_their_kernels_read(monkeypatch):
+    """Parameters that broadcast in the stock ops, a projection of another width, and an inner width that is
+    no whole number of heads: the kernels read by the promoted shapes."""
+    from fields_lm_amd import model as M
+
+    monkeypatch.setattr(M, "eager", _host_eager)
+
+    class Kernel:
+        def __getattr__(self, name):
+            raise AssertionError(name)
+
+    monkeypatch.setattr(M.nat, "load", Kernel)
+    one = lambda n=1: torch.nn.Parameter(torch.ones(n))  # noqa: E731
+    with torch.no_grad():
+        m = M.Mamba2Mixer(64)
+        z = m.in_proj(torch.randn(1, 3, 64))
+        assert m._native(z) and not m._native(z[..., :-2].contiguous()) and not m._native(torch.cat((z, z[..., :2]), -1))
+        for name in ("A_log", "dt_bias", "D"):
+            m = M.Mamba2Mixer(64)
+            setattr(m, name, one())
+            assert not m._native(z), name
+        for owner, name, value in (("norm", "weight", one()), ("conv1d", "bias", one()),
+                                   ("conv1d", "weight", torch.nn.Parameter(torch.ones(1, 1, 4)))):
+            m = M.Mamba2Mixer(64)
+            setattr(getattr(m, owner), name, value)
+            assert not m._native(z), name
+        m = M.Mamba2Mixer(48)  # 96 channels: one head and a half
+        assert not m._native(m.in_proj(torch.randn(1, 3, 48)))
+        m = M.Mamba2Mixer(64)
+        rows = torch.randn(1, 3, m.conv_dim).to(torch.bfloat16)
+        for name, value in (("bias", one()), ("weight", torch.nn.Parameter(torch.ones(1, 1, 4)))):
+            m = M.Mamba2Mixer(64)
+            setattr(m.conv1d, name, value)
+            assert m._conv_silu(rows).shape == rows.shape  # the stock ops: no kernel was called
+        monkeypatch.setattr(M, "_autocast_operands", lambda product, *others: product.dtype == torch.bfloat16)
+        m = M.Mamba2Mixer(64)
+        m.D = one()
+        b, h, c, s, p, length = 1, 2, 1, 4, 64, 3
+        y = torch.zeros(b, h, c, s, p, dtype=torch.bfloat16)
+        acs, xh = torch.zeros(b, h, c, s), torch.zeros(b, length, h, p)
+        zz = torch.zeros(b, length, h * p, dtype=torch.bfloat16)
+        assert m._finish(y, y, acs, xh, zz) is None
+        monkeypatch.setattr(M, "_autocast_operands",
+                            lambda product, *others: len(others) == 3)  # only the operands' kernel
+        y, _ = M.ssd_chunked(torch.randn(1, 8, 2, 4), torch.rand(1, 8, 1), -torch.ones(2), torch.randn(1, 8, 4),
+                             torch.randn(1, 8, 4), 8)
+        assert y.shape == (1, 8, 2, 4)
