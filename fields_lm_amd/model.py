@@ -270,9 +270,10 @@ class LandmarkAttention(nn.Module):
         return gqa_attention(q, lk, lv, None, False, chunk=self.landmark_chunk)
 
     def _plain(self, qlat: torch.Tensor) -> bool:
-        """``kv_up`` and the projection are what the kernels take their outputs for."""
+        """``kv_up``, the projection and the mix are what the kernels take them for."""
         up = self.kv_up
         return (plain_linear(up) and up.weight.shape == (2 * self.kv_heads * self.head_dim, self.latent_dim)
+                and self.global_mix_logit.numel() == 1
                 and qlat.shape[-1] == self.q_width + self.latent_dim)
 
     def _native(self, qlat: torch.Tensor) -> bool:

@@ -388,3 +388,19 @@ def test_mamba_routes_check_what_their_kernels_read(monkeypatch):
         y, _ = M.ssd_chunked(torch.randn(1, 8, 2, 4), torch.rand(1, 8, 1), -torch.ones(2), torch.randn(1, 8, 4),
                              torch.randn(1, 8, 4), 8)
         assert y.shape == (1, 8, 2, 4)
+
+
+@pytest.mark.parametrize("shape", [(64,), (4, 1, 1)])
+def test_refresh_attention_with_a_wider_mix_takes_the_stock_ops(monkeypatch, shape):
+    """global_mix_logit per dimension or per head broadcasts in the stock ops; the kernels read one value."""
+    from fields_lm_amd import model as M
+
+    monkeypatch.setattr(M, "eager", _host_eager)
+    att = M.cast_for_inference(M.LandmarkAttention(256, 4, 2, 16, 64, 32))
+    x = torch.randn(2, 5, 256).to(torch.bfloat16)
+    with torch.no_grad():
+        st = att.new_state(2, 40, x.device, x.dtype)
+        qlat, pos = att.q_latent_proj(x), torch.tensor(0)
+        assert att._native(qlat) and att._exact(x, qlat) and att._native_step(qlat[:, 0].contiguous(), pos, st)
+        att.global_mix_logit = torch.nn.Parameter(torch.zeros(shape, dtype=torch.bfloat16))
+        assert not (att._native(qlat) or att._exact(x, qlat) or att._native_step(qlat[:, 0].contiguous(), pos, st))
