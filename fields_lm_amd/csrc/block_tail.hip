@@ -40,12 +40,12 @@ __device__ __forceinline__ void load_weight(const void* w, int w16, int c, float
 // gate = sigmoid(g), prod = out * gate (in the GEMM output type G), x1 = x + prod (in the
 // residual type X), h = RMSNorm(x1) * w (fp32 math, rounded to X).
 // Bound by memory at prefill sizes (five [rows, dim] streams) and by the launch at decode sizes.
-// One wave per row, 16 bytes per lane and access with N = 8 (bf16). The sum of squares keeps one
+// One wave per row, 16 bytes per lane and access with N = 8 (bf16), four rows per block. The sum of squares keeps one
 // order for every N and launch shape: 256 strided chains over the row (c = i, i + 256, ...), each
 // 64 of them added by a butterfly, the four sums in sequence; the row's values reach their chains
 // through LDS (RES floats per wave; longer rows in pieces). So a row's result does not depend on
 // its alignment or on the size of the batch. Rows 8,192 x dim 1,024, bf16 (84 MB): 14.2 us,
-// 5.9 TB/s; one 256-thread block per row with 2-byte accesses and a library sigmoid took 19.2 us.
+// 5.9 TB/s; the block per row below takes 18.1 us.
 // ------------------------------------------------------------------------------------------
 template <typename XT, typename GT, int N, int RES>
 __global__ __launch_bounds__(256) void fl_gate_residual_norm_kernel(
@@ -115,32 +115,107 @@ __global__ __launch_bounds__(256) void fl_gate_residual_norm_kernel(
   }
 }
 
+// The same with a block of four waves per row, one element per thread and access: what a row without 16-byte
+// access takes, where a wave alone would run through its elements four times as long (and through its two
+// exponential chains twice, past one piece). NPER: elements that a thread keeps, 0 for longer rows, which are
+// formed twice. The sum has the order above: thread c's chain is columns c, c + 256, ...
+template <typename XT, typename GT, int NPER>
+__global__ __launch_bounds__(256) void fl_gate_residual_norm_block_kernel(
+    const XT* __restrict__ x, const GT* __restrict__ out, const GT* __restrict__ gpre, int64_t gstride, int dim,
+    const void* __restrict__ w, int w16, float eps, float inv_dim, XT* __restrict__ x_new, XT* __restrict__ normed) {
+  __shared__ float s_sum[4];
+  const int64_t base = (int64_t)blockIdx.x * dim;
+  const GT* grow = gpre + (int64_t)blockIdx.x * gstride;
+  auto residual = [&](int c) {
+    const float prod = round_as<GT>(load_as<GT>(out + base + c) * round_as<GT>(sigmoid<GT>(load_as<GT>(grow + c))));
+    return round_as<XT>(load_as<XT>(x + base + c) + prod);
+  };
+  float v[NPER > 0 ? NPER : 1], acc = 0.f;
+  if constexpr (NPER > 0) {
+#pragma unroll
+    for (int i = 0; i < NPER; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      v[i] = c < dim ? residual(c) : 0.f;
+      acc = fmaf(v[i], v[i], acc);
+    }
+  } else {
+    for (int c = threadIdx.x; c < dim; c += 256) {
+      const float r = residual(c);
+      acc = fmaf(r, r, acc);
+    }
+  }
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  const float tot = ((s_sum[0] + s_sum[1]) + s_sum[2]) + s_sum[3], scale = rsqrtf(fmaf(tot, inv_dim, eps));
+  auto put = [&](int c, float r, float weight) {
+    store_as(x_new + base + c, r);
+    store_as(normed + base + c, (r * scale) * weight);
+  };
+  if constexpr (NPER > 0) {
+#pragma unroll
+    for (int i = 0; i < NPER; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      if (c >= dim) continue;
+      float ww;
+      load_weight<1>(w, w16, c, &ww);
+      put(c, v[i], ww);
+    }
+  } else {
+    auto again = [&](const auto* weight) {  // a branch on the weight's type per element cost 5 %
+      for (int c = threadIdx.x; c < dim; c += 256) put(c, residual(c), load_as(weight + c));
+    };
+    if (w16) again(static_cast<const bf16_bits*>(w));
+    else again(static_cast<const float*>(w));
+  }
+}
+
 template <typename XT, typename GT>
 int launch_gate_residual_norm(const void* x, const void* out, const void* gate_pre, int64_t rows,
                               int64_t dim, int64_t gate_stride, const void* w, int w16, float eps,
                               void* x_new, void* normed, hipStream_t s) {
   const float inv = (float)(1.0 / (double)dim);
-  // four rows per block once that still gives every CU several blocks; below, one row per block,
-  // so that the rows of a decode batch spread over as many CUs as there are rows
-  const unsigned waves = rows >= 4096 ? 4 : 1;
-  const unsigned blocks = (unsigned)cdiv(rows, waves);
 #define FL_GRN1(N, RES)                                                                         \
   {                                                                                             \
-    fl_gate_residual_norm_kernel<XT, GT, N, RES><<<blocks, waves * 64, waves * RES * 4, s>>>(                 \
+    fl_gate_residual_norm_kernel<XT, GT, N, RES><<<(unsigned)cdiv(rows, 4), 256, 4 * RES * 4, s>>>( \
         static_cast<const XT*>(x), static_cast<const GT*>(out), static_cast<const GT*>(gate_pre), \
         gate_stride, rows, (int)dim, w, w16, eps, inv, static_cast<XT*>(x_new),                 \
         static_cast<XT*>(normed));                                                              \
     return hip_status(hipGetLastError());                                                       \
   }
+#define FL_GRB(NPER)                                                                              \
+  {                                                                                               \
+    fl_gate_residual_norm_block_kernel<XT, GT, NPER><<<(unsigned)rows, 256, 0, s>>>(              \
+        static_cast<const XT*>(x), static_cast<const GT*>(out), static_cast<const GT*>(gate_pre), \
+        gate_stride, (int)dim, w, w16, eps, inv, static_cast<XT*>(x_new), static_cast<XT*>(normed)); \
+    return hip_status(hipGetLastError());                                                         \
+  }
   // 16-byte accesses: whole vectors per row and every row start aligned
   const bool vec = dim % 8 == 0 && gate_stride % 8 == 0 && aligned(x, 16) && aligned(out, 16) &&
                    aligned(gate_pre, 16) && aligned(w, 16) && aligned(x_new, 16) && aligned(normed, 16);
-  if (vec) {
-    if (dim <= 512) FL_GRN1(8, 512)
-    if (dim <= 1024) FL_GRN1(8, 1024)
-    FL_GRN1(8, 2048)
+  // A wave per row and 16 bytes a lane pay once the rows are many enough to be bound by memory, and the
+  // sooner the fewer bytes a row has; with few rows four waves finish a row sooner than one. us, wave | block:
+  //   bf16 / bf16, dim 1,024:   64 rows 3.3 | 3.1,  1,000 4.2 | 4.0,  2,048 5.5 | 5.5,  4,096 8.6 | 9.8,  16,384 26 | 33
+  //   fp32 / bf16, dim 1,024:   2,048 rows 8.2 | 6.6,  4,096 14.1 | 13.1,  8,192 23.7 | 23.1,  16,384 49 | 56
+  //   fp32 / fp32, dim 1,024:   1,000 rows 5.7 | 4.7,  4,096 15.5 | 15.5,  16,384 66 | 65
+  //   bf16 / bf16, dim 4,096:   64 rows 9.8 | 8.3,  1,000 14.0 | 15.2,  4,096 40 | 44
+  //   256 and fewer columns:    bf16 8,192 rows 6.6 | 5.9,  16,384 11.2 | 12.0
+  //   no 16-byte access, bf16, dim 1,022:  64 rows 8.5 | 3.2,  4,096 21 | 10.4,  16,384 49 | 35
+  // (one row per block of the wave kernel instead of four: within 2 % from 512 rows on)
+  if constexpr (sizeof(XT) == 2 || sizeof(GT) == 2) {
+    if (vec && rows * dim >= (dim <= 256 ? 1 << 22 : sizeof(XT) == 2 ? 1 << 21 : 1 << 23)) {
+      if (dim <= 512) FL_GRN1(8, 512)
+      if (dim <= 1024) FL_GRN1(8, 1024)
+      FL_GRN1(8, 2048)
+    }
   }
-  FL_GRN1(1, 256)
+  if (dim <= 256 && rows >= 16384) FL_GRN1(1, 256)
+  if (dim <= 256) FL_GRB(1)
+  if (dim <= 512) FL_GRB(2)
+  if (dim <= 1024) FL_GRB(4)
+  if (dim <= 2048) FL_GRB(8)
+  FL_GRB(0)
+#undef FL_GRB
 #undef FL_GRN1
 }
 

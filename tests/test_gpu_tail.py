@@ -84,6 +84,28 @@ def test_gate_residual_norm_edges(dev, rows, dim, wdtype):
     _one_step(h, exp_h, out.float() * (exp_h.float() / xf.abs().clamp_min(1e-3)))
 
 
+@pytest.mark.parametrize("rows,dim,xt,gt", [(4034, 520, "bf16", "bf16"), (2050, 1024, "bf16", "f32"), (31776, 264, "f32", "bf16"),
+                                            (16385, 40, "bf16", "bf16"), (16384, 256, "f32", "bf16"), (1021, 2056, "bf16", "bf16")])
+def test_gate_residual_norm_routes_agree(dev, rows, dim, xt, gt):
+    """Where the wave per row begins: the same bits as the block per row gives a part of the same rows (and
+    as a misaligned copy gets), so that a row's result does not depend on its batch."""
+    from fields_lm_amd import gate_residual_norm
+
+    print(f"[case] gate_residual_norm routes {rows}x{dim} {xt}/{gt}", flush=True)
+    types = {"bf16": torch.bfloat16, "f32": torch.float32}
+    g = torch.Generator(device=dev).manual_seed(dim)
+    x, out, gp = (2 * torch.randn(rows, dim, device=dev, generator=g) for _ in range(3))
+    x, out, gp = x.to(types[xt]), out.to(types[gt]), gp.to(types[gt])
+    w = 1.0 + 0.3 * torch.randn(dim, device=dev, generator=g)
+    x1, h = gate_residual_norm(x, out, gp, w, 1e-6)
+    for n in (1, 37):
+        xp, hp = gate_residual_norm(x[-n:], out[-n:], gp[-n:], w, 1e-6)
+        assert torch.equal(xp, x1[-n:]) and torch.equal(hp, h[-n:])
+    shifted = torch.empty(x.numel() + 1, device=dev, dtype=x.dtype)[1:].view_as(x).copy_(x)
+    xs, hs = gate_residual_norm(shifted, out, gp, w, 1e-6)
+    assert torch.equal(xs, x1) and torch.equal(hs, h)
+
+
 @pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float32], ids=["w16", "w32"])
 @pytest.mark.parametrize("dim", [2, 256, 258, 1024, 2050])
 def test_transition_parameters_match_stock_ops(dev, dim, wdtype):
