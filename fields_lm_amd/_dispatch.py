@@ -31,10 +31,10 @@ def no_grad_needed(*tensors: torch.Tensor) -> bool:
 def plain_call(module: nn.Module, cls: type) -> bool:
     """``module`` is exactly ``cls`` and calling it is nothing but its forward: no hook, no replaced
     forward."""
-    m = nn.modules.module
-    return (type(module) is cls and "forward" not in module.__dict__
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
-                     or module._backward_pre_hooks or m._global_forward_hooks or m._global_forward_pre_hooks))
+    m, own = nn.modules.module, module.__dict__
+    return (type(module) is cls and "forward" not in own
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"]
+                     or own["_backward_pre_hooks"] or m._global_forward_hooks or m._global_forward_pre_hooks))
 
 
 def plain_linear(layer: nn.Module) -> bool:

@@ -3,7 +3,7 @@
 // field_only_v4_chunked_triton_wiki100.py:1167-1221; single-token steps have no counterpart there).
 //
 // A decode step reads every weight once: 26 MB per block at dim 1,024, 5 us at the rate of a large
-// copy. A block of the grid owns 16 output columns of 16 rows; its waves split the depth, so each
+// copy. A block of the grid owns 16 output columns of 16 rows (32 where rows are many); its waves split the depth, so each
 // wave's part is a few 16-byte loads per lane that are all in flight together, and the partial sums
 // meet in LDS in a fixed order. More rows per block read the weights fewer times from L2, but put the
 // reading of the rows on fewer CUs, each bound by its loads in flight: 64 rows in one tile took 56 us
@@ -44,13 +44,13 @@ struct LinearArgs {
 constexpr int kSlots = 8;    // partial sums kept in LDS (16 waves fold once before)
 constexpr int kAccRow = 20;  // floats per row of 16 columns
 
-// 16 rows, W waves, G depth steps of 32 loaded together
-template <int EPI, int W, int G>
+// 16 MT rows, W waves, G depth steps of 32 loaded together
+template <int EPI, int W, int G, int MT>
 __global__ __launch_bounds__(W * 64, W / 4) void fl_linear_rows_kernel(LinearArgs a) {
   constexpr int S = EPI == kNormSwiglu ? 2 : 1;  // column sets: gate and up share the rows' operand
-  __shared__ float s_acc[kSlots][S][16][kAccRow], s_sq[W][16];
+  __shared__ float s_acc[kSlots][S][16 * MT][kAccRow], s_sq[W][16 * MT];
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), r = lane & 15, k8 = 8 * (lane >> 4);
-  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16 * MT;
   if (n0 >= a.N) return;  // the grid's width is rounded up
   const int n = min(n0 + r, a.N - 1);
   const bf16_bits* wp[S];
@@ -60,17 +60,23 @@ __global__ __launch_bounds__(W * 64, W / 4) void fl_linear_rows_kernel(LinearArg
   } else {
     wp[0] = n < a.n1 ? a.w + (int64_t)n * a.K : a.w2 + (int64_t)(n - a.n1) * a.K;
   }
-  const bf16_bits* xp = a.x + (int64_t)min(m0 + r, a.M - 1) * a.x_stride;
+  const bf16_bits* xp[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xp[t] = a.x + (int64_t)min(m0 + 16 * t + r, a.M - 1) * a.x_stride;
 
   const int steps = (a.K + 31) / 32, per = (steps + W - 1) / W;
   const int first = min(wave * per, steps), last = min(first + per, steps);
-  f32x4 acc[S];
-  float sq = 0.f;
+  f32x4 acc[S][MT];
+  float sq[MT];
 #pragma unroll
-  for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < MT; ++t) {
+    sq[t] = 0.f;
+#pragma unroll
+    for (int s = 0; s < S; ++s) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   const u32x4 zero = {0u, 0u, 0u, 0u};
   for (int step = first; step < last; step += G) {
-    u32x4 wf[G][S], xf[G];
+    u32x4 wf[G][S], xf[G][MT];
     float nw[G][EPI == kNormSwiglu ? 8 : 1];
 #pragma unroll
     for (int i = 0; i < G; ++i) {
@@ -82,8 +88,11 @@ __global__ __launch_bounds__(W * 64, W / 4) void fl_linear_rows_kernel(LinearArg
         wf[i][s] = *reinterpret_cast<const u32x4*>(wp[s] + kc);
         if (!in) wf[i][s] = zero;
       }
-      xf[i] = *reinterpret_cast<const u32x4*>(xp + kc);
-      if (!in) xf[i] = zero;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        xf[i][t] = *reinterpret_cast<const u32x4*>(xp[t] + kc);
+        if (!in) xf[i][t] = zero;
+      }
       if constexpr (EPI == kNormSwiglu) {
         if (a.norm_w16) Vec<bf16_bits, 8>::load(static_cast<const bf16_bits*>(a.norm_w) + kc, nw[i]);
         else Vec<float, 8>::load(static_cast<const float*>(a.norm_w) + kc, nw[i]);
@@ -91,31 +100,38 @@ __global__ __launch_bounds__(W * 64, W / 4) void fl_linear_rows_kernel(LinearArg
     }
     __builtin_amdgcn_sched_barrier(0);  // every load of the group is issued before the first product
 #pragma unroll
-    for (int i = 0; i < G; ++i) {
-      u32x4 xv = xf[i];
-      if constexpr (EPI == kNormSwiglu) {
+    for (int i = 0; i < G; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float lo = bf16_lo(xv[e]), hi = bf16_hi(xv[e]);
-          sq = fmaf(lo, lo, fmaf(hi, hi, sq));
-          xv[e] = bf16_pair(lo * nw[i][2 * e], hi * nw[i][2 * e + 1]);
+      for (int t = 0; t < MT; ++t) {
+        u32x4 xv = xf[i][t];
+        if constexpr (EPI == kNormSwiglu) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float lo = bf16_lo(xv[e]), hi = bf16_hi(xv[e]);
+            sq[t] = fmaf(lo, lo, fmaf(hi, hi, sq[t]));
+            xv[e] = bf16_pair(lo * nw[i][2 * e], hi * nw[i][2 * e + 1]);
+          }
         }
-      }
 #pragma unroll
-      for (int s = 0; s < S; ++s)
-        acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i][s]),
-                                                         __builtin_bit_cast(bf16x8, xv), acc[s], 0, 0, 0);
-    }
+        for (int s = 0; s < S; ++s)
+          acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i][s]),
+                                                              __builtin_bit_cast(bf16x8, xv), acc[s][t], 0, 0, 0);
+      }
   }
   // lane: columns 4 (lane / 16) .. + 3 of row r
   if constexpr (EPI == kNormSwiglu) {
-    sq += __shfl_xor(sq, 16);
-    sq += __shfl_xor(sq, 32);
-    if (lane < 16) s_sq[wave][r] = sq;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      sq[t] += __shfl_xor(sq[t], 16);
+      sq[t] += __shfl_xor(sq[t], 32);
+      if (lane < 16) s_sq[wave][16 * t + r] = sq[t];
+    }
   }
   auto put = [&](int slot) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) *reinterpret_cast<f32x4*>(&s_acc[slot][s][r][k8 / 2]) = acc[s];
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4*>(&s_acc[slot][s][16 * t + r][k8 / 2]) = acc[s][t];
   };
   if constexpr (W > kSlots) {
     static_assert(W == 2 * kSlots, "one fold");
@@ -123,14 +139,17 @@ __global__ __launch_bounds__(W * 64, W / 4) void fl_linear_rows_kernel(LinearArg
     __syncthreads();
     if (wave < kSlots) {
 #pragma unroll
-      for (int s = 0; s < S; ++s) acc[s] += *reinterpret_cast<const f32x4*>(&s_acc[wave][s][r][k8 / 2]);
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          acc[s][t] += *reinterpret_cast<const f32x4*>(&s_acc[wave][s][16 * t + r][k8 / 2]);
       put(wave);  // its own slot, read by itself alone
     }
   } else {
     put(wave);
   }
   __syncthreads();
-  if (tid < 16 * 8) {
+  if (tid < MT * 16 * 8) {
     const int row = tid >> 3, c = 2 * (tid & 7), m = m0 + row;
     if (m >= a.M) return;
     float v[S][2];
@@ -174,19 +193,29 @@ __global__ __launch_bounds__(W * 64, W / 4) void fl_linear_rows_kernel(LinearArg
   }
 }
 
-template <int EPI>
-int launch_linear(const LinearArgs& a, hipStream_t s) {
+// 16 columns and 16 MT rows a block
+template <int EPI, int MT>
+void launch_tiles(const LinearArgs& a, hipStream_t s) {
   // Row tiles of one column tile lie a multiple of 8 blocks apart: on one XCD, whose L2 then holds
   // their common weights.
-  const dim3 grid((unsigned)(cdiv(cdiv(a.N, 16), 8) * 8), (unsigned)cdiv(a.M, 16));
-  // 8 waves reach a depth of 1,024 with one group of loads each; deeper products take 16.
+  const dim3 grid((unsigned)(cdiv(cdiv(a.N, 16), 8) * 8), (unsigned)cdiv(a.M, 16 * MT));
+  // 8 waves reach a depth of 1,024 (1,280 with a group of 5) with one group of loads each; deeper products
+  // take 16.
   if constexpr (EPI == kNormSwiglu) {
-    fl_linear_rows_kernel<EPI, 8, 4><<<grid, 512, 0, s>>>(a);
+    fl_linear_rows_kernel<EPI, 8, 4, MT><<<grid, 512, 0, s>>>(a);
   } else if (a.K <= 1024) {
-    fl_linear_rows_kernel<EPI, 8, 4><<<grid, 512, 0, s>>>(a);
+    fl_linear_rows_kernel<EPI, 8, 4, MT><<<grid, 512, 0, s>>>(a);
+  } else if (a.K <= 1280) {
+    fl_linear_rows_kernel<EPI, 8, 5, MT><<<grid, 512, 0, s>>>(a);
   } else {
-    fl_linear_rows_kernel<EPI, 16, 5><<<grid, 1024, 0, s>>>(a);
+    fl_linear_rows_kernel<EPI, 16, 5, MT><<<grid, 1024, 0, s>>>(a);
   }
+}
+
+template <int EPI>
+int launch_linear(const LinearArgs& a, bool two, hipStream_t s) {
+  if (two) launch_tiles<EPI, 2>(a, s);
+  else launch_tiles<EPI, 1>(a, s);
   return hip_status(hipGetLastError());
 }
 
@@ -220,11 +249,16 @@ int fl_block_step(const void* x, int64_t rows, int64_t dim, int64_t hidden, cons
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto bf = [](const void* p) { return static_cast<const bf16_bits*>(p); };
   const int M = (int)rows, D = (int)dim, H = (int)hidden;
+  // Two row tiles a block once the blocks of one no longer fit the chip side by side. us in a graph over cold
+  // weights, one | two: dim 512: 96 rows 33.1 | 34.3; 768: 80 rows 39.8 | 43.2, 96 48.3 | 44.9; 1,024: 64 rows
+  // 42.3 | 47.5, 80 54.1 | 45.8, 128 60.1 | 55.5; 1,152: 48 rows 57.2 | 60.3, 64 70.0 | 65.3; 1,280: 32 rows
+  // 51.9 | 56.4, 64 76.4 | 66.9, 128 113.7 | 105.5; 2,048: 32 rows 76.9 | 90.4, 48 104.2 | 94.8
+  const bool two = rows * dim > 65536;
 
   LinearArgs in{};
   in.x = bf(x); in.x_stride = dim; in.w = bf(write_w); in.w2 = bf(gate_w); in.b = bf(write_b); in.b2 = bf(gate_b);
   in.M = M; in.N = (int)wide; in.K = D; in.n1 = (int)(3 * C); in.out = y;
-  int rc = launch_linear<kBias>(in, s);
+  int rc = launch_linear<kBias>(in, two, s);
   if (rc != FL_OK) return rc;
 
   rc = fl_decode_norm_step(y, FL_DTYPE_BF16, rows, C, wide, tr, ti, gamma, state, read_norm_w, read_eps, normed,
@@ -234,20 +268,20 @@ int fl_block_step(const void* x, int64_t rows, int64_t dim, int64_t hidden, cons
   LinearArgs o{};
   o.x = normed; o.x_stride = 2 * dim; o.w = o.w2 = bf(out_w); o.b = o.b2 = bf(out_b);
   o.M = M; o.N = D; o.K = 2 * D; o.n1 = D; o.gate = y + 3 * C; o.gate_stride = wide; o.res = bf(x); o.out = x1;
-  rc = launch_linear<kGatedResidual>(o, s);
+  rc = launch_linear<kGatedResidual>(o, two, s);
   if (rc != FL_OK) return rc;
 
   LinearArgs u{};
   u.x = x1; u.x_stride = dim; u.w = bf(up_w); u.w2 = bf(up_w) + hidden * dim;
   u.M = M; u.N = H; u.K = D; u.n1 = H; u.norm_w = ff_norm_w; u.norm_w16 = ff_norm_dtype == FL_DTYPE_BF16;
   u.eps = ff_eps; u.out = act;
-  rc = launch_linear<kNormSwiglu>(u, s);
+  rc = launch_linear<kNormSwiglu>(u, two, s);
   if (rc != FL_OK) return rc;
 
   LinearArgs d{};
   d.x = act; d.x_stride = hidden; d.w = d.w2 = bf(down_w);
   d.M = M; d.N = D; d.K = H; d.n1 = D; d.res = x1; d.out = static_cast<bf16_bits*>(out);
-  return launch_linear<kResidual>(d, s);
+  return launch_linear<kResidual>(d, two, s);
 }
 
 size_t fl_block_step_workspace_bytes(int64_t rows, int64_t dim, int64_t hidden) {

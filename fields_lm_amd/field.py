@@ -735,6 +735,15 @@ _MIXER_METHODS = frozenset(("in_proj", "normed_step", "step", "decode_params", "
                             "_read_dtype", "_project", "normed_read", "_unfused_read_dtype"))
 
 
+# Weights x rows up to which one token takes ``fl_block_step``: its blocks read their weights again for every
+# row tile, the library's products do not. The line lies where eager calls take equal times: the separate
+# launches 138 us of host time at any size (160 at dim 4,096), fl_block_step 55 us at dim 1,024 x 128 rows, 105
+# at 1,280 x 128, 104 at 2,048 x 64, 125 at 1,536 x 96 and 158 at 4,096 x 16, but 148 at 2,048 x 96, 206 at
+# 4,096 x 32 and 583 at 4,096 x 128. In a graph the separate launches' 59, 76, 76, 61 and 160 us of device time
+# count: there fl_block_step is the faster one up to 128 rows at dim 1,024, 48 at 1,280, 16 at 1,536 and 2,048.
+_STEP_WORK = 3 << 30
+
+
 def _ff_layers(ff: nn.Module) -> Tuple[nn.Module, nn.Module]:
     """The input and output products of either feed-forward layout."""
     return (ff.w12, ff.w3) if hasattr(ff, "w12") else (ff.gate_up, ff.down)
@@ -830,8 +839,7 @@ class FieldBlock(nn.Module):
 
     def _native_step(self, x_t: torch.Tensor, state: torch.Tensor, params):
         """The tensors that ``fl_block_step`` reads where it takes this token, else None: bf16, up to 128
-        rows (past them the library's products are as fast), plain layers, nothing of the mixer
-        replaced, no gradient."""
+        rows and :data:`_STEP_WORK`, plain layers, nothing of the mixer replaced, no gradient."""
         if (torch.is_grad_enabled() or not free_rounding() or x_t.dtype != torch.bfloat16 or x_t.ndim != 2
                 or not 0 < x_t.shape[0] <= 128 or params is None or len(params) < 4 or state is None):
             return None
@@ -859,11 +867,12 @@ class FieldBlock(nn.Module):
         vectors = tuple(t for t in (wb, gb, ob) if t is not None)
         fp32 = (tr, ti, gamma, read_w, state)
         if not (ub is None and db is None and hidden % 8 == 0 and 0 < hidden <= 65536
+                and rows * (9 * dim * dim // 2 + 3 * dim * hidden) <= _STEP_WORK
                 and [t.shape for t in matrices] == [(3 * m.channels, dim), (dim, dim), (dim, 2 * dim),
                                                     (2 * hidden, dim), (dim, hidden)]
-                and [t.shape for t in vectors] == [t.shape[:1] for t, b in zip(matrices, (wb, gb, ob)) if b is not None]
+                and (wb is None or wb.numel() == 3 * m.channels) and (gb is None or gb.numel() == dim)
+                and (ob is None or ob.numel() == dim) and norm.numel() == dim
                 and tr.numel() == ti.numel() == gamma.numel() == m.channels and read_w.numel() == 2 * dim
-                and norm.shape == (dim,)
                 and state.shape == (rows, dim) and norm.dtype in KERNEL_DTYPES
                 and eager(x_t, norm, *fp32, *matrices, *vectors)):
             return None

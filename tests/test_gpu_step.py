@@ -38,7 +38,7 @@ def _block(dev, dim, hidden, seed):
 
 
 @pytest.mark.parametrize("dim,hidden,B", [(1024, 2528, 64), (1024, 2528, 1), (1024, 2784, 128), (136, 352, 16), (136, 352, 17),
-                                          (1112, 2976, 33), (256, 96, 65), (64, 8, 31), (16, 24, 2), (520, 264, 48)])
+                                          (1112, 2976, 33), (1280, 3424, 65), (2056, 96, 33), (1288, 96, 32), (256, 96, 65), (64, 8, 31), (16, 24, 2), (520, 264, 48)])
 def test_block_step_kernels(dev, dim, hidden, B):
     print(f"[case] block step dim={dim} hidden={hidden} B={B}", flush=True)
     b = _block(dev, dim, hidden, seed=dim + B)

@@ -404,3 +404,15 @@ def test_refresh_attention_with_a_wider_mix_takes_the_stock_ops(monkeypatch, sha
         assert att._native(qlat) and att._exact(x, qlat) and att._native_step(qlat[:, 0].contiguous(), pos, st)
         att.global_mix_logit = torch.nn.Parameter(torch.zeros(shape, dtype=torch.bfloat16))
         assert not (att._native(qlat) or att._exact(x, qlat) or att._native_step(qlat[:, 0].contiguous(), pos, st))
+
+
+def test_step_route_ends_where_its_products_lose(monkeypatch):
+    """Wide blocks with many rows take the library's products; the line is weights x rows."""
+    from fields_lm_amd import field
+
+    block, x, state, params = _step_call(monkeypatch)
+    work = 2 * (9 * 16 * 16 // 2 + 3 * 16 * 24)
+    with torch.no_grad():
+        for limit, native in ((work, True), (work - 1, False)):
+            monkeypatch.setattr(field, "_STEP_WORK", limit)
+            assert (block._native_step(x, state, params) is not None) == native
