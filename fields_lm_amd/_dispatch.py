@@ -39,7 +39,10 @@ def plain_call(module: nn.Module, cls: type) -> bool:
 
 def plain_linear(layer: nn.Module) -> bool:
     """An nn.Linear whose call is nothing but its GEMM on an ordinary weight."""
-    return plain_call(layer, nn.Linear) and type(layer.weight) in (nn.Parameter, torch.Tensor)
+    if not plain_call(layer, nn.Linear):
+        return False
+    weight = layer._parameters.get("weight")  # (an attribute of the module costs ten times a dict's entry)
+    return type(layer.weight if weight is None else weight) in (nn.Parameter, torch.Tensor)
 
 
 def free_rounding() -> bool:

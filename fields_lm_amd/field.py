@@ -858,7 +858,10 @@ class FieldBlock(nn.Module):
         if not (plain_call(inner["read_norm"], RMSNorm) and plain_call(ff_norm, RMSNorm)
                 and all(plain_linear(layer) for layer in layers)):
             return None
-        tensors = [(p["weight"], p["bias"]) for p in (layer._parameters for layer in layers)]
+        own = [layer._parameters for layer in layers]
+        if not all("weight" in p and "bias" in p for p in own):
+            return None
+        tensors = [(p["weight"], p["bias"]) for p in own]
         (ww, wb), (gw, gb), (ow, ob), (uw, ub), (dw, db) = tensors
         hidden = dw.shape[1]
         norm = ff_norm.weight

@@ -416,3 +416,15 @@ def test_step_route_ends_where_its_products_lose(monkeypatch):
         for limit, native in ((work, True), (work - 1, False)):
             monkeypatch.setattr(field, "_STEP_WORK", limit)
             assert (block._native_step(x, state, params) is not None) == native
+
+
+@pytest.mark.parametrize("attr", ["weight", "bias"])
+def test_step_route_without_a_registered_parameter(monkeypatch, attr):
+    """A weight or bias kept as a plain attribute (no longer a parameter) takes the separate launches."""
+    block, x, state, params = _step_call(monkeypatch)
+    layer = block.mixer.out_proj
+    value = getattr(layer, attr).detach()
+    delattr(layer, attr)
+    setattr(layer, attr, value)
+    with torch.no_grad():
+        assert block._native_step(x, state, params) is None
