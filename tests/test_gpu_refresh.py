@@ -55,6 +55,8 @@ def test_attention_against_fp32(dev, heads, kv, window, chunk, B, T):
     with torch.no_grad():
         y = att(x)
         exp, st_exp = ref.prefill(x.float(), T + 70)
+        used = [torch.full(t.shape, float("nan"), device=dev, dtype=x.dtype) for t in st_exp.values()]
+        del used  # what an unwritten slot would hold
         yp, st = att.prefill(x, T + 70)
     assert torch.equal(y, yp)
     e, e_stock = _norm(y, exp), _norm(stock, exp)
@@ -63,8 +65,12 @@ def test_attention_against_fp32(dev, heads, kv, window, chunk, B, T):
     assert set(st) == set(st_exp)
     for name in st:
         assert st[name].shape == st_exp[name].shape and st[name].dtype == (torch.float32 if name == "lat_sum" else x.dtype)
-        assert torch.equal(st[name] == 0, st_exp[name] == 0) or _norm(st[name], st_exp[name]) <= 1e-2, name
         assert _norm(st[name], st_exp[name]) <= 1e-2, name
+    n, full = T % window, T // chunk  # slots in use: the open window's tokens; landmarks after the null slot
+    for name, unused in (("kt", st["kt"][..., n:]), ("v", st["v"][:, :, n:]), ("null key", st["lkt"][..., :1]),
+                         ("null value", st["lv"][:, :, :1]), ("lkt", st["lkt"][..., 1 + full:]),
+                         ("lv", st["lv"][:, :, 1 + full:])):
+        assert not unused.any(), name
 
 
 @pytest.mark.parametrize("T", [40, 63, 130])
