@@ -195,3 +195,51 @@ def test_promoted_model_bf16_decode_equals_forward(dev):
     assert logits.shape == (2, 300, 16384) and torch.isfinite(logits).all()
     assert oracle.rel_err(last.float().cpu(), logits[:, 279].float().cpu()) <= 2e-2
     assert oracle.rel_err(torch.stack(steps, 1).float().cpu(), logits[:, 280:].float().cpu()) <= 2e-2
+
+
+def test_promoted_model_bf16_weights_without_autocast(dev):
+    """The route that runs every kernel (bf16 weights by ``cast_for_inference``, no autocast): logits of a
+    prompt, of its prefill and of decode steps, eager and replayed from a HIP graph, against the same weights
+    in fp32, no further off than the autocast route by more than 10 %: both round every layer to bf16, the
+    kernels once where the stock ops round several times."""
+    import copy
+
+    print("[case] promoted model, bf16 weights, no autocast", flush=True)
+    core = M.cast_for_inference(M.build_official_fields(device=dev).core_model).eval()
+    ref = copy.deepcopy(core).float()
+    tokens = torch.randint(0, 16384, (2, 560), device=dev, generator=torch.Generator(device=dev).manual_seed(5))
+    prompt, n = 530, 20
+
+    def err(got, exp):
+        return float((got.double() - exp.double()).norm() / exp.double().norm())
+
+    with torch.no_grad():
+        exp = ref.states_logits(tokens)[1]
+        logits = core.states_logits(tokens)[1]
+        with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
+            auto = core.states_logits(tokens)[1]
+        last, cache = core.prefill(tokens[:, :prompt], max_len=600)
+        field = [i for i, k in enumerate(core.kinds()) if k == "field"]
+        x = core.emb(tokens[:, prompt])
+        assert all(core.blocks[i]._native_step(x, cache["blocks"][i], cache["params"][i]) is not None for i in field)
+        fresh = copy.deepcopy(cache)
+        steps = [core.step(tokens[:, prompt + i], cache).clone() for i in range(n)]
+        tok = tokens[:, prompt].clone()
+        _copy_cache(cache, fresh)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = core.step(tok, cache)
+        _copy_cache(cache, fresh)
+        for i in range(n):
+            tok.copy_(tokens[:, prompt + i])
+            graph.replay()
+            torch.cuda.synchronize()
+            assert err(out, steps[i]) <= 1e-6, i
+    e, e_auto = err(logits, exp), err(auto, exp)
+    e_step = err(torch.stack(steps, 1), exp[:, prompt:prompt + n])
+    e_step_auto = err(auto[:, prompt:prompt + n], exp[:, prompt:prompt + n])
+    print(f"[case] prompt {e:.2e} (autocast {e_auto:.2e}), last {err(last, exp[:, prompt - 1]):.2e}, "
+          f"steps {e_step:.2e} (autocast forward {e_step_auto:.2e})", flush=True)
+    assert torch.isfinite(logits).all()
+    assert e <= 1.1 * e_auto and err(last, exp[:, prompt - 1]) <= 1.1 * e_step_auto + 2e-3
+    assert e_step <= 1.1 * e_step_auto + 2e-3
