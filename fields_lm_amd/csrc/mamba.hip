@@ -540,7 +540,10 @@ int prefill_impl(const T* zx, int64_t B, int64_t L, int64_t H, int64_t sb, int64
                                                                dt_bias, frags, dts);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_status(e);
-  if (B * H * 2 >= 256) {
+  // A block takes 32 channels of a head once blocks of 16 would be more than the 256 CUs (they share less
+  // of C, B and C B^T). us, 16 | 32 channels, 32 heads: 1 x 2,048 tokens 114 | 155, 2 x 1,024 73 | 94,
+  // 3 x 1,024 120 | 98, 4 x 1,024 123 | 102, 8 x 1,024 222 | 182
+  if (B * H * 4 > 256) {
     fl_mamba_scan_kernel<T, 2><<<(unsigned)(B * H * 2), 512, 0, s>>>(xbc, sb, st, (int)L, (int)H, nc, conv, A_log,
                                                                      D, frags, dts, y, ssm_out);
   } else {

@@ -63,7 +63,7 @@ def _f64(m, u):
 
 
 @pytest.mark.parametrize("dim,B,L", [(64, 2, 1), (128, 1, 3), (512, 1, 64), (512, 2, 65), (128, 3, 63), (512, 9, 129),
-                                     (1024, 4, 200), (192, 2, 128)])
+                                     (1024, 4, 200), (192, 2, 128), (1024, 2, 70), (512, 5, 66)])
 def test_mamba_prefill_fp32(dev, dim, B, L):
     print(f"[case] mamba prefill fp32 dim={dim} B={B} L={L}", flush=True)
     m = _mixer(dev, dim, seed=L)
