@@ -427,7 +427,9 @@ __global__ __launch_bounds__(256) void fl_gated_norm_kernel(
 template <typename T, typename OT>
 int launch_gated_norm(const float* y, const T* z, int64_t zsb, int64_t zst, int64_t rows, int L, int dim,
                       const void* w, int w16, float eps, OT* out, hipStream_t s) {
-  const unsigned waves = rows >= 4096 ? 4 : 1;  // one row per CU slot while there are few rows
+  // one row per block while the rows are few; whole call, one | four rows a block: 64 x 64 tokens 136.0 | 135.4 us,
+  // 64 x 1 107.1 | 107.3, 8 x 64 33.1 | 33.5
+  const unsigned waves = rows >= 4096 ? 4 : 1;
   const unsigned blocks = (unsigned)cdiv(rows, waves);
   const float inv = (float)(1.0 / (double)dim);
 #define FL_GN(N, NV)                                                                              \
