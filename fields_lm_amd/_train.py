@@ -20,10 +20,10 @@ def _stock_grads(fn, inputs, grads):
         inputs = [t.view_as(t) for t in inputs]
         outs = fn(*inputs)
         outs = outs if isinstance(outs, tuple) else (outs,)
-        pairs = [(o, g) for o, g in zip(outs, grads) if g is not None]
+        pairs = [(o, g) for o, g in zip(outs, grads) if o.requires_grad]
         wanted = [t for t in inputs if t.requires_grad]
         got = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True,
-                                       allow_unused=True))
+                                       allow_unused=True) if wanted else ())
     return [next(got) if t.requires_grad else None for t in inputs]
 
 

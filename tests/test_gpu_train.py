@@ -124,6 +124,23 @@ def test_training_double_backward_matches_stock(dev):
         assert _norm(a, e) <= 1e-4
 
 
+@pytest.mark.parametrize("wanted", [("ff_norm.weight",), ("mixer.theta", "ff_norm.weight")])
+def test_training_double_backward_with_frozen_parameters(dev, wanted):
+    print(f"[case] block training, double backward, only {wanted}", flush=True)
+    b = _block(dev, 32, 24)
+    for n, p in b.named_parameters():
+        p.requires_grad_(n in wanted)
+    params = [dict(b.named_parameters())[n] for n in wanted]
+    x = torch.randn(2, 7, 32, device=dev)
+    out = []
+    for native in (True, False):
+        b.fuse_tail = native
+        grads = torch.autograd.grad(b(x).square().sum(), params, create_graph=True)
+        out.append(torch.autograd.grad(sum(g.square().sum() for g in grads), params[-1:]))
+    for a, e in zip(*out):
+        assert _norm(a, e) <= 1e-4
+
+
 def test_training_replaced_parts_keep_the_stock_ops(dev):
     print("[case] block training, replaced parts", flush=True)
     b = _block(dev, 64, 40)

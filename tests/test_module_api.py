@@ -428,3 +428,16 @@ def test_step_route_without_a_registered_parameter(monkeypatch, attr):
     setattr(layer, attr, value)
     with torch.no_grad():
         assert block._native_step(x, state, params) is None
+
+
+def test_stock_gradients_with_frozen_inputs():
+    """Differentiable gradients where some inputs, or some outputs with them, need none."""
+    from fields_lm_amd import _train
+
+    a, b, g = torch.randn(3), torch.randn(3), torch.randn(3)
+    assert _train._stock_grads(lambda o, s: o * s, (a, b), (g,)) == [None, None]
+    b.requires_grad_()
+    ga, gb = _train._stock_grads(lambda o, s: (o * 2, s * s), (a, b), (g, g))  # the first output needs none
+    assert ga is None
+    torch.testing.assert_close(gb, 2 * b * g)
+    assert _train._stock_grads(_train.transition_ops, (a, b), (g, g, g))[0] is None  # gamma depends on a alone
