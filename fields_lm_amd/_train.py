@@ -2,7 +2,8 @@
 (``csrc/train.hip``; canon:300-325, 1169-1173, 1193-1195, 1219-1221).
 
 A backward that must itself be differentiable (``create_graph``) runs the stock ops instead, from the
-tensors as they came in (saved before any copy for alignment, so that they keep their graph).
+tensors as they came in (saved before any copy for alignment, so that they keep their graph). Autograd
+materialises the gradients of unused outputs as zeros, so that no backward sees a missing one.
 """
 from __future__ import annotations
 
@@ -99,15 +100,13 @@ class GateNorm(torch.autograd.Function):
         x_new, out, gate, w, rstd = ctx.saved_tensors
         if torch.is_grad_enabled():
             # through the norm from x_new, then through the gated sum, whose value x_new already is
-            gx, gw = (None, None) if g_normed is None else \
-                _stock_grads(lambda a, b: _norm_ops(a, b, ctx.eps, ctx.dtype), (x_new, w), (g_normed,))
-            gx = g_x if gx is None else gx if g_x is None else g_x + gx
+            gx, gw = _stock_grads(lambda a, b: _norm_ops(a, b, ctx.eps, ctx.dtype), (x_new, w), (g_normed,))
+            gx = g_x if gx is None else g_x + gx
             g_out, g_gate = _stock_grads(lambda o, g: (o * torch.sigmoid(g)).to(x_new.dtype), (out, gate), (gx,))
             return gx, g_out, g_gate, gw, None, None
         lib, dim = nat.load(), x_new.shape[-1]
         out, gate = _aligned(out), _aligned(gate)
-        g_x = torch.zeros_like(x_new) if g_x is None else _aligned(g_x)
-        g_normed = torch.zeros_like(x_new, dtype=ctx.dtype) if g_normed is None else _aligned(g_normed)
+        g_x, g_normed = _aligned(g_x), _aligned(g_normed)
         gx, g_out, g_gate, gw = (torch.empty_like(t) for t in (x_new, out, gate, w))
         ws = _workspace(lib, dim, x_new.device)
         nat.check(lib.fl_train_gate_norm_backward(
@@ -177,7 +176,7 @@ class Transition(torch.autograd.Function):
         if torch.is_grad_enabled():
             return tuple(_stock_grads(transition_ops, (radius_logit, theta), grads))
         lib, c = nat.load(), radius_logit.numel()
-        grads = [torch.zeros_like(theta) if g is None else g.contiguous() for g in grads]
+        grads = [g.contiguous() for g in grads]
         gl, gt = torch.empty_like(radius_logit), torch.empty_like(theta)
         nat.check(lib.fl_field_params_backward(nat.ptr(radius_logit), nat.ptr(theta), c, *[nat.ptr(g) for g in grads],
                                                nat.ptr(gl), nat.ptr(gt), nat.stream_handle(theta.device)),
