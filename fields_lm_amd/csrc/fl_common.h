@@ -132,20 +132,20 @@ __device__ __forceinline__ float sigmoid_bf16(float x) {
 
 // x / (1 + e^-x) to about an ulp: v_exp_f32 of the rounded product x log2(e) with the product's
 // rounding error put back (first order), and one residual step on the reciprocal's quotient. The
-// exponent is held within +-88.7, where e^-x is finite; below, the result is -0 (NaN for -inf). Where the
-// residual is 0 or NaN (an infinite x) the plain quotient stands. For every bf16 x the result rounds to
-// the stock op's bf16 value.
+// exponent is held within the first float whose rounded product reaches 128 (its error is positive, so that
+// the corrected power is inf, not NaN): below, the quotient is -0, and NaN for -inf. Where the residual
+// is 0 or NaN the plain quotient stands. For every bf16 x the result rounds to the stock op's bf16 value.
 __device__ __forceinline__ float silu_precise(float x) {
   constexpr float kL = -kLog2e, kLlo = -1.9259629911266175e-8f;  // -log2(e) = kL + kLlo
-  const float xc = __builtin_amdgcn_fmed3f(x, -88.7f, 88.7f);
+  constexpr float kLimit = 88.72283935546875f;
+  const float xc = __builtin_amdgcn_fmed3f(x, -kLimit, kLimit);
   const float hi = xc * kL;
   const float lo = fmaf(xc, kLlo, fmaf(xc, kL, -hi));
   const float e0 = __builtin_amdgcn_exp2f(hi);
   const float corr = fmaf(e0, lo * 0.6931471805599453f, e0);
   const float d = 1.0f + corr, r = rcp_one_plus(corr), q = x * r;
   const float res = fmaf(-q, d, x);
-  const float y = __builtin_fabsf(res) > 0.0f ? fmaf(res, r, q) : q;
-  return x < -88.7f ? x * 0.0f : y;
+  return __builtin_fabsf(res) > 0.0f ? fmaf(res, r, q) : q;
 }
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }

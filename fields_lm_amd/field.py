@@ -785,21 +785,23 @@ class FieldBlock(nn.Module):
         fp32 residual stream and fp32 parameters (under bf16 autocast or none), every module between
         the products its own class, called without hooks, and plain layers behind the norms, whose bf16 output
         is the cast such a layer makes of its input."""
-        m, ff, dim = self.mixer, self.ff, x.shape[-1]
-        if not (torch.is_grad_enabled() and x.dtype == torch.float32 and x.numel() > 0 and x.ndim == 3
-                and dim == m.dim and dim % 8 == 0 and dim <= 2048 and x.numel() // dim < 1 << 31
-                and type(self) is FieldBlock and plain_call(m, IndependentVacancyField)
-                and plain_call(self.ff_norm, RMSNorm) and plain_call(m.read_norm, RMSNorm)
-                and _plain_ff(ff) and plain_linear(m.out_proj) and plain_linear(_ff_layers(ff)[0])
-                and _MIXER_METHODS.isdisjoint(m.__dict__) and m.read_dtype == "auto" and self.fuse_tail
+        if not (torch.is_grad_enabled() and x.dtype == torch.float32 and x.ndim == 3 and type(self) is FieldBlock
+                and self.fuse_tail):
+            return False
+        m, ff, ff_norm, dim = self.mixer, self.ff, self.ff_norm, x.shape[-1]
+        if not (x.numel() > 0 and dim == m.dim and dim % 8 == 0 and dim <= 2048 and x.numel() // dim < 1 << 31
+                and plain_call(m, IndependentVacancyField) and m.read_dtype == "auto"
+                and _MIXER_METHODS.isdisjoint(m.__dict__)):
+            return False
+        read_norm = m.read_norm
+        if not (plain_call(ff_norm, RMSNorm) and plain_call(read_norm, RMSNorm) and _plain_ff(ff)
+                and plain_linear(m.out_proj) and plain_linear(_ff_layers(ff)[0])
                 and (not torch.is_autocast_enabled() or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
             return False
-        norms = (m.read_norm.weight, self.ff_norm.weight)
-        ring = (m.radius_logit, m.theta)
-        return (norms[0].shape == (2 * dim,) and norms[1].shape == (dim,)
-                and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in norms)
-                and all(t.dtype == torch.float32 and t.is_contiguous() and t.shape == (m.channels,) for t in ring)
-                and eager(x, *norms, *ring))
+        norms, ring = (read_norm.weight, ff_norm.weight), (m.radius_logit, m.theta)
+        return ([t.shape for t in (*norms, *ring)] == [(2 * dim,), (dim,), (m.channels,), (m.channels,)]
+                and all(t.dtype == torch.float32 and t.is_contiguous() for t in (*norms, *ring))
+                and (norms[0].data_ptr() | norms[1].data_ptr()) % 16 == 0 and eager(x, *norms, *ring))
 
     def _train_forward(self, x: torch.Tensor) -> torch.Tensor:
         m = self.mixer

@@ -763,20 +763,23 @@ class Mamba2Mixer(nn.Module):
     def _native(self, zxbcdt: torch.Tensor) -> bool:
         """The kernels of ``fl_mamba_prefill`` / ``fl_mamba_step`` take this call: the promoted
         geometry, no gradient, every tensor where and what they read."""
-        params = (self.conv1d.weight, self.conv1d.bias, self.A_log, self.dt_bias, self.D, self.norm.weight)
-        heads, inner, channels = self.nheads, self.d_inner, self.conv_dim
-        return (free_rounding() and type(self) is Mamba2Mixer and plain_call(self.norm, GatedRMSNorm)
-                and (self.headdim, self.d_state, self.d_conv) == (64, 128, 4) and heads <= 1024
-                and inner == 64 * heads and zxbcdt.shape[-1] == inner + channels + heads
+        if not (free_rounding() and type(self) is Mamba2Mixer and zxbcdt.dtype in KERNEL_DTYPES
+                and (self.headdim, self.d_state, self.d_conv) == (64, 128, 4)):
+            return False
+        conv, norm, heads, inner, channels = self.conv1d, self.norm, self.nheads, self.d_inner, self.conv_dim
+        params = conv_w, conv_b, _, _, _, norm_w = (conv.weight, conv.bias, self.A_log, self.dt_bias, self.D,
+                                                    norm.weight)
+        shape = zxbcdt.shape
+        return (plain_call(norm, GatedRMSNorm) and inner == 64 * heads and heads <= 1024
+                and shape[-1] == inner + channels + heads
                 and [t.shape for t in params] == [(channels, 1, 4), (channels,), (heads,), (heads,), (heads,), (inner,)]
                 and no_grad_needed(zxbcdt, *params) and eager(zxbcdt, *params)
-                and zxbcdt.dtype in KERNEL_DTYPES and zxbcdt.is_contiguous() and zxbcdt.numel() > 0
-                and zxbcdt.shape[-1] % 2 == 0 and zxbcdt.data_ptr() % 8 == 0
-                and self.conv1d.weight.dtype == self.conv1d.bias.dtype and self.conv1d.weight.is_contiguous()
-                and self.conv1d.bias.is_contiguous() and self.norm.weight.is_contiguous()
-                and self.conv1d.weight.dtype in KERNEL_DTYPES and self.norm.weight.dtype in KERNEL_DTYPES
-                and zxbcdt.shape[0] <= 65535 and zxbcdt.shape[0] * self.nheads <= 1 << 20
-                and zxbcdt.shape[-2] <= 1 << 26)
+                and zxbcdt.is_contiguous() and zxbcdt.numel() > 0
+                and shape[-1] % 2 == 0 and zxbcdt.data_ptr() % 8 == 0
+                and conv_w.dtype == conv_b.dtype and conv_w.is_contiguous()
+                and conv_b.is_contiguous() and norm_w.is_contiguous()
+                and conv_w.dtype in KERNEL_DTYPES and norm_w.dtype in KERNEL_DTYPES
+                and shape[0] <= 65535 and shape[0] * heads <= 1 << 20 and shape[-2] <= 1 << 26)
 
     def _native_call(self, name: str, zxbcdt: torch.Tensor, length: int, shape, strides, out_dtype, *state):
         """Runs ``name`` (its arguments past the strides are alike); returns what out_proj reads."""
@@ -974,20 +977,22 @@ class BoundaryStateMixer(nn.Module):
 
     def _native(self, x: torch.Tensor, tokens: torch.Tensor) -> bool:
         """The kernels of ``fl_softpatch_norm`` / ``fl_softpatch_scan`` take this call."""
-        score, norm, down, up, lut = self.score, self.norm, self.down, self.up, self._boundary_lut
-        if not (free_rounding() and type(self) is BoundaryStateMixer and self.learned and x.ndim == 3
-                and plain_call(norm, RMSNorm) and plain_linear(score) and score.bias is not None
-                and plain_linear(down) and down.bias is None and plain_linear(up) and up.bias is None
-                and x.is_contiguous() and x.data_ptr() % 16 == 0):
+        if not (free_rounding() and x.dtype == torch.bfloat16 and type(self) is BoundaryStateMixer and self.learned
+                and x.ndim == 3 and x.is_contiguous() and x.data_ptr() % 16 == 0):
             return False
-        params = (norm.weight, score.weight, score.bias, down.weight, up.weight)
-        dim, rank = x.shape[-1], down.weight.shape[0]
-        return (rms_norm_takes(x, norm.weight) and no_grad_needed(*params) and 0 < rank <= 1 << 16
+        score, norm, down, up, lut = self.score, self.norm, self.down, self.up, self._boundary_lut
+        if not (plain_call(norm, RMSNorm) and plain_linear(score) and plain_linear(down) and plain_linear(up)
+                and score.bias is not None and down.bias is None and up.bias is None):
+            return False
+        params = norm_w, score_w, _, down_w, _ = (norm.weight, score.weight, score.bias, down.weight, up.weight)
+        dim, rank = x.shape[-1], down_w.shape[0]
+        return (dim % 8 == 0 and dim <= 4096 and 0 < x.numel() < dim << 31 and 0 < rank <= 1 << 16
+                and x.shape[0] <= 65535 and x.shape[1] <= 1 << 26 and no_grad_needed(x, *params)
                 and [t.shape for t in params] == [(dim,), (1, dim), (1,), (rank, dim), (dim, 2 * rank)]
                 and eager(x, tokens, lut, *params)
                 and lut.dtype == torch.float32 and lut.ndim == 1 and tokens.shape == x.shape[:2]
-                and all(t.dtype == x.dtype and t.is_contiguous() for t in params)
-                and score.weight.data_ptr() % 16 == 0 and x.shape[0] <= 65535 and x.shape[1] <= 1 << 26)
+                and all(t.dtype == torch.bfloat16 and t.is_contiguous() for t in params)
+                and (norm_w.data_ptr() | score_w.data_ptr()) % 16 == 0)
 
     def _native_forward(self, x: torch.Tensor, tokens: torch.Tensor):
         lib, stream = nat.load(), nat.stream_handle(x.device)
