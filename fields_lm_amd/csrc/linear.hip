@@ -13,9 +13,9 @@
 //   up:    RMSNorm of its input (the row's scale is applied to the sums, the weight to the operand),
 //          gate and up columns in one block, then silu(gate) * up
 //   down:  the FFN's output product, added to the residual
-// 64 rows, dim 1,024, hidden 2,528: 39.8 us of kernels with the weights in the Infinity Cache and 40.7 us
-// in a graph over 12 blocks' cold weights, where the library's products and separate launches took
-// 51.5 and 62.5 us; one row 27.3 us cold against 59.8 us.
+// 64 rows, dim 1,024, hidden 2,528: 41.1 us of kernels with the weights in the Infinity Cache (in 9.3, norm
+// 3.7, out 9.0, up 13.5, down 5.7) and 42 us in a graph over 12 blocks' cold weights, where the library's
+// products and separate launches take 58 us; one row 27 us cold against 56.
 #include "fl_common.h"
 
 namespace {

@@ -7,9 +7,9 @@
 // All of them are bound by memory: each tensor is read and written once, 16 bytes per lane and access
 // (8 for fp32 twice), one wave per row, where the stock ops made six to ten passes each way. Weight
 // gradients: a wave adds its rows in registers, a block its waves in LDS, and a second launch the blocks,
-// in a fixed order. 4,096 tokens, dim 1,024, bf16 autocast: read_norm 12.2 us forward and 21.1 + 4.3 us
-// backward (fp32 [4096, 2048]: 50 MB and 84 MB), gated residual and norm 10.3 and 18.5 + 4.3 us, SwiGLU
-// backward 17.8 us; a training pass of the block 1,416 -> 876 us of kernels, 144 -> 56 launches.
+// in a fixed order. 4,096 tokens, dim 1,024, bf16 autocast: read_norm 12.0 us forward and 22.3 + 4.3 us
+// backward (fp32 [4096, 2048]: 50 MB and 84 MB), gated residual and norm 11.0 and 18.4 + 4.3 us, SwiGLU
+// backward 17.3 us; a training pass of the block 865 us of kernels in 57 launches (stock ops: 1,416 in 144).
 #include "fl_common.h"
 
 namespace {

@@ -1,5 +1,7 @@
-"""The promoted Fields model (18F/2M/4R + PCAF) for inference, with the Field blocks on the HIP
-kernels and every other block as stock PyTorch-ROCm ops.
+"""The promoted Fields model (18F/2M/4R + PCAF) for inference: every block on this package's HIP kernels
+around the library's products where a call is one they take (plain eager tensors, no gradient, the geometry
+and types each route checks), and on stock PyTorch-ROCm ops otherwise. Under autocast only kernels run that
+keep the stock ops' bits; without it, with ``cast_for_inference`` weights, all of them.
 
 Reference (paths relative to src/fields_official/):
   api  = fields_official.py                       FieldsConfig / FieldsForCausalLM / build_official_fields
@@ -100,7 +102,7 @@ class GateUpSwiGLU(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         h = self.gate_up(x)
         if (h.dtype == torch.bfloat16 and no_grad_needed(h) and eager(h) and h.numel() > 0 and h.shape[-1] % 2 == 0):
-            return self.down(swiglu(h))  # the stock ops' bits
+            return self.down(swiglu(h))  # the stock ops' bits, for every bf16 gate
         gate, up = h.chunk(2, dim=-1)
         return self.down(F.silu(gate) * up)
 
