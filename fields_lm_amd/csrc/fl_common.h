@@ -134,7 +134,9 @@ __device__ __forceinline__ float sigmoid_bf16(float x) {
 // rounding error put back (first order), and one residual step on the reciprocal's quotient. The
 // exponent is held within the first float whose rounded product reaches 128 (its error is positive, so that
 // the corrected power is inf, not NaN): below, the quotient is -0, and NaN for -inf. Where the residual
-// is 0 or NaN the plain quotient stands. For every bf16 x the result rounds to the stock op's bf16 value.
+// is 0 or NaN the plain quotient stands. For every bf16 x the result rounds to the stock op's bf16 value;
+// without SUBNORMAL (two operations less) it is -0 from -87.3 down, where the stock value is under 1.1e-36.
+template <bool SUBNORMAL = true>
 __device__ __forceinline__ float silu_precise(float x) {
   constexpr float kL = -kLog2e, kLlo = -1.9259629911266175e-8f;  // -log2(e) = kL + kLlo
   constexpr float kLimit = 88.72283935546875f;
@@ -143,7 +145,7 @@ __device__ __forceinline__ float silu_precise(float x) {
   const float lo = fmaf(xc, kLlo, fmaf(xc, kL, -hi));
   const float e0 = __builtin_amdgcn_exp2f(hi);
   const float corr = fmaf(e0, lo * 0.6931471805599453f, e0);
-  const float d = 1.0f + corr, r = rcp_one_plus(corr), q = x * r;
+  const float d = 1.0f + corr, r = SUBNORMAL ? rcp_one_plus(corr) : __builtin_amdgcn_rcpf(d), q = x * r;
   const float res = fmaf(-q, d, x);
   return __builtin_fabsf(res) > 0.0f ? fmaf(res, r, q) : q;
 }

@@ -81,7 +81,7 @@ __device__ __forceinline__ float conv_silu(const float* wt, float bias, float a,
   float v = fmaf(a, wt[0], bias);
   v = fmaf(b, wt[1], v);
   v = fmaf(c, wt[2], v);
-  return silu_precise(fmaf(d, wt[3], v));
+  return silu_precise<false>(fmaf(d, wt[3], v));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(256) void fl_gated_norm_kernel(
     Vec<float, N>::load(yr + c, v);
     Vec<T, N>::load(zr + c, g);
 #pragma unroll
-    for (int j = 0; j < N; ++j) v[j] *= silu_precise(g[j]);
+    for (int j = 0; j < N; ++j) v[j] *= silu_precise<false>(g[j]);
   };
   auto finish = [&](int c, const float* v, float scale) {
     float ww[N], q[N];

@@ -788,20 +788,21 @@ class FieldBlock(nn.Module):
         if not (torch.is_grad_enabled() and x.dtype == torch.float32 and x.ndim == 3 and type(self) is FieldBlock
                 and self.fuse_tail):
             return False
-        m, ff, ff_norm, dim = self.mixer, self.ff, self.ff_norm, x.shape[-1]
+        parts = self._modules
+        m, ff, ff_norm, dim = parts["mixer"], parts["ff"], parts["ff_norm"], x.shape[-1]
         if not (x.numel() > 0 and dim == m.dim and dim % 8 == 0 and dim <= 2048 and x.numel() // dim < 1 << 31
                 and plain_call(m, IndependentVacancyField) and m.read_dtype == "auto"
                 and _MIXER_METHODS.isdisjoint(m.__dict__)):
             return False
-        read_norm = m.read_norm
+        read_norm = m._modules["read_norm"]
         if not (plain_call(ff_norm, RMSNorm) and plain_call(read_norm, RMSNorm) and _plain_ff(ff)
-                and plain_linear(m.out_proj) and plain_linear(_ff_layers(ff)[0])
+                and plain_linear(m._modules["out_proj"]) and plain_linear(_ff_layers(ff)[0])
                 and (not torch.is_autocast_enabled() or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
             return False
-        norms, ring = (read_norm.weight, ff_norm.weight), (m.radius_logit, m.theta)
-        return ([t.shape for t in (*norms, *ring)] == [(2 * dim,), (dim,), (m.channels,), (m.channels,)]
-                and all(t.dtype == torch.float32 and t.is_contiguous() for t in (*norms, *ring))
-                and (norms[0].data_ptr() | norms[1].data_ptr()) % 16 == 0 and eager(x, *norms, *ring))
+        params = norm1, norm2, _, _ = read_norm.weight, ff_norm.weight, m.radius_logit, m.theta
+        return ([t.shape for t in params] == [(2 * dim,), (dim,), (m.channels,), (m.channels,)]
+                and all(t.dtype == torch.float32 and t.is_contiguous() for t in params)
+                and (norm1.data_ptr() | norm2.data_ptr()) % 16 == 0 and eager(x, *params))
 
     def _train_forward(self, x: torch.Tensor) -> torch.Tensor:
         m = self.mixer
