@@ -277,7 +277,9 @@ int fl_gate_residual_norm_w(const void* x, int x_dtype, const void* out, const v
  * x, out [rows, dim] contiguous; weights as their layers hold them ([out features, in features]),
  * 16-byte aligned; dim and hidden multiples of 8; biases may be NULL; tr, ti, gamma, read_norm_w
  * fp32, ff_norm_w of ff_norm_dtype; state [rows, dim] fp32 advances in place. Rounded to bf16 where the
- * separate ops round, except that the RMSNorm's row scale is applied to the fp32 sums.
+ * separate ops round, except that the RMSNorm's row scale is applied to the fp32 sums. The weights are
+ * read once per row tile of 16 (32 from rows x dim of 65,536 on): wide blocks with many rows are faster
+ * through products that read them once.
  */
 size_t fl_block_step_workspace_bytes(int64_t rows, int64_t dim, int64_t hidden);
 int fl_block_step(const void* x, int64_t rows, int64_t dim, int64_t hidden, const void* write_w, const void* write_b,
